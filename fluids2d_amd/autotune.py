@@ -115,9 +115,9 @@ def _test_rhs(shape, msk):
 def tune_poisson(mesh, maindiag=0.0, reps=4, candidates=None, cache=True, verbose=False):
     """Best multigrid schedule (a dict of Poisson2D tuning options) for the
     vertex operator of `mesh` with mass term `maindiag`; {} when the
-    operator is solved directly (FFT or capacitance solve: nothing to
+    operator is solved directly (FFT, eigenvector or capacitance solve: nothing to
     tune)."""
-    from .elliptic import Poisson2D, get_msk_from_mesh
+    from .elliptic import DIRECT, Poisson2D, get_msk_from_mesh
     msk = get_msk_from_mesh(mesh, "v")
     key = poisson_key(mesh, msk, maindiag)
     if cache and key in _load():
@@ -130,7 +130,7 @@ def tune_poisson(mesh, maindiag=0.0, reps=4, candidates=None, cache=True, verbos
     rhs = [torch.from_numpy(r).to(mesh.device, dtype) for r in _test_rhs(mesh.shape, msk)]
     for opts in cands:
         ps = Poisson2D(mesh, "v", maindiag=maindiag, tuning=opts)
-        if ps.method in ("fft", "capacitance"):
+        if ps.method in DIRECT:
             return {}  # a direct solve: no multigrid schedule to pick
         ok = True
         for b in rhs:

@@ -39,6 +39,7 @@
 #include "f2d_capacitance.hpp"
 #include "f2d_common.hpp"
 #include "f2d_fft.hpp"
+#include "f2d_modal.hpp"
 #include "f2d_neumann.hpp"
 
 namespace f2d {
@@ -1517,6 +1518,7 @@ struct f2d_poisson {
   f2d::FftSolver* fft = nullptr;  // direct spectral solve, when it applies
   f2d::NeumannSolver* neu = nullptr;  // Neumann (cell) operator: Jacobi-PCG
   f2d::CapSolver* cap = nullptr;  // masked operator: spectral + capacitance
+  f2d::ModalSolver* modal = nullptr;  // fully wet rectangles of other sizes
   int64_t fft_unmeasured = 0;     // FFT solves made without statistics
   int refine_next = -1;  // FP32 direct solves: refinements (0: none), -1 options
   std::vector<void*> allocs;
@@ -1532,6 +1534,8 @@ static void* dalloc(f2d_poisson* h, size_t bytes) {
   h->allocs.push_back(p);
   return p;
 }
+
+static bool pow2_size(int64_t v) { return (v & (v - 1)) == 0; }
 
 static dim3 tiles(const LevelDev& L, int fc) {
   return dim3((unsigned)((L.nx + fc - 1) / fc), (unsigned)((L.ny + fc - 1) / fc));
@@ -2279,7 +2283,10 @@ int f2d_poisson_create(const int8_t* unknowns_host, const f2d_grid* g,
                                h->opts.mode == F2D_POISSON_F64);
     const bool cells_fft = h->opts.neumann && fits &&
                            fft_applicable_cells(h->ny, h->nx, h->xper, h->yper, nwet);
-    if (h->opts.neumann && !(cells_fft && h->opts.solver != F2D_SOLVER_MG)) {
+    const bool modal_ok =
+        h->opts.solver == F2D_SOLVER_AUTO && !(pow2_size(h->ny) && pow2_size(h->nx)) &&
+        modal_applicable(h->ny, h->nx, h->xper, h->yper, nwet, h->opts.neumann != 0);
+    if (h->opts.neumann && !modal_ok && !(cells_fft && h->opts.solver != F2D_SOLVER_MG)) {
       F2D_REQUIRE(h->opts.solver != F2D_SOLVER_FFT,
                   "FFT solver requested for a Neumann operator with dry cells or sizes "
                   "that are not powers of two");
@@ -2339,10 +2346,19 @@ int f2d_poisson_create(const int8_t* unknowns_host, const f2d_grid* g,
                           h->opts.mode == F2D_POISSON_F64,
                           h->opts.mode != F2D_POISSON_F64, h->xper, h->yper,
                           h->opts.neumann != 0);
+    // any other fully wet rectangle: the eigenvector solve.  Multigrid CG
+    // took 2.17 ms a solve on an 800 x 304 channel (0.1 ms a whole stage
+    // now), Jacobi-PCG 4.4 ms on the 40^2 cell operator, and multigrid does
+    // not converge where halving leaves a coarsest level of many points
+    // (300^2, 500^2, 1000^2).  (Grids of two powers of two that the FFT's LDS
+    // limit excludes keep multigrid.)
+    if (!h->fft && modal_ok)
+      h->modal = modal_create(h->ny, h->nx, g->dx, g->dy, maindiag, h->xper, h->yper,
+                              h->opts.neumann != 0);
     // a masked vertex operator inside a rectangle the spectral solve
     // handles: the direct capacitance solve (auto: with a boundary of at
     // most CAP_AUTO_MAX points, and multigrid if its set-up fails)
-    if (!h->fft && !h->opts.neumann && h->opts.solver != F2D_SOLVER_MG &&
+    if (!h->fft && !h->modal && !h->opts.neumann && h->opts.solver != F2D_SOLVER_MG &&
         h->opts.mode != F2D_POISSON_F32) {
       const bool f64m = h->opts.mode == F2D_POISSON_F64;
       const int64_t nb = cap_boundary(m.data(), h->ny, h->nx, h->xper, h->yper, maindiag, f64m);
@@ -2369,6 +2385,7 @@ int f2d_poisson_create(const int8_t* unknowns_host, const f2d_grid* g,
   });
   if (rc != 0 && h) {
     if (h->fft) fft_destroy(h->fft);
+    if (h->modal) modal_destroy(h->modal);
     if (h->cap) cap_destroy(h->cap);
     if (h->neu) neu_destroy(h->neu);
     for (void* p : h->allocs) (void)hipFree(p);
@@ -2382,6 +2399,7 @@ int f2d_poisson_destroy(f2d_poisson* h) {
     if (!h) return;
     F2D_HIP(hipDeviceSynchronize());
     if (h->fft) fft_destroy(h->fft);
+    if (h->modal) modal_destroy(h->modal);
     if (h->cap) cap_destroy(h->cap);
     if (h->neu) neu_destroy(h->neu);
     for (void* p : h->allocs) F2D_HIP(hipFree(p));
@@ -2427,6 +2445,13 @@ static int solve_common(f2d_poisson* h, const void* b, void* x, int gmode,
                       h->opts.fft_warm != 0, sync, c->stats, s);
         fill_x<float>(h, (float*)x, s);
       }
+      if (!sync) h->fft_unmeasured++;
+    } else if (h->modal) {
+      Ctl* c = mode == F2D_POISSON_F64 ? h->p64.ctl : h->p32.ctl;
+      if (mode == F2D_POISSON_F64)
+        modal_solve<double>(h->modal, (const double*)b, gmode, (double*)x, sync, c->stats, s);
+      else
+        modal_solve<float>(h->modal, (const float*)b, gmode, (float*)x, sync, c->stats, s);
       if (!sync) h->fft_unmeasured++;
     } else if (h->fft) {
       Ctl* c = mode == F2D_POISSON_F64 ? h->p64.ctl : h->p32.ctl;
@@ -2485,6 +2510,7 @@ int f2d_poisson_method(f2d_poisson* h) {
   if (!h) return -1;
   if (h->neu) return F2D_SOLVER_NEUMANN_CG;
   if (h->cap) return F2D_SOLVER_CAP;
+  if (h->modal) return F2D_SOLVER_MODAL;
   return h->fft ? F2D_SOLVER_FFT : F2D_SOLVER_MG;
 }
 

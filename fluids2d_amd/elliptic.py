@@ -19,6 +19,10 @@ DEFAULT_RTOL = {"fp64": 1e-13, "fp32": 1e-9}
 DEFAULT_MAXIT = {"fp64": 100, "fp32": 8}
 
 
+# methods that solve directly: no iteration count to learn, no rtol test
+DIRECT = ("fft", "capacitance", "modal")
+
+
 def _destroy(h, name="f2d_poisson_destroy"):
     try:
         getattr(_lib.lib(), name)(h)
@@ -109,8 +113,9 @@ class Poisson2D:
                   self.maindiag, ctypes.byref(opts), ctypes.byref(h))
         self._h = h
         # "fft": direct spectral solve (exact to rounding, no rtol test);
-        # "mg": multigrid-preconditioned CG to rtol
-        self.method = {2: "fft", 3: "neumann", 4: "capacitance"}.get(
+        # "modal": direct eigenvector solve; "capacitance": direct masked
+        # solve; "mg": multigrid-preconditioned CG to rtol
+        self.method = {2: "fft", 3: "neumann", 4: "capacitance", 5: "modal"}.get(
             _lib.lib().f2d_poisson_method(h), "mg")
         self.last_iters = 0
         self.last_relres = 0.0
@@ -182,7 +187,7 @@ class Poisson2D:
         return None
 
     def _accepted(self, relres):
-        if self.method in ("fft", "capacitance"):
+        if self.method in DIRECT:
             # direct: exact up to rounding.  FP32 transforms refined once from
             # the previous solution: the FP64 residual of FP32 rounding at
             # the high wavenumbers (the operator amplifies them by k^2)
@@ -245,7 +250,7 @@ class Poisson2D:
     def graph_replayed(self, nsolves, captured):
         """Account for the direct solves of a graph replay (nsolves) and of
         its capture (captured, enqueued but never run)."""
-        if self.method in ("fft", "capacitance"):
+        if self.method in DIRECT:
             self.replayed += nsolves - captured
 
     def read_stats(self):

@@ -23,6 +23,7 @@ import torch
 
 from . import _lib
 from . import operators as op
+from .elliptic import DIRECT
 from .equations import _Base
 from .states import allocate_device, leaves
 
@@ -352,8 +353,8 @@ _Du = namedtuple("prognostic", ("u",))
 class Euler(_SW):
     """Euler in momentum-pressure form (equations.py:9-24): vortex force and
     kinetic-energy gradient, then the pressure projection
-    (operators.py:114-119) with the Neumann cell Poisson solve.  With the
-    direct solve (all-wet domains, power-of-two sizes) stages may skip the
+    (operators.py:114-119) with the Neumann cell Poisson solve.  With a
+    direct solve (all-wet domains) stages may skip the
     host check and steps are graph-captured; the Jacobi-PCG solve always
     checks convergence on the host, so its steps are not."""
     prognostic = ("u",)
@@ -361,7 +362,7 @@ class Euler(_SW):
 
     @property
     def capturable(self):
-        return self.mesh.poisson_centers.method == "fft"
+        return self.mesh.poisson_centers.method in DIRECT
 
     def rhs(self, s, ds):
         m, p = self.mesh, self.param
@@ -384,7 +385,7 @@ class Euler(_SW):
              _lib.ptr(s.div))
         rhs = s.div * (-m.area)
         pc = m.poisson_centers
-        pc.solve(rhs, s.p, stats=self._stats if pc.method == "fft" else True)
+        pc.solve(rhs, s.p, stats=self._stats if pc.method in DIRECT else True)
         _ops("f2d_addgrad", dt, g, _lib.ptr(s.p), _lib.ptr(m.d_mskx), _lib.ptr(m.d_msky),
              _lib.ptr(s.u.x), _lib.ptr(s.u.y))
         op.fill(m, s.u.x)

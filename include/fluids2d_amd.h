@@ -449,7 +449,9 @@ typedef struct f2d_poisson_opts {
                             neighbours' coefficients minus maindiag).  Every
                             cell wet and power-of-two sizes: the direct
                             solve (even extensions about closed walls; zero
-                            mean when singular) unless solver is MG; else
+                            mean when singular) unless solver is MG; every
+                            cell wet, other sizes and solver AUTO: the
+                            eigenvector solve; else
                             Jacobi-preconditioned CG in FP64 (x keeps the
                             constant of its initial guess)                 */
 } f2d_poisson_opts;
@@ -460,11 +462,18 @@ typedef struct f2d_poisson_opts {
  * extension on the doubled periodic grid; the operator is then diagonalised
  * by the 2-D DFT) and, in F2D_POISSON_F64, the transformed (doubled when
  * closed) sizes are at most 2048 (one row in a workgroup's LDS); the
- * multigrid-preconditioned CG otherwise. */
+ * eigenvector solve (F2D_SOLVER_MODAL) for a fully wet rectangle of other
+ * sizes; the multigrid-preconditioned CG otherwise. */
 #define F2D_SOLVER_AUTO 0
 #define F2D_SOLVER_MG 1
 #define F2D_SOLVER_FFT 2
 #define F2D_SOLVER_NEUMANN_CG 3  /* reported by f2d_poisson_method only */
+/* Reported by f2d_poisson_method only: the direct solve AUTO takes for a
+ * fully wet rectangle (closed, periodic or mixed; vertex or Neumann cell
+ * operator) of sizes 8 to 4096 that are not both powers of two.  Dense
+ * transforms by the eigenvectors of the two second differences, FP64 in
+ * every mode; zero mean when singular.  Statistics as the FFT solve's. */
+#define F2D_SOLVER_MODAL 5
 /* The masked vertex operator of a mask inside a rectangle the FFT solve
  * handles (power-of-two sizes, a closed direction or maindiag > 0): the
  * masked operator is the rectangle operator's principal submatrix on the
@@ -491,9 +500,9 @@ int f2d_poisson_destroy(f2d_poisson* h);
 int f2d_poisson_solve(f2d_poisson* h, const void* b, void* x, double rtol,
                       int maxit, int* iters, double* relres, void* stream);
 /* The method a handle solves with, F2D_SOLVER_MG, F2D_SOLVER_FFT,
- * F2D_SOLVER_NEUMANN_CG or F2D_SOLVER_CAP (-1 for NULL); no counterpart in
- * the reference, whose SuperLU factor is its only method (elliptic.py:78).
- * With FFT or CAP the solve is direct: `maxit` is unused, *iters receives
+ * F2D_SOLVER_NEUMANN_CG, F2D_SOLVER_CAP or F2D_SOLVER_MODAL (-1 for NULL);
+ * no counterpart in the reference, whose SuperLU factor is its only method
+ * (elliptic.py:78).  With FFT, CAP or MODAL the solve is direct: `maxit` is unused, *iters receives
  * 1 + the FP64 refinements, *relres the measured true relative residual,
  * and the solve counts as converged when that residual is below 1e-6
  * (`rtol` is not its acceptance test: a direct FP64 solve reaches eps times
