@@ -52,6 +52,7 @@ struct ModalPass {
   // pass 4: first unknown of the padded array, wrap sizes (0: closed)
   int64_t x0;
   int wx, wy;          // periods for the halo images of columns and rows
+  const double* skip;  // device flag: nonzero, the pass does nothing (may be NULL)
 };
 
 enum { EPI_MODES = 0, EPI_SCALED = 1, EPI_POINTS = 2, EPI_PADDED = 3 };
@@ -98,6 +99,7 @@ __global__ __launch_bounds__(256, 2) void k_modal(ModalPass a) {
   const int per = (int)(gridDim.x >> 3);
   const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
   if (tile >= njt * nmt) return;
+  if (a.skip && *a.skip != 0.0) return;
   const int m0 = (tile / njt) * BM, j0 = (tile % njt) * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wk = wave % WK, wn = (wave / WK) % WN, wm = wave / (WK * WN);
@@ -571,11 +573,12 @@ static void launch_pass(const ModalPass& a, hipStream_t s) {
 
 template <class T>
 void modal_solve(ModalSolver* m, const T* b, int gmode, T* x, bool measure, double* stats,
-                 hipStream_t s) {
+                 hipStream_t s, const double* skip) {
   const ModalDir &dx = m->x, &dy = m->y;
   F2D_REQUIRE(!gmode || (dx.cell && dy.cell), "the cell operator takes b on the cells");
   // 1: rows of b -> modes of x (t1: one row per mode)
   ModalPass a{};
+  a.skip = skip;
   a.mat = gmode ? dx.cell : dx.fwd;
   a.in = b + (gmode ? m->c0 : m->k0);
   a.out = m->t1;
@@ -593,6 +596,7 @@ void modal_solve(ModalSolver* m, const T* b, int gmode, T* x, bool measure, doub
   launch_pass<true, EPI_MODES, T, double>(a, s);
   // 2: -> modes of y, divided by the eigenvalues (t2)
   ModalPass p{};
+  p.skip = skip;
   p.mat = gmode ? dy.cell : dy.fwd;
   p.in = m->t1;
   p.out = m->t2;
@@ -612,6 +616,7 @@ void modal_solve(ModalSolver* m, const T* b, int gmode, T* x, bool measure, doub
   launch_pass<true, EPI_SCALED, double, double>(p, s);
   // 3: modes of x -> points of x (t1)
   ModalPass q{};
+  q.skip = skip;
   q.mat = dx.back;
   q.in = m->t2;
   q.out = m->t1;
@@ -629,6 +634,7 @@ void modal_solve(ModalSolver* m, const T* b, int gmode, T* x, bool measure, doub
   launch_pass<false, EPI_POINTS, double, double>(q, s);
   // 4: modes of y -> x
   ModalPass r{};
+  r.skip = skip;
   r.mat = dy.back;
   r.in = m->t1;
   r.out = x;
@@ -658,8 +664,8 @@ void modal_solve(ModalSolver* m, const T* b, int gmode, T* x, bool measure, doub
 }
 
 template void modal_solve<double>(ModalSolver*, const double*, int, double*, bool, double*,
-                                  hipStream_t);
+                                  hipStream_t, const double*);
 template void modal_solve<float>(ModalSolver*, const float*, int, float*, bool, double*,
-                                 hipStream_t);
+                                 hipStream_t, const double*);
 
 }  // namespace f2d

@@ -32,9 +32,10 @@ void modal_destroy(ModalSolver* m);
 // at the unknowns; 1 (vertices): b = centerstovertices of the cell field
 // (operators.py:126-133, formed inside the first transform: the averaged
 // eigenvectors).  measure: the relative residual goes to `stats` (8 doubles,
-// device), as the other direct solves record it.
+// device), as the other direct solves record it.  skip: a device flag; the
+// passes of a solve enqueued behind a nonzero one do nothing.
 template <class T>
 void modal_solve(ModalSolver* m, const T* b, int gmode, T* x, bool measure, double* stats,
-                 hipStream_t s);
+                 hipStream_t s, const double* skip = nullptr);
 
 }  // namespace f2d

@@ -2,7 +2,8 @@
 // get_Laplacian_sparse (elliptic.py:114-195, neumann branch of :186-190):
 // the off-diagonals dy/dx (E/W) and dx/dy (N/S) of the unknown neighbours
 // (x-periodic wrap, y-periodic as an extension), the diagonal minus their
-// sum minus maindiag.  Solved by Jacobi-preconditioned CG in FP64.
+// sum minus maindiag.  Solved in FP64 by CG, preconditioned by the direct
+// solve of the whole rectangle or by the diagonal (Jacobi).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -13,9 +14,11 @@ namespace f2d {
 
 struct NeumannSolver;
 
-// m_host: int8 unknown mask on the padded (ny+6) x (nx+6) grid (interior only)
+// m_host: int8 unknown mask on the padded (ny+6) x (nx+6) grid (interior
+// only).  direct: precondition by the rectangle's direct solve where one
+// takes the grid (sizes 8 to 4096)
 NeumannSolver* neu_create(const int8_t* m_host, int64_t ny, int64_t nx, int xper,
-                          int yper, double dx, double dy, double maindiag);
+                          int yper, double dx, double dy, double maindiag, bool direct);
 void neu_destroy(NeumannSolver* n);
 
 // Solve A x = b at the unknowns (b, x of dtype F2D_F64 or F2D_F32, padded;

@@ -2290,7 +2290,8 @@ int f2d_poisson_create(const int8_t* unknowns_host, const f2d_grid* g,
       F2D_REQUIRE(h->opts.solver != F2D_SOLVER_FFT,
                   "FFT solver requested for a Neumann operator with dry cells or sizes "
                   "that are not powers of two");
-      h->neu = neu_create(m.data(), h->ny, h->nx, h->xper, h->yper, g->dx, g->dy, maindiag);
+      h->neu = neu_create(m.data(), h->ny, h->nx, h->xper, h->yper, g->dx, g->dy, maindiag,
+                          h->opts.solver != F2D_SOLVER_MG);
       *out = h;
       return;
     }
