@@ -470,8 +470,8 @@ int64_t cap_boundary(const int8_t* unk, int64_t ny, int64_t nx, int xper, int yp
   if (xper && yper && maindiag == 0.0) return -1;  // singular rectangle
   const int64_t nx2 = xper ? nx : 2 * nx, ny2 = yper ? ny : 2 * ny;
   // the Green's function is an FP64 spectral solve on the doubled grid
-  if (!fft_fits(ny2, nx2, 1, 1, true) || nx2 > 4096 || ny2 > 4096) return -1;
-  if (!fft_fits(ny, nx, xper, yper, f64_mode)) return -1;
+  if (!fft_fits(ny2, nx2, 1, 1, true, true) || nx2 > 4096 || ny2 > 4096) return -1;
+  if (!fft_fits(ny, nx, xper, yper, f64_mode, true)) return -1;
   const int64_t NXP = nx + 6, NYP = ny + 6;
   int64_t nw = 0, nr = 0;
   for (int64_t j = 0; j < NYP; j++)

@@ -71,6 +71,7 @@ struct FftArgs {
   // problem's sizes, NXP its padded row length.
   int ex, ey;
   int onx, ony;
+  int ipx, ipy;  // rows, columns transformed in place (fft_inplace)
 };
 
 // Forward DFTs of `nf` contiguous length-N sequences held in LDS buffer `a`
@@ -127,6 +128,36 @@ __device__ cplx<T>* fft_lds(cplx<T>* a, cplx<T>* b, int N, int lgN, int nf,
   return a;
 }
 
+// The same transform of one sequence of N = 4 blockDim points in place, for
+// lengths whose two buffers and twiddles do not fit LDS (FP64 4096): a thread
+// holds one butterfly, so a pass reads, waits for the others and writes over
+// the input.  Twiddles come from global memory (L2), which leaves a CU room
+// for two workgroups.  Same operations in the same order as fft_lds.
+// Measured: the doubly periodic 4096^2 FP64 step 36.4 ms with the multigrid
+// solve these grids had, 1.80 ms with this one.
+template <class T>
+__device__ void fft_inplace(cplx<T>* a, int N, const cplx<T>* __restrict__ tw) {
+  const int j = threadIdx.x, nb = N >> 2;
+  for (int Ns = 1; Ns < N; Ns <<= 2) {
+    const int jm = j & (Ns - 1);
+    const cplx<T>* tp = tw + (Ns - 1);
+    const cplx<T> t1 = tp[jm], t2 = tp[Ns + jm], t3 = tp[2 * Ns + jm];
+    const cplx<T> a0 = a[j];
+    const cplx<T> a1 = cmul<T>(a[j + nb], t1);
+    const cplx<T> a2 = cmul<T>(a[j + 2 * nb], t2);
+    const cplx<T> a3 = cmul<T>(a[j + 3 * nb], t3);
+    const cplx<T> b0 = cadd<T>(a0, a2), b1 = csub<T>(a0, a2);
+    const cplx<T> b2 = cadd<T>(a1, a3), b3 = csub<T>(a1, a3);
+    const int base = ((j - jm) << 2) + jm;
+    __syncthreads();
+    a[base] = cadd<T>(b0, b2);
+    a[base + Ns] = mk<T>(b1.x + b3.y, b1.y - b3.x);
+    a[base + 2 * Ns] = csub<T>(b0, b2);
+    a[base + 3 * Ns] = mk<T>(b1.x - b3.y, b1.y + b3.x);
+    __syncthreads();
+  }
+}
+
 // right-hand side at interior vertex k (padded index): b itself, or
 // centerstovertices (operators.py:126-133) of the cell field
 template <class TB>
@@ -168,6 +199,7 @@ __device__ __forceinline__ double bsum256(double v, double* sh) {
 // the FP32 step from 0.425 to 0.449 ms, 256 threads made both slower.
 template <class T>
 static inline int fft_threads(int points) {
+  // (in place, FP64 4096: exactly one butterfly a thread, 1024)
   if (sizeof(T) == 8 && points >= 2048) return 1024;
   return points >= 4096 ? 1024 : (points >= 1024 ? 512 : 256);
 }
@@ -346,7 +378,8 @@ __global__ __launch_bounds__(1024) void k_fft_rows_fwd(FftArgs a,
   cplx<T>* b0 = reinterpret_cast<cplx<T>*>(smem);
   cplx<T>* b1 = b0 + P * nx;
   cplx<T>* tl = b1 + P * nx;  // twiddles, staged in LDS
-  for (int w = threadIdx.x; w < nx; w += blockDim.x) tl[w] = tw[w];
+  if (!a.ipx)
+    for (int w = threadIdx.x; w < nx; w += blockDim.x) tl[w] = tw[w];
   const int y0 = row_block(blockIdx.x, gridDim.x) * 2 * P;
   double mb = 0.0;
   if ((x64 || x32) && bpin) {
@@ -433,7 +466,11 @@ __global__ __launch_bounds__(1024) void k_fft_rows_fwd(FftArgs a,
     if (threadIdx.x == 0) bpart[blockIdx.x] = sum;
   }
   __syncthreads();
-  const cplx<T>* r = fft_lds<T>(b0, b1, nx, lg, P, tl);
+  const cplx<T>* r = b0;
+  if (a.ipx)
+    fft_inplace<T>(b0, nx, tw);
+  else
+    r = fft_lds<T>(b0, b1, nx, lg, P, tl);
   // half spectra of the two rows: Xa = (C + D) / 2, Xb = -i (C - D) / 2 with
   // C = F(k), D = conj(F(nx - k))
   const int n2 = a.nk * 2 * P;
@@ -569,9 +606,14 @@ __global__ __launch_bounds__(1024) void k_fft_cols(FftArgs a,
   } else {
     for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) b0[w] = col[w];
   }
-  for (int w = threadIdx.x; w < ny; w += blockDim.x) tl[w] = tw[w];
+  if (!a.ipy)
+    for (int w = threadIdx.x; w < ny; w += blockDim.x) tl[w] = tw[w];
   __syncthreads();
-  cplx<T>* r = fft_lds<T>(b0, b1, ny, lg, nq, tl);
+  cplx<T>* r = b0;
+  if (a.ipy)
+    fft_inplace<T>(b0, ny, tw);
+  else
+    r = fft_lds<T>(b0, b1, ny, lg, nq, tl);
   cplx<T>* o = r == b0 ? b1 : b0;
   const double inv = 1.0 / ((double)a.nx * (double)a.ny);
   for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) {
@@ -582,7 +624,11 @@ __global__ __launch_bounds__(1024) void k_fft_cols(FftArgs a,
     r[w] = mk<T>(v.x * s, -(v.y * s));  // conjugate: inverse by forward
   }
   __syncthreads();
-  const cplx<T>* z = fft_lds<T>(r, o, ny, lg, nq, tl);
+  const cplx<T>* z = r;
+  if (a.ipy)
+    fft_inplace<T>(r, ny, tw);
+  else
+    z = fft_lds<T>(r, o, ny, lg, nq, tl);
   // (closed y: the row pass reads the problem's rows only)
   for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) {
     if (a.ey && (w & (ny - 1)) >= a.ony) continue;
@@ -634,33 +680,33 @@ __global__ __launch_bounds__(1024) void k_fft_rows_inv(FftArgs a,
   cplx<T>* b0 = reinterpret_cast<cplx<T>*>(smem);
   cplx<T>* b1 = b0 + P * nx;
   cplx<T>* tl = b1 + P * nx;
-  for (int w = threadIdx.x; w < nx; w += blockDim.x) tl[w] = tw[w];
+  if (!a.ipx)
+    for (int w = threadIdx.x; w < nx; w += blockDim.x) tl[w] = tw[w];
   const int y0 = row_block(blockIdx.x, gridDim.x) * 2 * P;
-  // Xa -> b1, Xb -> b0 (k = 0 .. nx/2)
-  const int n2 = a.nk * 2 * P;
+  // conj(C) with C(k) = Xa(k) + i Xb(k) and C(nx - k) = conj(Xa(k)) +
+  // i conj(Xb(k)), k = 0 .. nx/2: a thread reads both rows' entries of its k
   const int lgP = __ffs(P) - 1;  // P is a power of two
-  for (int w = threadIdx.x; w < n2; w += blockDim.x) {
-    const int ab = w & 1, p = (w >> 1) & (P - 1), k = (w >> 1) >> lgP;
-    const int64_t at = (int64_t)k * a.ny + y0 + 2 * p + ab;
-    cplx<T> X;
+  for (int w = threadIdx.x; w < a.nk * P; w += blockDim.x) {
+    const int p = w & (P - 1), k = w >> lgP;
+    const int64_t at = (int64_t)k * a.ny + y0 + 2 * p;
+    cplx<T> Xa, Xb;
     if (a.ex == 1) {  // odd x: the imaginary part stored
-      X = mk<T>(T(0), reinterpret_cast<const T*>(S)[at]);
+      Xa = mk<T>(T(0), reinterpret_cast<const T*>(S)[at]);
+      Xb = mk<T>(T(0), reinterpret_cast<const T*>(S)[at + 1]);
     } else {
-      X = S[at];
+      Xa = S[at];
+      Xb = S[at + 1];
     }
-    (ab == 0 ? b1 : b0)[p * nx + k] = X;
+    cplx<T>* c = b0 + p * nx;
+    c[k] = mk<T>(Xa.x - Xb.y, -(Xa.y + Xb.x));
+    if (k > 0 && k < h) c[nx - k] = mk<T>(Xa.x + Xb.y, -(Xb.x - Xa.y));
   }
   __syncthreads();
-  // conj(C) with C(k) = Xa(k) + i Xb(k) and C(nx - k) = conj(Xa(k)) +
-  // i conj(Xb(k)), written over b1 (each thread reads its own k first)
-  for (int p = 0; p < P; p++)
-    for (int k = threadIdx.x; k <= h; k += blockDim.x) {
-      const cplx<T> Xa = b1[p * nx + k], Xb = b0[p * nx + k];
-      b1[p * nx + k] = mk<T>(Xa.x - Xb.y, -(Xa.y + Xb.x));
-      if (k > 0 && k < h) b1[p * nx + nx - k] = mk<T>(Xa.x + Xb.y, -(Xb.x - Xa.y));
-    }
-  __syncthreads();
-  const cplx<T>* r = fft_lds<T>(b1, b0, nx, lg, P, tl);
+  const cplx<T>* r = b0;
+  if (a.ipx)
+    fft_inplace<T>(b0, nx, tw);
+  else
+    r = fft_lds<T>(b0, b1, nx, lg, P, tl);
   // conj of the result: row a = Re, row b = -Im of r
   for (int w = threadIdx.x; w < P * nx; w += blockDim.x) {
     const int p = w >> lg, n = w & (nx - 1);
@@ -879,12 +925,20 @@ static int ilog2(int64_t v) {
 
 static bool pow2(int64_t v) { return v > 0 && (v & (v - 1)) == 0; }
 
-bool fft_fits(int64_t ny, int64_t nx, int xper, int yper, bool f64) {
+// a transform of n points in place: 4096 points of a workgroup of 1024
+// threads, where two buffers and the twiddles exceed the LDS
+static bool inplace(int64_t n, bool f64) { return f64 && n == 4096; }
+
+bool fft_fits(int64_t ny, int64_t nx, int xper, int yper, bool f64, bool two_buffers) {
   // one row (column) per workgroup: two FFT buffers and the twiddles in LDS
-  // (plan_blocks)
+  // (plan_blocks), or 4096 points of a periodic direction in place (closed
+  // directions: the column pass of an odd x reads a mirror entry)
   const size_t c = f64 ? 16 : 8;
   const int64_t tx = xper ? nx : 2 * nx, ty = yper ? ny : 2 * ny;
-  return 3 * (size_t)tx * c <= 160 * 1024 && 3 * (size_t)ty * c <= 160 * 1024;
+  auto lds = [&](int64_t n) { return 3 * (size_t)n * c <= 160 * 1024; };
+  const bool okx = lds(tx) || (!two_buffers && inplace(tx, f64) && xper);
+  const bool oky = lds(ty) || (!two_buffers && inplace(ty, f64) && xper && yper);
+  return okx && oky;
 }
 
 bool fft_applicable_cells(int64_t ny, int64_t nx, int xper, int yper, int64_t nwet) {
@@ -951,13 +1005,14 @@ static void plan_blocks(const FftArgs& a, int& P, int& Q, size_t& lr, size_t& lc
   // (odd x: a unit is a pair of columns; as many workgroups as unpaired)
   if (a.ex == 1 && Q > 1) Q >>= 1;
   while (Q > 1 && (2 * Q + 1) * a.ny * c > LDS_CAP) Q >>= 1;
-  lr = (2 * (size_t)P + 1) * a.nx * c;
-  lc = (2 * (size_t)Q + 1) * a.ny * c;
+  lr = (a.ipx ? 1 : 2 * (size_t)P + 1) * a.nx * c;
+  lc = (a.ipy ? 1 : 2 * (size_t)Q + 1) * a.ny * c;
 }
 
 template <class T>
 static void set_lds(size_t lr, size_t lc) {
-  if (lr > 64 * 1024) {
+  // (the row passes hold 2 KB of static LDS besides)
+  if (lr > 62 * 1024) {
     F2D_HIP(hipFuncSetAttribute((const void*)k_fft_rows_fwd<T, double>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr));
     F2D_HIP(hipFuncSetAttribute((const void*)k_fft_rows_fwd<T, float>,
@@ -968,8 +1023,10 @@ static void set_lds(size_t lr, size_t lc) {
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr));
     F2D_HIP(hipFuncSetAttribute((const void*)k_fft_rows_inv<T, T, 2>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr));
+    F2D_HIP(hipFuncSetAttribute((const void*)k_fft_rows_inv<T, T, 3>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr));
   }
-  if (lc > 64 * 1024)
+  if (lc > 62 * 1024)
     F2D_HIP(hipFuncSetAttribute((const void*)k_fft_cols<T>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lc));
 }
@@ -1020,6 +1077,10 @@ FftSolver* fft_create(int64_t ny, int64_t nx, double dx, double dy,
     f->rowsum[0] = falloc<double>(f, sizeof(double) * (ny / 2 + 1));
     f->rowsum[1] = falloc<double>(f, sizeof(double) * (ny / 2 + 1));
     if (f64) {
+      // (a plan of both precisions would share these: none is made)
+      a.ipx = inplace(nx, true) ? 1 : 0;
+      a.ipy = inplace(ny, true) ? 1 : 0;
+      F2D_REQUIRE(!(a.ipx || a.ipy) || !f32, "in-place plans are FP64 only");
       f->twx64 = twiddles<double2>(f, (int)nx);
       f->twy64 = twiddles<double2>(f, (int)ny);
       f->S64 = falloc<double2>(f, sizeof(double2) * nspec);

@@ -2279,8 +2279,10 @@ int f2d_poisson_create(const int8_t* unknowns_host, const f2d_grid* g,
     h->nwet = (double)nwet;
     // the Neumann cell operator: the direct solve when every cell is wet
     // (closed directions as even extensions), Jacobi-PCG otherwise
+    // (an explicit request keeps to the two-buffer transforms)
     const bool fits = fft_fits(h->ny, h->nx, h->xper, h->yper,
-                               h->opts.mode == F2D_POISSON_F64);
+                               h->opts.mode == F2D_POISSON_F64,
+                               h->opts.solver == F2D_SOLVER_FFT);
     const bool cells_fft = h->opts.neumann && fits &&
                            fft_applicable_cells(h->ny, h->nx, h->xper, h->yper, nwet);
     const bool modal_ok =

@@ -461,7 +461,8 @@ typedef struct f2d_poisson_opts {
  * two in [8, 4096] ([8, 2048] in a closed direction, solved as the odd
  * extension on the doubled periodic grid; the operator is then diagonalised
  * by the 2-D DFT) and, in F2D_POISSON_F64, the transformed (doubled when
- * closed) sizes are at most 2048 (one row in a workgroup's LDS); the
+ * closed) sizes are at most 2048 (one row in a workgroup's LDS), or 4096 in
+ * a periodic direction (x periodic; transformed in place, AUTO only); the
  * eigenvector solve (F2D_SOLVER_MODAL) for a fully wet rectangle of other
  * sizes; the multigrid-preconditioned CG otherwise. */
 #define F2D_SOLVER_AUTO 0
