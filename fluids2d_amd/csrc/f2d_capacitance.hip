@@ -16,6 +16,10 @@
 //   k_cap_out    x = y at the unknowns W
 // The FP32 mode wraps the same sequence, in FP32 with an FP32 M, into FP64
 // refinement (k_cap_res forms the FP64 residual, k_cap_acc accumulates).
+//
+// Rectangles whose sizes are not powers of two take the eigenvector solve
+// (f2d_modal) in place of the spectral passes, in FP64 for every precision of
+// b and x: no refinement to make, and its last pass writes x at W itself.
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>
 
@@ -24,6 +28,7 @@
 
 #include "f2d_capacitance.hpp"
 #include "f2d_fft.hpp"
+#include "f2d_modal.hpp"
 
 namespace f2d {
 
@@ -282,8 +287,10 @@ __global__ __launch_bounds__(256) void k_cap_norms(CapGeo g, const TB* __restric
 // one block: relative residual into the solve statistics
 // [iterations, relres, converged, refinements | failed, max, solves]
 // (a direct solve is accepted unless its residual is above 1e-6 or not finite)
+// nan_fails: a norm that is not a number is reported (as multigrid does)
 __global__ __launch_bounds__(256) void k_cap_stats(const double* __restrict__ part, int nb,
-                                                   int passes, double* __restrict__ st) {
+                                                   int passes, int nan_fails,
+                                                   double* __restrict__ st) {
   __shared__ double sh[4];
   double a = 0.0, c = 0.0;
   for (int i = threadIdx.x; i < nb; i += 256) {
@@ -293,7 +300,8 @@ __global__ __launch_bounds__(256) void k_cap_stats(const double* __restrict__ pa
   a = bsum(a, sh);
   c = bsum(c, sh);
   if (threadIdx.x != 0) return;
-  const double rel = c > 0.0 ? sqrt(a / c) : 0.0;
+  double rel = c > 0.0 ? sqrt(a / c) : 0.0;
+  if (nan_fails && !(a - a == 0.0 && c - c == 0.0)) rel = NAN;
   const double conv = (rel <= 1e-6) ? 1.0 : 0.0;
   st[0] = (double)passes;
   st[1] = rel;
@@ -422,7 +430,8 @@ struct CapSolver {
   double* part = nullptr;   // residual-norm partials
   int nbres = 0;
   bool solved = false;      // a warm start needs an earlier solve
-  FftSolver* fft = nullptr; // the rectangle's spectral solve
+  FftSolver* fft = nullptr; // the rectangle's spectral solve, or
+  ModalSolver* modal = nullptr;  // its eigenvector solve (f64 then)
   std::vector<void*> allocs;
 };
 
@@ -465,13 +474,18 @@ static std::vector<int64_t> boundary_points(const int8_t* unk, int64_t ny, int64
 }
 
 int64_t cap_boundary(const int8_t* unk, int64_t ny, int64_t nx, int xper, int yper,
-                     double maindiag, bool f64_mode) {
-  if (!pw2(nx) || !pw2(ny)) return -1;
+                     double maindiag, bool f64_mode, bool modal) {
   if (xper && yper && maindiag == 0.0) return -1;  // singular rectangle
   const int64_t nx2 = xper ? nx : 2 * nx, ny2 = yper ? ny : 2 * ny;
-  // the Green's function is an FP64 spectral solve on the doubled grid
-  if (!fft_fits(ny2, nx2, 1, 1, true, true) || nx2 > 4096 || ny2 > 4096) return -1;
-  if (!fft_fits(ny, nx, xper, yper, f64_mode, true)) return -1;
+  if (modal) {
+    // the Green's function is an eigenvector solve on the doubled grid
+    if ((pw2(nx) && pw2(ny)) || nx < 8 || ny < 8 || nx2 > 4096 || ny2 > 4096) return -1;
+  } else {
+    if (!pw2(nx) || !pw2(ny)) return -1;
+    // the Green's function is an FP64 spectral solve on the doubled grid
+    if (!fft_fits(ny2, nx2, 1, 1, true, true) || nx2 > 4096 || ny2 > 4096) return -1;
+    if (!fft_fits(ny, nx, xper, yper, f64_mode, true)) return -1;
+  }
   const int64_t NXP = nx + 6, NYP = ny + 6;
   int64_t nw = 0, nr = 0;
   for (int64_t j = 0; j < NYP; j++)
@@ -493,11 +507,13 @@ static void rocblas_check(rocblas_status st, const char* what) {
 }
 
 CapSolver* cap_create(const int8_t* unk, int64_t ny, int64_t nx, double dx, double dy,
-                      double maindiag, int xper, int yper, bool f64_mode) {
-  F2D_REQUIRE(cap_boundary(unk, ny, nx, xper, yper, maindiag, f64_mode) > 0,
+                      double maindiag, int xper, int yper, bool f64_mode, bool modal) {
+  F2D_REQUIRE(cap_boundary(unk, ny, nx, xper, yper, maindiag, f64_mode, modal) > 0,
               "capacitance solve does not apply to this operator");
+  if (modal) f64_mode = true;
   CapSolver* c = new CapSolver();
   FftSolver* gfs = nullptr;
+  ModalSolver* gms = nullptr;
   rocblas_handle rb = nullptr;
   try {
     const int64_t NXP = nx + 6, NYP = ny + 6, N = NXP * NYP;
@@ -537,7 +553,10 @@ CapSolver* cap_create(const int8_t* unk, int64_t ny, int64_t nx, double dx, doub
     // direction: the zero-mean solution, whose constant the odd images cancel.
     const int64_t nx2 = xper ? nx : 2 * nx, ny2 = yper ? ny : 2 * ny;
     const int64_t N2 = (nx2 + 6) * (ny2 + 6);
-    gfs = fft_create(ny2, nx2, dx, dy, maindiag, true, false, 1, 1);
+    if (modal)
+      gms = modal_create(ny2, nx2, dx, dy, maindiag, 1, 1, false);
+    else
+      gfs = fft_create(ny2, nx2, dx, dy, maindiag, true, false, 1, 1);
     double* src = nullptr;
     double* G = nullptr;
     F2D_HIP(hipMalloc(&src, sizeof(double) * N2));
@@ -546,7 +565,10 @@ CapSolver* cap_create(const int8_t* unk, int64_t ny, int64_t nx, double dx, doub
     F2D_HIP(hipMemset(G, 0, sizeof(double) * N2));
     const double one = 1.0;
     F2D_HIP(hipMemcpy(src + 3 * (nx2 + 6) + 3, &one, sizeof(double), hipMemcpyHostToDevice));
-    fft_solve_f64(gfs, src, 0, G, 0.0, false, nullptr, 0);
+    if (modal)
+      modal_solve(gms, src, 0, G, false, nullptr, 0);
+    else
+      fft_solve_f64(gfs, src, 0, G, 0.0, false, nullptr, 0);
     double* A = nullptr;
     F2D_HIP(hipMalloc(&A, sizeof(double) * (size_t)n * n));
     const int64_t ne = (int64_t)n * n;
@@ -558,6 +580,8 @@ CapSolver* cap_create(const int8_t* unk, int64_t ny, int64_t nx, double dx, doub
     (void)hipFree(G);
     fft_destroy(gfs);
     gfs = nullptr;
+    modal_destroy(gms);
+    gms = nullptr;
 
     // M = (-C)^-1 by Cholesky factorisation and inversion (lower triangle)
     rocblas_check(rocblas_create_handle(&rb), "rocblas_create_handle");
@@ -597,11 +621,15 @@ CapSolver* cap_create(const int8_t* unk, int64_t ny, int64_t nx, double dx, doub
     if (!f64_mode) c->x64 = (double*)calloc_dev(c, sizeof(double) * (size_t)N);
     c->nbres = (int)((N + 255) / 256);
     c->part = (double*)calloc_dev(c, sizeof(double) * 2 * c->nbres);
-    c->fft = fft_create(ny, nx, dx, dy, maindiag, f64_mode, !f64_mode, xper, yper);
+    if (modal)
+      c->modal = modal_create(ny, nx, dx, dy, maindiag, xper, yper, false);
+    else
+      c->fft = fft_create(ny, nx, dx, dy, maindiag, f64_mode, !f64_mode, xper, yper);
     F2D_HIP(hipDeviceSynchronize());
   } catch (...) {
     if (rb) rocblas_destroy_handle(rb);
     if (gfs) fft_destroy(gfs);
+    if (gms) modal_destroy(gms);
     cap_destroy(c);
     throw;
   }
@@ -612,11 +640,14 @@ void cap_destroy(CapSolver* c) {
   if (!c) return;
   (void)hipDeviceSynchronize();
   if (c->fft) fft_destroy(c->fft);
+  if (c->modal) modal_destroy(c->modal);
   for (void* p : c->allocs) (void)hipFree(p);
   delete c;
 }
 
 int64_t cap_size(const CapSolver* c) { return c ? c->n : 0; }
+
+bool cap_modal(const CapSolver* c) { return c->modal != nullptr; }
 
 static unsigned blocks(int64_t n) { return (unsigned)((n + 255) / 256); }
 
@@ -633,12 +664,36 @@ template <class TB, class TX>
 static void measure_res(CapSolver* c, const TB* b, int gmode, const TX* x, int passes,
                         double* stats, hipStream_t s) {
   k_cap_norms<TB, TX><<<c->nbres, 256, 0, s>>>(c->g, b, gmode, c->mw, x, c->part);
-  k_cap_stats<<<1, 256, 0, s>>>(c->part, c->nbres, passes, stats);
+  k_cap_stats<<<1, 256, 0, s>>>(c->part, c->nbres, passes, c->modal != nullptr, stats);
 }
+
+template <class T>
+void cap_solve_modal(CapSolver* c, const T* b, int gmode, T* x, bool measure, double* stats,
+                     hipStream_t s) {
+  F2D_REQUIRE(c->modal, "capacitance solver built on the spectral solve");
+  const int64_t N = (int64_t)c->g.NYP * c->g.NXP;
+  double* rhs = (double*)c->rhs;
+  double* y = (double*)c->y;
+  k_cap_rhs<T, double><<<blocks(N), 256, 0, s>>>(c->g, b, gmode, c->mw, rhs);
+  modal_solve(c->modal, rhs, 0, y, false, nullptr, s);
+  gemv<double>(c, s);
+  modal_solve(c->modal, rhs, 0, x, false, nullptr, s, nullptr, c->mw);
+  if (measure && stats) {
+    // (FP32 x: the residual of the FP64 result, as modal_solve measures it)
+    if (sizeof(T) == 4) modal_solve(c->modal, rhs, 0, y, false, nullptr, s, nullptr, c->mw);
+    measure_res<T, double>(c, b, gmode, sizeof(T) == 4 ? y : (double*)x, 1, stats, s);
+  }
+  c->solved = true;
+}
+
+template void cap_solve_modal(CapSolver*, const double*, int, double*, bool, double*,
+                              hipStream_t);
+template void cap_solve_modal(CapSolver*, const float*, int, float*, bool, double*,
+                              hipStream_t);
 
 void cap_solve_f64(CapSolver* c, const double* b, int gmode, double* x, bool measure,
                    double* stats, hipStream_t s) {
-  F2D_REQUIRE(c->f64, "capacitance solver built for FP32");
+  F2D_REQUIRE(c->f64 && !c->modal, "capacitance solver built for FP32");
   const int64_t N = (int64_t)c->g.NYP * c->g.NXP;
   double* rhs = (double*)c->rhs;
   double* y = (double*)c->y;

@@ -28,15 +28,25 @@ struct CapSolver;
 // the LDS limits), the mask must not cover the whole rectangle, every
 // unknown must be a rectangle unknown, and the rectangle operator must be
 // non-singular (a closed direction or maindiag > 0).
+// modal: the rectangle is to be solved by its eigenvectors (sizes not both
+// powers of two, at most 4096, 2048 in a closed direction).
 int64_t cap_boundary(const int8_t* unk, int64_t ny, int64_t nx, int xper, int yper,
-                     double maindiag, bool f64_mode);
+                     double maindiag, bool f64_mode, bool modal = false);
 
 // f64_mode: FP64 solves (M in FP64); otherwise FP32 spectral solves and an
-// FP32 M inside FP64 refinement.  Synchronises the device.
+// FP32 M inside FP64 refinement.  modal: FP64 solves by eigenvectors whatever
+// the precision of b and x.  Synchronises the device.
 CapSolver* cap_create(const int8_t* unk, int64_t ny, int64_t nx, double dx, double dy,
-                      double maindiag, int xper, int yper, bool f64_mode);
+                      double maindiag, int xper, int yper, bool f64_mode, bool modal = false);
 void cap_destroy(CapSolver* c);
 int64_t cap_size(const CapSolver* c);
+bool cap_modal(const CapSolver* c);
+
+// x = A^-1 b of a modal solver, arguments as cap_solve_f64 (T: b's and x's
+// type, double or float)
+template <class T>
+void cap_solve_modal(CapSolver* c, const T* b, int gmode, T* x, bool measure, double* stats,
+                     hipStream_t s);
 
 // x = A^-1 b at the unknowns (other entries untouched, halo not filled).
 // gmode 0: b at the vertices; 1: b = centerstovertices of the cell field.

@@ -52,6 +52,7 @@ struct ModalPass {
   // pass 4: first unknown of the padded array, wrap sizes (0: closed)
   int64_t x0;
   int wx, wy;          // periods for the halo images of columns and rows
+  const int8_t* only;  // pass 4: write at the set points only (may be NULL)
   const double* skip;  // device flag: nonzero, the pass does nothing (may be NULL)
 };
 
@@ -64,6 +65,10 @@ __device__ __forceinline__ double inv_lam(double l) { return l != 0.0 ? 1.0 / l 
 template <class T>
 __device__ __forceinline__ void put_wrapped(T* x, const ModalPass& a, int r, int c, T v) {
   const int64_t k = a.x0 + (int64_t)r * a.ldo + c;
+  if (a.only) {
+    if (a.only[k]) x[k] = v;
+    return;
+  }
   const int64_t sx = !a.wx ? 0 : (c < 3 ? a.wx : (c >= a.wx - 3 ? -a.wx : 0));
   const int64_t sy = !a.wy ? 0 : (r < 3 ? (int64_t)a.wy * a.ldo
                                         : (r >= a.wy - 3 ? -(int64_t)a.wy * a.ldo : 0));
@@ -365,9 +370,9 @@ __global__ __launch_bounds__(256) void k_modal_bsum(ModalRes g, const T* __restr
   if (threadIdx.x == 0) part[blockIdx.x] = v;
 }
 
-template <class T>
-__global__ __launch_bounds__(256) void k_modal_norms(ModalRes g, const T* __restrict__ b,
-                                                     const T* __restrict__ x, int singular,
+template <class TB, class TX>
+__global__ __launch_bounds__(256) void k_modal_norms(ModalRes g, const TB* __restrict__ b,
+                                                     const TX* __restrict__ x, int singular,
                                                      const double* __restrict__ bpart,
                                                      double* __restrict__ part) {
   __shared__ double sh[4];
@@ -443,6 +448,7 @@ struct ModalSolver {
   int singular = 0;
   double *t1 = nullptr, *t2 = nullptr;
   double* part = nullptr;
+  double* x64 = nullptr;  // FP64 result of a measured FP32 solve (on first use)
   std::vector<void*> allocs;
 };
 
@@ -571,9 +577,9 @@ static void launch_pass(const ModalPass& a, hipStream_t s) {
     launch_tile<16, 16, 1, 1, 4, 32, 2, FOLD, EPI, TI, TO>(a, s);
 }
 
-template <class T>
-void modal_solve(ModalSolver* m, const T* b, int gmode, T* x, bool measure, double* stats,
-                 hipStream_t s, const double* skip) {
+template <class TB, class TX>
+void modal_solve(ModalSolver* m, const TB* b, int gmode, TX* x, bool measure, double* stats,
+                 hipStream_t s, const double* skip, const int8_t* only) {
   const ModalDir &dx = m->x, &dy = m->y;
   F2D_REQUIRE(!gmode || (dx.cell && dy.cell), "the cell operator takes b on the cells");
   // 1: rows of b -> modes of x (t1: one row per mode)
@@ -593,7 +599,7 @@ void modal_solve(ModalSolver* m, const T* b, int gmode, T* x, bool measure, doub
   a.ne = dx.ne;
   a.no = dx.no;
   a.nj = dx.ne;
-  launch_pass<true, EPI_MODES, T, double>(a, s);
+  launch_pass<true, EPI_MODES, TB, double>(a, s);
   // 2: -> modes of y, divided by the eigenvalues (t2)
   ModalPass p{};
   p.skip = skip;
@@ -652,20 +658,37 @@ void modal_solve(ModalSolver* m, const T* b, int gmode, T* x, bool measure, doub
   r.x0 = m->k0;
   r.wx = dx.bc == BC_RING ? dx.n : 0;
   r.wy = dy.bc == BC_RING ? dy.n : 0;
-  launch_pass<false, EPI_PADDED, double, T>(r, s);
+  r.only = only;
+  launch_pass<false, EPI_PADDED, double, TX>(r, s);
   if (measure && stats) {
     ModalRes g = m->res;
     g.gmode = gmode;
-    if (m->singular) k_modal_bsum<T><<<MODAL_NB, 256, 0, s>>>(g, b, m->part + 3 * MODAL_NB);
-    k_modal_norms<T><<<MODAL_NB, 256, 0, s>>>(g, b, x, m->singular, m->part + 3 * MODAL_NB,
-                                              m->part);
+    double* sum = m->part + 3 * MODAL_NB;
+    if (m->singular) k_modal_bsum<TB><<<MODAL_NB, 256, 0, s>>>(g, b, sum);
+    if constexpr (sizeof(TX) == 4) {
+      // the residual of x rounded to FP32 (1e-3 at 1024^2, the operator
+      // amplifies the rounding) says nothing: that of the FP64 result
+      if (!m->x64) {
+        const size_t n = (size_t)m->NXP * (m->y.n + 6);
+        m->x64 = malloc_dev<double>(m, sizeof(double) * n);
+      }
+      r.out = m->x64;
+      r.only = nullptr;
+      launch_pass<false, EPI_PADDED, double, double>(r, s);
+      k_modal_norms<TB, double><<<MODAL_NB, 256, 0, s>>>(g, b, m->x64, m->singular, sum,
+                                                         m->part);
+    } else {
+      k_modal_norms<TB, double><<<MODAL_NB, 256, 0, s>>>(g, b, x, m->singular, sum, m->part);
+    }
     k_modal_stats<<<1, 256, 0, s>>>(m->part, (double)g.ny * g.nx, m->singular, stats);
   }
 }
 
-template void modal_solve<double>(ModalSolver*, const double*, int, double*, bool, double*,
-                                  hipStream_t, const double*);
-template void modal_solve<float>(ModalSolver*, const float*, int, float*, bool, double*,
-                                 hipStream_t, const double*);
+template void modal_solve(ModalSolver*, const double*, int, double*, bool, double*,
+                          hipStream_t, const double*, const int8_t*);
+template void modal_solve(ModalSolver*, const float*, int, float*, bool, double*, hipStream_t,
+                          const double*, const int8_t*);
+template void modal_solve(ModalSolver*, const double*, int, float*, bool, double*, hipStream_t,
+                          const double*, const int8_t*);
 
 }  // namespace f2d

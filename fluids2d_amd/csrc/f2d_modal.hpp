@@ -28,14 +28,16 @@ ModalSolver* modal_create(int64_t ny, int64_t nx, double dx, double dy, double m
 void modal_destroy(ModalSolver* m);
 
 // x = A^-1 b at the unknowns and their periodic halo images, on the padded
-// layout; T is b's and x's type, the arithmetic is FP64.  gmode 0: b given
-// at the unknowns; 1 (vertices): b = centerstovertices of the cell field
-// (operators.py:126-133, formed inside the first transform: the averaged
-// eigenvectors).  measure: the relative residual goes to `stats` (8 doubles,
-// device), as the other direct solves record it.  skip: a device flag; the
-// passes of a solve enqueued behind a nonzero one do nothing.
-template <class T>
-void modal_solve(ModalSolver* m, const T* b, int gmode, T* x, bool measure, double* stats,
-                 hipStream_t s, const double* skip = nullptr);
+// layout; TB is b's and TX x's type, the arithmetic is FP64.  gmode 0: b
+// given at the unknowns; 1 (vertices): b = centerstovertices of the cell
+// field (operators.py:126-133, formed inside the first transform: the
+// averaged eigenvectors).  measure: the relative residual goes to `stats` (8
+// doubles, device), as the other direct solves record it.  skip: a device
+// flag; the passes of a solve enqueued behind a nonzero one do nothing.
+// only: a mask on the padded layout; x is written where it is set, without
+// halo images.
+template <class TB, class TX>
+void modal_solve(ModalSolver* m, const TB* b, int gmode, TX* x, bool measure, double* stats,
+                 hipStream_t s, const double* skip = nullptr, const int8_t* only = nullptr);
 
 }  // namespace f2d

@@ -2373,10 +2373,15 @@ int f2d_poisson_create(const int8_t* unknowns_host, const f2d_grid* g,
                         std::to_string(CAP_MAX) + " boundary points)");
         h->cap = cap_create(m.data(), h->ny, h->nx, g->dx, g->dy, maindiag, h->xper,
                             h->yper, f64m);
-      } else if (nb > 0 && nb <= CAP_AUTO_MAX) {
-        try {
+      } else {
+        // auto: also the rectangles the eigenvector solve handles
+        const bool modal = nb < 0;
+        const int64_t nm = modal ? cap_boundary(m.data(), h->ny, h->nx, h->xper, h->yper,
+                                                maindiag, f64m, true)
+                                 : nb;
+        if (nm > 0 && nm <= CAP_AUTO_MAX) try {
           h->cap = cap_create(m.data(), h->ny, h->nx, g->dx, g->dy, maindiag, h->xper,
-                              h->yper, f64m);
+                              h->yper, f64m, modal);
         } catch (const Error&) {
           h->cap = nullptr;  // multigrid solves this operator
           (void)hipGetLastError();
@@ -2437,7 +2442,13 @@ static int solve_common(f2d_poisson* h, const void* b, void* x, int gmode,
     }
     if (h->cap) {
       Ctl* c = mode == F2D_POISSON_F64 ? h->p64.ctl : h->p32.ctl;
-      if (mode == F2D_POISSON_F64) {
+      if (mode == F2D_POISSON_F64 && cap_modal(h->cap)) {
+        cap_solve_modal(h->cap, (const double*)b, gmode, (double*)x, sync, c->stats, s);
+        fill_x<double>(h, (double*)x, s);
+      } else if (cap_modal(h->cap)) {
+        cap_solve_modal(h->cap, (const float*)b, gmode, (float*)x, sync, c->stats, s);
+        fill_x<float>(h, (float*)x, s);
+      } else if (mode == F2D_POISSON_F64) {
         cap_solve_f64(h->cap, (const double*)b, gmode, (double*)x, sync, c->stats, s);
         fill_x<double>(h, (double*)x, s);
       } else {
@@ -2452,9 +2463,9 @@ static int solve_common(f2d_poisson* h, const void* b, void* x, int gmode,
     } else if (h->modal) {
       Ctl* c = mode == F2D_POISSON_F64 ? h->p64.ctl : h->p32.ctl;
       if (mode == F2D_POISSON_F64)
-        modal_solve<double>(h->modal, (const double*)b, gmode, (double*)x, sync, c->stats, s);
+        modal_solve(h->modal, (const double*)b, gmode, (double*)x, sync, c->stats, s);
       else
-        modal_solve<float>(h->modal, (const float*)b, gmode, (float*)x, sync, c->stats, s);
+        modal_solve(h->modal, (const float*)b, gmode, (float*)x, sync, c->stats, s);
       if (!sync) h->fft_unmeasured++;
     } else if (h->fft) {
       Ctl* c = mode == F2D_POISSON_F64 ? h->p64.ctl : h->p32.ctl;
@@ -2512,7 +2523,7 @@ int f2d_poisson_set_refine(f2d_poisson* h, int nref) {
 int f2d_poisson_method(f2d_poisson* h) {
   if (!h) return -1;
   if (h->neu) return F2D_SOLVER_NEUMANN_CG;
-  if (h->cap) return F2D_SOLVER_CAP;
+  if (h->cap) return cap_modal(h->cap) ? F2D_SOLVER_MODAL_CAP : F2D_SOLVER_CAP;
   if (h->modal) return F2D_SOLVER_MODAL;
   return h->fft ? F2D_SOLVER_FFT : F2D_SOLVER_MG;
 }

@@ -20,7 +20,7 @@ DEFAULT_MAXIT = {"fp64": 100, "fp32": 8}
 
 
 # methods that solve directly: no iteration count to learn, no rtol test
-DIRECT = ("fft", "capacitance", "modal")
+DIRECT = ("fft", "capacitance", "modal", "modal_capacitance")
 
 
 def _destroy(h, name="f2d_poisson_destroy"):
@@ -113,9 +113,11 @@ class Poisson2D:
                   self.maindiag, ctypes.byref(opts), ctypes.byref(h))
         self._h = h
         # "fft": direct spectral solve (exact to rounding, no rtol test);
-        # "modal": direct eigenvector solve; "capacitance": direct masked
-        # solve; "mg": multigrid-preconditioned CG to rtol
-        self.method = {2: "fft", 3: "neumann", 4: "capacitance", 5: "modal"}.get(
+        # "modal": direct eigenvector solve; "capacitance",
+        # "modal_capacitance": direct masked solves around them; "mg":
+        # multigrid-preconditioned CG to rtol
+        self.method = {2: "fft", 3: "neumann", 4: "capacitance", 5: "modal",
+                       6: "modal_capacitance"}.get(
             _lib.lib().f2d_poisson_method(h), "mg")
         self.last_iters = 0
         self.last_relres = 0.0

@@ -475,6 +475,12 @@ typedef struct f2d_poisson_opts {
  * transforms by the eigenvectors of the two second differences, FP64 in
  * every mode; zero mean when singular.  Statistics as the FFT solve's. */
 #define F2D_SOLVER_MODAL 5
+/* Reported by f2d_poisson_method only: the capacitance solve around the
+ * eigenvector solve, which AUTO takes for a masked vertex operator inside a
+ * rectangle of sizes that are not both powers of two (at most 4096, 2048 in
+ * a closed direction; a closed direction or maindiag > 0; at most 8192
+ * boundary points).  FP64 in every mode; not taken into batches. */
+#define F2D_SOLVER_MODAL_CAP 6
 /* The masked vertex operator of a mask inside a rectangle the FFT solve
  * handles (power-of-two sizes, a closed direction or maindiag > 0): the
  * masked operator is the rectangle operator's principal submatrix on the
@@ -501,9 +507,10 @@ int f2d_poisson_destroy(f2d_poisson* h);
 int f2d_poisson_solve(f2d_poisson* h, const void* b, void* x, double rtol,
                       int maxit, int* iters, double* relres, void* stream);
 /* The method a handle solves with, F2D_SOLVER_MG, F2D_SOLVER_FFT,
- * F2D_SOLVER_NEUMANN_CG, F2D_SOLVER_CAP or F2D_SOLVER_MODAL (-1 for NULL);
- * no counterpart in the reference, whose SuperLU factor is its only method
- * (elliptic.py:78).  With FFT, CAP or MODAL the solve is direct: `maxit` is unused, *iters receives
+ * F2D_SOLVER_NEUMANN_CG, F2D_SOLVER_CAP, F2D_SOLVER_MODAL or
+ * F2D_SOLVER_MODAL_CAP (-1 for NULL); no counterpart in the reference, whose
+ * SuperLU factor is its only method (elliptic.py:78).  With all but MG and
+ * NEUMANN_CG the solve is direct: `maxit` is unused, *iters receives
  * 1 + the FP64 refinements, *relres the measured true relative residual,
  * and the solve counts as converged when that residual is below 1e-6
  * (`rtol` is not its acceptance test: a direct FP64 solve reaches eps times
