@@ -310,6 +310,7 @@ __global__ __launch_bounds__(256) void k_cap_stats(const double* __restrict__ pa
   st[4] += conv > 0.0 ? 0.0 : 1.0;
   if ((double)(passes - 1) > st[5]) st[5] = (double)(passes - 1);
   st[6] += 1.0;
+  if (st[7] == st[7] && !(rel <= st[7])) st[7] = rel;  // a NaN stays
 }
 
 // one member of a batched FP32 solve (device table, blockIdx.y = member)

@@ -887,6 +887,7 @@ __global__ __launch_bounds__(256) void k_fft_stats(const double* __restrict__ pa
   st[4] += conv > 0.0 ? 0.0 : 1.0;
   if ((double)nref > st[5]) st[5] = (double)nref;
   st[6] += 1.0;
+  if (st[7] == st[7] && !(rel <= st[7])) st[7] = rel;  // a NaN stays
 }
 
 // ---------------------------------------------------------------------------

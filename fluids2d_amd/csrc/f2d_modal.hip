@@ -426,6 +426,7 @@ __global__ __launch_bounds__(256) void k_modal_stats(const double* __restrict__ 
   st[3] = 0.0;
   st[4] += conv > 0.0 ? 0.0 : 1.0;
   st[6] += 1.0;
+  if (st[7] == st[7] && !(rel <= st[7])) st[7] = rel;  // a NaN stays
 }
 
 // ---------------------------------------------------------------------------

@@ -1520,6 +1520,7 @@ struct f2d_poisson {
   f2d::CapSolver* cap = nullptr;  // masked operator: spectral + capacitance
   f2d::ModalSolver* modal = nullptr;  // fully wet rectangles of other sizes
   int64_t fft_unmeasured = 0;     // FFT solves made without statistics
+  int measure = 0;  // direct solves record their residual without a host check
   int refine_next = -1;  // FP32 direct solves: refinements (0: none), -1 options
   std::vector<void*> allocs;
   double* reg(int r) { return part + (int64_t)r * region; }
@@ -2440,37 +2441,39 @@ static int solve_common(f2d_poisson* h, const void* b, void* x, int gmode,
       }
       return;
     }
+    // (direct solves)
+    const bool measure = sync || h->measure;
     if (h->cap) {
       Ctl* c = mode == F2D_POISSON_F64 ? h->p64.ctl : h->p32.ctl;
       if (mode == F2D_POISSON_F64 && cap_modal(h->cap)) {
-        cap_solve_modal(h->cap, (const double*)b, gmode, (double*)x, sync, c->stats, s);
+        cap_solve_modal(h->cap, (const double*)b, gmode, (double*)x, measure, c->stats, s);
         fill_x<double>(h, (double*)x, s);
       } else if (cap_modal(h->cap)) {
-        cap_solve_modal(h->cap, (const float*)b, gmode, (float*)x, sync, c->stats, s);
+        cap_solve_modal(h->cap, (const float*)b, gmode, (float*)x, measure, c->stats, s);
         fill_x<float>(h, (float*)x, s);
       } else if (mode == F2D_POISSON_F64) {
-        cap_solve_f64(h->cap, (const double*)b, gmode, (double*)x, sync, c->stats, s);
+        cap_solve_f64(h->cap, (const double*)b, gmode, (double*)x, measure, c->stats, s);
         fill_x<double>(h, (double*)x, s);
       } else {
         const int nref = h->refine_next >= 0
                              ? h->refine_next
                              : (h->opts.fft_refine > 0 ? h->opts.fft_refine : 1);
         cap_solve_f32(h->cap, (const float*)b, gmode, (float*)x, nref,
-                      h->opts.fft_warm != 0, sync, c->stats, s);
+                      h->opts.fft_warm != 0, measure, c->stats, s);
         fill_x<float>(h, (float*)x, s);
       }
-      if (!sync) h->fft_unmeasured++;
+      if (!measure) h->fft_unmeasured++;
     } else if (h->modal) {
       Ctl* c = mode == F2D_POISSON_F64 ? h->p64.ctl : h->p32.ctl;
       if (mode == F2D_POISSON_F64)
-        modal_solve(h->modal, (const double*)b, gmode, (double*)x, sync, c->stats, s);
+        modal_solve(h->modal, (const double*)b, gmode, (double*)x, measure, c->stats, s);
       else
-        modal_solve(h->modal, (const float*)b, gmode, (float*)x, sync, c->stats, s);
-      if (!sync) h->fft_unmeasured++;
+        modal_solve(h->modal, (const float*)b, gmode, (float*)x, measure, c->stats, s);
+      if (!measure) h->fft_unmeasured++;
     } else if (h->fft) {
       Ctl* c = mode == F2D_POISSON_F64 ? h->p64.ctl : h->p32.ctl;
       if (mode == F2D_POISSON_F64) {
-        fft_solve_f64(h->fft, (const double*)b, gmode, (double*)x, rtol, sync,
+        fft_solve_f64(h->fft, (const double*)b, gmode, (double*)x, rtol, measure,
                       c->stats, s);
       } else {
         const int nref = mode == F2D_POISSON_F32
@@ -2480,9 +2483,9 @@ static int solve_common(f2d_poisson* h, const void* b, void* x, int gmode,
                                     : (h->opts.fft_refine > 0 ? h->opts.fft_refine : 1));
         fft_solve_f32_refine(h->fft, (const float*)b, gmode, (float*)x, nref,
                              h->opts.fft_warm != 0, rtol,
-                             sync, c->stats, s);
+                             measure, c->stats, s);
       }
-      if (!sync) h->fft_unmeasured++;
+      if (!measure) h->fft_unmeasured++;
     } else if (mode == F2D_POISSON_F64) {
       do_solve<double>(h, (const double*)b, x, gmode, rtol, maxit, sync, s);
     } else {
@@ -2517,6 +2520,15 @@ int f2d_poisson_set_refine(f2d_poisson* h, int nref) {
     F2D_REQUIRE(h, "handle is NULL");
     F2D_REQUIRE(nref >= -1 && nref <= 16, "refinements must be in -1 .. 16");
     h->refine_next = nref;
+  });
+}
+
+int f2d_poisson_measure(f2d_poisson* h, int on) {
+  return guarded([&] {
+    F2D_REQUIRE(h, "handle is NULL");
+    F2D_REQUIRE(!on || h->fft || h->modal || h->cap,
+                "only direct solves are measured without a host check");
+    h->measure = on ? 1 : 0;
   });
 }
 

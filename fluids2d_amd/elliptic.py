@@ -158,6 +158,8 @@ class Poisson2D:
         stats=False (device tensors, once a host-checked solve has set the
         learned count): no host round trip, as in ``solve_c2v``."""
         host = not isinstance(x, torch.Tensor)
+        if stats == "device":
+            return self._solve_measured("f2d_poisson_solve", b, x)
         if not host and not stats and self.est is not None:
             self.calls += 1
             n = min(self.est + self.margin, self.maxit)
@@ -210,6 +212,8 @@ class Poisson2D:
         learned iteration count plus a margin (iterations past convergence
         return at once) and leaves its outcome in the device counters that
         ``read_stats()`` returns."""
+        if stats == "device":
+            return self._solve_measured("f2d_poisson_solve_c2v", omega, x)
         self.calls += 1
         if stats or self.est is None:
             it, rr = ctypes.c_int(), ctypes.c_double()
@@ -229,6 +233,32 @@ class Poisson2D:
             n = min(self.est + self.margin, self.maxit)
             _lib.call("f2d_poisson_solve_c2v", self._h, _lib.ptr(omega), _lib.ptr(x),
                       self.rtol, n, None, None, _lib.stream_ptr())
+
+    def _solve_measured(self, name, b, x):
+        """stats="device" (direct methods): the host-checked solve, its
+        residual left in the device statistics (``worst``) for a later
+        check."""
+        self.calls += 1
+        _lib.call("f2d_poisson_measure", self._h, 1)
+        try:
+            _lib.call(name, self._h, _lib.ptr(b), _lib.ptr(x), self.rtol, self.maxit, None,
+                      None, _lib.stream_ptr())
+        finally:
+            _lib.call("f2d_poisson_measure", self._h, 0)
+
+    def worst(self):
+        """Device address of the largest relative residual measured since the
+        last reset (float64)."""
+        return ctypes.c_void_p(_lib.lib().f2d_poisson_stats(self._h) + 7 * 8)
+
+    def check_worst(self, relres):
+        """Raise as a host-checked solve does when the residual is not
+        accepted."""
+        self.last_relres = relres
+        if not self._accepted(relres):
+            raise PoissonNotConverged(
+                f"Poisson solve reached relres {relres:.3e} > {self.rtol:.1e} "
+                f"after 1 iterations")
 
     def set_refine(self, nref):
         """FP64 refinements of the following direct (FFT or capacitance)

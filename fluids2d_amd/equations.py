@@ -29,6 +29,11 @@ class _Base:
     def cfl_velocity(self, s):
         return s.U
 
+    def graph_operands(self, s):
+        """Device copies of host operands that a captured step holds: brought
+        up to date (outside a capture) and returned as a key."""
+        return ()
+
 
 class EulerPsi(_Base):
     """Euler in vorticity-streamfunction form (equations.py:269-282)."""
@@ -156,6 +161,9 @@ class QG(_Base):
                 d = torch.from_numpy(np.array(a)).to(like.device).to(like.dtype)  # a writable copy
             self._f_src, self._f_dev = f, d.contiguous()
         return self._f_dev
+
+    def graph_operands(self, s):
+        return (self._planetary(s.work).data_ptr(),) if self.param.beta != 0 else ()
 
     def _inversion_rhs(self, s):
         """work = centerstovertices(pv - hb*qgcoef) - f (operators.py:186-190;

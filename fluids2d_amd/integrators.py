@@ -23,6 +23,7 @@ import torch
 
 from . import _lib
 from . import operators as op
+from .elliptic import DIRECT
 from .equations import get_device_model
 from .states import (Prognostic, allocate_device, download, get_specs, leaves,
                      upload)
@@ -64,6 +65,15 @@ class RKIntegrator:
         self.d_dtn = torch.zeros(1, dtype=torch.float64, device=dev)
         self._dt_written = None  # (value, buffer) of the last fixed dt written
         self._h_dt = torch.zeros(1, dtype=torch.float64).pin_memory()
+        # run loop (device_step): captured host-checked steps, the pinned
+        # array they leave the next dt [0] and the solvers' worst residuals
+        # in, the solvers of the step whose residuals are to be checked
+        self._checked = {}
+        self._h_run = torch.zeros(4, dtype=torch.float64).pin_memory()
+        self._dt_on_host = False
+        self._unchecked = ()
+        self._run_steps, self._run_mesh = 0, None
+        self._no_replay = False
         self._dtn_valid = False
         # Models with ``defers_cfl``: the last stage leaves the next step's
         # CFL step as block maxima in _cfl (_dtn_part: d_dtn is not written
@@ -127,6 +137,7 @@ class RKIntegrator:
         return [a for n in self.specs.prognostic for a in leaves(getattr(s, n))]
 
     def _host_rhs(self, s, ds):
+        self._check_step()
         upload(s, self.dstate)
         dds = self.dscratch[0]
         self.model.rhs(self.dstate, dds)
@@ -135,6 +146,7 @@ class RKIntegrator:
             download(self.dstate, s, names=["flx"])
 
     def _host_diag(self, s):
+        self._check_step()
         upload(s, self.dstate)
         self.model.diag(self.dstate)
         self.model.materialize(self.dstate)
@@ -153,11 +165,13 @@ class RKIntegrator:
     # -- device path --------------------------------------------------------------
     def begin(self, state):
         """Host state -> device twin."""
+        self._check_step()
         upload(state, self.dstate)
         self._dtn_valid = self._dtn_part = self._dt_part = False
 
     def end(self, state, names=None):
         """Device twin -> host state."""
+        self._check_step()
         self.model.materialize(self.dstate, names)
         download(self.dstate, state, names)
 
@@ -165,6 +179,7 @@ class RKIntegrator:
         """Model.set_dt (model.py:71-87): dt on the device and on the host."""
         p = self.param
         if p.dt > 0:
+            self._check_step()
             time.dt = p.dt
             self._write_dt(p.dt)
             return
@@ -182,6 +197,10 @@ class RKIntegrator:
             self._finish_cfl(self.d_dtn)
         self._dtn_part = self._dt_part = False
         self.d_dt, self.d_dtn = self.d_dtn, self.d_dt
+        if self._dt_on_host:  # left there by the step's graph
+            self._check_step()
+            time.dt = float(self._h_run[0])
+            return
         self._h_dt.copy_(self.d_dt, non_blocking=True)
         torch.cuda.current_stream().synchronize()
         time.dt = float(self._h_dt[0])
@@ -219,6 +238,7 @@ class RKIntegrator:
         """Names of the prognostic fields of the device state with a
         non-finite value on a wet cell (one flag per field, read on the host:
         a synchronisation point)."""
+        self._check_step()
         names = [n for n in self.specs.prognostic]
         flags = torch.zeros(len(names), dtype=torch.int32, device=self.d_dt.device)
         m = self.mesh
@@ -236,6 +256,7 @@ class RKIntegrator:
     def advance(self, stats=True, dt_log=None):
         """One RK step on the device with the dt already in d_dt; dt_log (a
         one-element float64 device tensor) receives that dt."""
+        self._check_step()
         s, alt = self.dstate, self.dalt
         dtn = self.d_dtn if self._wants_dtn() else None
         if self.forcings:
@@ -284,6 +305,7 @@ class RKIntegrator:
         stage).  Running pre, the solve, post, cfl for k = 0, 1, ... is the
         step.  The dt is the one in d_dt now (call after _select_dt)."""
         assert not self.forcings and hasattr(self.model, "stage_split")
+        self._check_step()
         self._dt_ready()
         if dt_log is not None and not getattr(self.model, "logs_dt", False):
             self._log_dt(dt_log)
@@ -303,8 +325,100 @@ class RKIntegrator:
         return plan
 
     def device_step(self, time):
-        self.advance()
+        """One host-checked step (Model.run's): with direct solvers and
+        ``param.hipgraph``, after two eager steps, the replay of a captured
+        step whose solves leave their measured residuals on the device.
+        They are checked -- the same test, the same exception -- where the
+        loop next waits for the device: at set_dt or end."""
+        self._check_step()
+        g = self._checked_step() if self._can_replay() else None
+        if g is None:
+            self.advance()
+            self._run_steps += 1
+        else:
+            graph, (self.dstate, self.dalt), sols = g[:3]
+            graph.replay()
+            self._dtn_valid = self._wants_dtn()
+            self._dt_part = self._dtn_part = False
+            self._dt_on_host = self._dtn_valid
+            self._unchecked = sols
+            for e in sols:
+                e.calls += self.nstages
         time.pushforward()
+
+    def _can_replay(self):
+        if self._run_mesh != self.mesh.version:
+            # a re-finalised mesh builds its solvers in the next eager steps
+            self._run_mesh, self._run_steps = self.mesh.version, 0
+        return (getattr(self.param, "hipgraph", True) and not self.forcings
+                and self._run_steps >= 2 and not self._dt_part and not self._no_replay
+                and getattr(self.model, "capturable", True)
+                and getattr(self.model, "events", None) is None
+                and all(e.method in DIRECT for e in self._solvers()))
+
+    def _check_step(self):
+        """Wait for the last replayed step and check its solves."""
+        if not (self._dt_on_host or self._unchecked):
+            return
+        torch.cuda.current_stream().synchronize()
+        sols, self._unchecked, self._dt_on_host = self._unchecked, (), False
+        for k, e in enumerate(sols):
+            e.check_worst(float(self._h_run[1 + k]))
+
+    def _checked_step(self):
+        """The captured host-checked step of the current buffers and
+        parameters: (graph, state and alternate state after it, solvers).
+        The next step's dt and the solvers' worst residuals go to pinned host
+        memory by kernels of the graph."""
+        p, m = self.param, self.mesh
+        key = self._graph_key() + self.model.graph_operands(self.dstate) + (
+            p.cfl, p.dtmax, p.dt > 0, p.compflux, p.vortexforce, p.innerproduct, p.f0, p.g, p.H,
+            p.beta, getattr(p, "poisson_refine", "every"), m.grid.tile,
+            getattr(self.model, "fused", True), tuple(id(e) for e in self._solvers()))
+        got = self._checked.get(key)
+        if got is not None:
+            return got
+        if len(self._checked) >= 16:  # parameters that change as the run goes
+            self._checked.clear()
+        keep = (self.dstate, self.dalt, self._dtn_valid, self._dtn_part, self._dt_part)
+        sols = self._solvers()
+        graph = torch.cuda.CUDAGraph()
+        side = torch.cuda.Stream(m.device)
+        side.wait_stream(torch.cuda.current_stream())
+        calls = [e.calls for e in sols]
+        try:
+            with torch.cuda.stream(side), _lib.no_gc():
+                # (thread-local: other threads' runs go on meanwhile)
+                graph.capture_begin(capture_error_mode="thread_local")
+                try:
+                    for e in sols:  # this step's worst, not an earlier solve's
+                        _lib.call("f2d_set_scalar", e.worst(), 0.0, _lib.stream_ptr())
+                    self.advance(stats="device")
+                    if self._dtn_part:
+                        self._finish_cfl(self.d_dtn)
+                    if self._wants_dtn():
+                        _lib.call("f2d_copy_f64", _lib.ptr(self._h_run), _lib.ptr(self.d_dtn),
+                                  1, _lib.stream_ptr())
+                    # the solvers this step called
+                    used = [e for e, c in zip(sols, calls) if e.calls > c]
+                    for k, e in enumerate(used):
+                        _lib.call("f2d_copy_f64", _lib.ptr(self._h_run[1 + k:]), e.worst(), 1,
+                                  _lib.stream_ptr())
+                finally:
+                    graph.capture_end()
+                    after = (self.dstate, self.dalt)
+        except (RuntimeError, _lib.F2DError):
+            self._no_replay = True  # eager steps need no graph
+            return None
+        finally:
+            self.dstate, self.dalt, self._dtn_valid, self._dtn_part, self._dt_part = keep
+            torch.cuda.current_stream().wait_stream(side)
+            for e, c in zip(sols, calls):
+                e.calls = c
+        # (the model and the solvers live as long as their addresses may be
+        # replayed: the key names them)
+        got = self._checked[key] = (graph, after, used, self.model, sols)
+        return got
 
     def _select_dt(self, defer=False):
         """The dt of the next step into d_dt, on the device (Model.set_dt,
@@ -312,6 +426,7 @@ class RKIntegrator:
         pending as block maxima stays so, and the step's first stage forms
         it."""
         p = self.param
+        self._check_step()
         self._dt_part = False
         if p.dt > 0:
             self._write_dt(p.dt)
@@ -390,6 +505,7 @@ class RKIntegrator:
         if self._graph_mesh != self.mesh.version:
             # a re-finalised mesh has new solvers and masks: drop old graphs
             self._graphs = {}
+            self._checked = {}
             self._graph_mesh = self.mesh.version
         return (self.mesh.version, id(self.model),
                 tuple(t.data_ptr() for t in leaves(self.dstate)),

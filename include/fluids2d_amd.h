@@ -531,13 +531,22 @@ int f2d_poisson_solve_c2v(f2d_poisson* h, const void* omega, void* x,
  * solve [0] iterations (F32_REFINE: inner iterations summed), [1] relative
  * residual, [2] converged flag, [3] refinements; since the last reset
  * [4] number of solves that did not converge, [5] maximum iterations
- * (F32_REFINE: refinements), [6] number of solves.  Without iters/relres a
+ * (F32_REFINE: refinements), [6] number of solves,
+ * [7] the largest relative residual a direct solve measured (NaN once one
+ * was NaN).  Without iters/relres a
  * solve enqueues exactly `maxit` iterations (refinements), those after
  * convergence returning at once, and never synchronises: these counters are
  * how a caller checks such solves afterwards. */
 /* (no counterpart in the reference: SuperLU is direct, elliptic.py:78-87) */
 const double* f2d_poisson_stats(f2d_poisson* h);
-/* Zero the counters [4..6] (no counterpart in the reference). */
+/* on != 0: the following direct solves (FFT, CAP, MODAL, MODAL_CAP) made
+ * without iters/relres measure their residual all the same and record it in
+ * the device statistics, so that a caller can check many solves at once (the
+ * solve is the host-checked one, bit for bit); 0: they measure nothing.  Host
+ * state: a captured graph keeps what its solves were made with (no counterpart
+ * in the reference, whose SuperLU measures nothing). */
+int f2d_poisson_measure(f2d_poisson* h, int on);
+/* Zero the counters [4..7] (no counterpart in the reference). */
 int f2d_poisson_reset_stats(f2d_poisson* h, void* stream);
 /* Copy the 8 statistics above to host memory, synchronising `stream`
  * (no counterpart in the reference).  FFT solves made without iters/relres

@@ -1,0 +1,114 @@
+"""Model.run's captured host-checked steps (integrators.RKIntegrator.device_step)
+against the same run with eager launches (hipgraph off), bit for bit: states,
+times and dt, every model, direct and iterative solvers, parameters changed
+and meshes re-finalised between runs, and the solver's check of every step."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_euler import _device
+from helpers import random_mask
+
+pytestmark = pytest.mark.gpu
+
+
+def _start(model, nx, ny, nisl, precision, hipgraph, dt=0.0, **kw):
+    p = dict(model=model, nx=nx, ny=ny, Lx=nx / ny, Ly=1.0, tend=1e9, maxite=11, dt=dt,
+             nprint=10 ** 9, hipgraph=hipgraph, **kw)
+    msk = random_mask(ny, nx, 6, p.get("xperiodic", False), False, nisl=nisl) if nisl else None
+    m = _device(p, msk, precision)
+    rng = np.random.default_rng(3)
+    x, y = m.mesh.xy("c")
+    w = (np.exp(-((x - 0.5 * nx / ny) ** 2 + (y - 0.5) ** 2) / 0.02)
+         + 1e-2 * rng.standard_normal(x.shape)) * m.mesh.msk * m.mesh.area
+    s = m.state
+    if model == "euler":
+        s.u.x[...] = w * m.mesh.mskx
+        s.u.y[...] = -w * m.mesh.msky
+    elif model in ("rsw", "qgrsw"):
+        s.h[...] = (m.mesh.area * m.mesh.msk + 0.05 * w)
+    else:
+        getattr(s, {"qg": "pv", "advection": "q"}.get(model, "omega"))[...] = w
+    if model == "advection":
+        s.U.x[...] = 0.3 * m.mesh.mskx / m.mesh.dx
+    if kw.get("beta"):
+        m.mesh.f = 0.1 * np.broadcast_to(y, x.shape) * m.mesh.area
+    m.mesh.fill(s[0])
+    m.integrator.diag(s)
+    return m
+
+
+def _leaves(m):
+    out = []
+    for v in m.state:
+        out += list(v) if isinstance(v, tuple) else [v]
+    return out
+
+
+@pytest.mark.parametrize("model,nx,ny,nisl,precision,kw", [
+    ("euler", 40, 40, 0, "fp64", {}), ("euler", 48, 40, 3, "fp64", {}),
+    ("euler", 64, 64, 0, "fp32", {}),
+    ("eulerpsi", 64, 64, 0, "fp64", {}), ("eulerpsi", 48, 40, 0, "fp32", dict(xperiodic=True)),
+    ("eulerpsi", 64, 64, 0, "fp32", dict(xperiodic=True, yperiodic=True)),
+    ("eulerpsi", 64, 64, 3, "fp64", dict(dt=0.01)),
+    ("eulerpsi", 40, 40, 0, "fp64", dict(poisson_solver="mg")),
+    ("qg", 64, 48, 0, "fp64", dict(beta=1.0, f0=5.0)), ("qgrsw", 64, 64, 1, "fp32", dict(dtmax=0.02)),
+    ("rsw", 50, 40, 3, "fp64", {}), ("advection", 50, 40, 0, "fp64", {})])
+def test_run_replays_match_eager(dev, model, nx, ny, nisl, precision, kw):
+    print(f"\nrun {model} {nx}x{ny} islands={nisl} {precision} {kw}", flush=True)
+    a, b = (_start(model, nx, ny, nisl, precision, g, **kw) for g in (True, False))
+    for k in range(3):
+        if k == 1:  # the next runs bake another CFL number
+            for m in (a, b):
+                m.param.cfl = 0.7
+        if k == 2:
+            for m in (a, b):
+                m.mesh.finalize()
+                m.integrator.diag(m.state)
+        for m in (a, b):
+            m.time.ite0, m.param.maxite = m.time.ite, 11 + k
+            m.run()
+        assert a.time.ite == b.time.ite and a.time.t == b.time.t and a.time.dt == b.time.dt
+        for u, v in zip(_leaves(a), _leaves(b)):
+            assert np.array_equal(u, v, equal_nan=True)
+    captured = len(a.integrator._checked)
+    direct = kw.get("poisson_solver") != "mg" and not (model == "euler" and nisl)
+    assert (captured > 0) == direct and not b.integrator._checked
+    for e, f in zip(a.integrator._solvers(), b.integrator._solvers()):
+        if direct:
+            assert e.read_stats()["solves"] == f.read_stats()["solves"] and e.calls == f.calls
+
+
+def test_replayed_steps_are_checked(dev, monkeypatch):
+    """A solve whose residual is not accepted ends the run with
+    PoissonNotConverged, replayed or not, and does not linger."""
+    from fluids2d_amd.elliptic import PoissonNotConverged
+    m = _start("eulerpsi", 64, 64, 0, "fp64", True)
+    m.run()
+    assert m.integrator._checked
+    pois = m.mesh.poisson_vertices
+    with monkeypatch.context() as mp:
+        mp.setattr(type(pois), "_accepted", lambda self, r: r <= 1e-30)
+        m.time.ite0 = m.time.ite
+        with pytest.raises(PoissonNotConverged):
+            m.run()
+    m.time.ite0 = m.time.ite
+    m.run()
+
+
+def test_planetary_vorticity_rebound_between_steps(dev):
+    """qg with beta: mesh.f bound to another array during a run reaches the
+    replayed steps, as it does the eager ones."""
+    out = []
+    for g in (True, False):
+        m = _start("qg", 64, 64, 0, "fp64", g, beta=1.0)
+
+        def rebind():
+            if m.time.ite == 6:
+                m.mesh.f = 3.0 * m.mesh.f
+        rebind.device = True
+        rebind.finalize = lambda: None
+        m.diags.append(rebind)
+        m.run()
+        out.append(m.state.pv.copy())
+    assert np.array_equal(*out)
