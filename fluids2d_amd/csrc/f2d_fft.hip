@@ -14,6 +14,7 @@
 // between two LDS buffers) with twiddles from a table in pass order;
 // inverse transforms conjugate on the way in and out.
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "f2d_fft.hpp"
@@ -63,7 +64,7 @@ struct FftArgs {
   int Q;         // spectral columns per workgroup (column pass)
   double cx, cy, d;
   int singular;
-  int pad;
+  int real0;     // drop the imaginary parts of the modes kx = 0, nx / 2
   // Closed directions (ex, ey nonzero): the problem's onx x ony interior is
   // solved as its extension on the periodic doubled grid (nx = 2 onx when
   // ex, ny = 2 ony when ey): 1 odd (vertex unknowns, Dirichlet boundary
@@ -71,7 +72,6 @@ struct FftArgs {
   // problem's sizes, NXP its padded row length.
   int ex, ey;
   int onx, ony;
-  int ipx, ipy;  // rows, columns transformed in place (fft_inplace)
 };
 
 // Forward DFTs of `nf` contiguous length-N sequences held in LDS buffer `a`
@@ -128,33 +128,193 @@ __device__ cplx<T>* fft_lds(cplx<T>* a, cplx<T>* b, int N, int lgN, int nf,
   return a;
 }
 
-// The same transform of one sequence of N = 4 blockDim points in place, for
-// lengths whose two buffers and twiddles do not fit LDS (FP64 4096): a thread
-// holds one butterfly, so a pass reads, waits for the others and writes over
-// the input.  Twiddles come from global memory (L2), which leaves a CU room
-// for two workgroups.  Same operations in the same order as fft_lds.
-// Measured: the doubly periodic 4096^2 FP64 step 36.4 ms with the multigrid
-// solve these grids had, 1.80 ms with this one.
+// Register transforms of N = 2^LG points, LG 8 .. 12: N / 8 threads a
+// sequence, 8 points a thread.  Thread j takes points j + m N/8 (m = 0 .. 7)
+// and returns entries j + q N/8, so a pass's global loads and stores are
+// coalesced without LDS, and a column's forward transform hands its entries
+// straight to the inverse one.  Passes: one of radix 2 or 4 where LG is not
+// a multiple of 3, then radix 8; between two passes the entries go through
+// LDS (index i at i + i / 8: the stride-8 writes of the first passes then
+// spread over the banks).  Against radix-4 passes through LDS (fft_lds) a
+// 1024-point row makes 3 LDS exchanges instead of 5 and a column 6 instead
+// of 11.  Every twiddle comes from the table (no products of twiddles: the
+// FP32 rounding is that of one factor a pass), loaded ahead of the exchange.
+// Bound by HBM from 2048 points: a FP64 4096^2 solve takes 301 us for the
+// 1.2 GB that its passes read and write (4.0 TB/s), 2048^2 83 us (fft_lds
+// 111 us), closed 1024^2 44 us (63), channel 1024^2 40 us (49); FP32 4096^2
+// 214 us (346), closed 2048^2 127 us (199).
+template <class T> struct Vec2 {
+  typedef T type __attribute__((ext_vector_type(2)));  // (a struct in an
+  // array held over a loop is kept in scratch memory, an ext_vector is not)
+};
+template <class T> using vec2 = typename Vec2<T>::type;
+
+__device__ __forceinline__ float fma_t(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fma_t(double a, double b, double c) { return fma(a, b, c); }
+// (fused: one rounding less a component)
 template <class T>
-__device__ void fft_inplace(cplx<T>* a, int N, const cplx<T>* __restrict__ tw) {
-  const int j = threadIdx.x, nb = N >> 2;
-  for (int Ns = 1; Ns < N; Ns <<= 2) {
-    const int jm = j & (Ns - 1);
-    const cplx<T>* tp = tw + (Ns - 1);
-    const cplx<T> t1 = tp[jm], t2 = tp[Ns + jm], t3 = tp[2 * Ns + jm];
-    const cplx<T> a0 = a[j];
-    const cplx<T> a1 = cmul<T>(a[j + nb], t1);
-    const cplx<T> a2 = cmul<T>(a[j + 2 * nb], t2);
-    const cplx<T> a3 = cmul<T>(a[j + 3 * nb], t3);
-    const cplx<T> b0 = cadd<T>(a0, a2), b1 = csub<T>(a0, a2);
-    const cplx<T> b2 = cadd<T>(a1, a3), b3 = csub<T>(a1, a3);
-    const int base = ((j - jm) << 2) + jm;
+__device__ __forceinline__ vec2<T> vmul(vec2<T> a, vec2<T> b) {
+  return vec2<T>{fma_t(a.x, b.x, -(a.y * b.y)), fma_t(a.x, b.y, a.y * b.x)};
+}
+// a / sqrt 2 to half an ulp: the constant with its rounding error
+template <class T>
+__device__ __forceinline__ T half_sqrt(T a) {
+  const T hi = T(0.70710678118654752440);
+  const T lo = T(sizeof(T) == 4 ? 0.70710678118654752440 - (double)0.70710678118654752440f
+                                : -4.8336466567264567e-17);
+  return fma_t(hi, a, lo * a);
+}
+// a times -i
+template <class T>
+__device__ __forceinline__ vec2<T> vmi(vec2<T> a) {
+  return vec2<T>{a.y, -a.x};
+}
+
+__device__ __forceinline__ constexpr int pad8(int i) { return i + (i >> 3); }
+
+template <int LG> struct RegFft {
+  static constexpr int N = 1 << LG, TPF = N / 8, R0 = 1 << (LG % 3), PN = N + N / 8;
+  // offset of the twiddles of the radix-8 pass of sub-length NS
+  static constexpr int off(int ns) {
+    int o = 0;
+    for (int m = R0 == 1 ? 8 : R0; m < ns; m *= 8) o += 7 * m;
+    return o;
+  }
+  // LDS exchanges of one transform
+  static constexpr int exchanges = (LG / 3) + (R0 > 1 ? 1 : 0) - 1;
+  // FP64 4096: one LDS buffer (two would leave a CU one workgroup)
+  template <class T> static constexpr bool one() { return sizeof(T) == 8 && LG == 12; }
+};
+
+// the threads of a sequence meet: a wave's LDS operations are in order
+template <int TPF>
+__device__ __forceinline__ void seq_sync() {
+  if (TPF > 64) {
     __syncthreads();
-    a[base] = cadd<T>(b0, b2);
-    a[base + Ns] = mk<T>(b1.x + b3.y, b1.y - b3.x);
-    a[base + 2 * Ns] = csub<T>(b0, b2);
-    a[base + 3 * Ns] = mk<T>(b1.x - b3.y, b1.y + b3.x);
-    __syncthreads();
+  } else {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+}
+
+template <class T>
+__device__ __forceinline__ void dft8(vec2<T>* v) {
+  typedef vec2<T> V;
+  const V a0 = v[0] + v[4], a4 = v[0] - v[4], a1 = v[1] + v[5], a5 = v[1] - v[5];
+  const V a2 = v[2] + v[6], a6 = v[2] - v[6], a3 = v[3] + v[7], a7 = v[3] - v[7];
+  const V b0 = a0 + a2, b2 = a0 - a2, b1 = a1 + a3, b3 = vmi<T>(a1 - a3);
+  v[0] = b0 + b1;
+  v[4] = b0 - b1;
+  v[2] = b2 + b3;
+  v[6] = b2 - b3;
+  const V c1 = V{half_sqrt(a5.x + a5.y), half_sqrt(a5.y - a5.x)};  // times (1 - i) / sqrt 2
+  const V c2 = vmi<T>(a6);
+  const V c3 = V{half_sqrt(a7.y - a7.x), -half_sqrt(a7.x + a7.y)};  // (-1 - i) / sqrt 2
+  const V d0 = a4 + c2, d2 = a4 - c2, d1 = c1 + c3, d3 = vmi<T>(c1 - c3);
+  v[1] = d0 + d1;
+  v[5] = d0 - d1;
+  v[3] = d2 + d3;
+  v[7] = d2 - d3;
+}
+
+// LDS regions of one sequence: buffer e & 1 of exchange e (one buffer: the
+// same, after a wait for its readers)
+template <class T, int LG>
+__device__ __forceinline__ vec2<T>* xbuf(vec2<T>* b0, vec2<T>* b1, int e) {
+  return RegFft<LG>::template one<T>() || !(e & 1) ? b0 : b1;
+}
+template <class T, int LG>
+__device__ __forceinline__ void xwait() {
+  if (RegFft<LG>::template one<T>()) seq_sync<RegFft<LG>::TPF>();
+}
+template <class T, int LG>
+__device__ __forceinline__ void xread(vec2<T>* v, const vec2<T>* b, int j) {
+  constexpr int st = RegFft<LG>::TPF + RegFft<LG>::TPF / 8;
+  const vec2<T>* p = b + pad8(j);
+#pragma unroll
+  for (int m = 0; m < 8; m++) v[m] = p[m * st];
+}
+// entries j + q N/8 to their places (natural order, padded)
+template <class T, int LG>
+__device__ __forceinline__ void xwrite(const vec2<T>* v, vec2<T>* b, int j) {
+  constexpr int st = RegFft<LG>::TPF + RegFft<LG>::TPF / 8;
+  vec2<T>* p = b + pad8(j);
+#pragma unroll
+  for (int m = 0; m < 8; m++) p[m * st] = v[m];
+}
+
+template <class T, int LG, int NS>
+__device__ __forceinline__ void load_tw(vec2<T>* t, const vec2<T>* __restrict__ tw, int j) {
+  const vec2<T>* p = tw + RegFft<LG>::off(NS) + (j & (NS - 1));
+#pragma unroll
+  for (int q = 0; q < 7; q++) t[q] = p[q * NS];
+}
+
+// the radix-8 pass of sub-length NS and those after it; E: its exchange
+template <class T, int LG, int NS, int E>
+__device__ __forceinline__ void pass8(vec2<T>* v, vec2<T>* t, vec2<T>* b0, vec2<T>* b1, int j,
+                                      const vec2<T>* __restrict__ tw) {
+  typedef RegFft<LG> R;
+  if (NS > 1) {
+#pragma unroll
+    for (int q = 1; q < 8; q++) v[q] = vmul<T>(v[q], t[q - 1]);
+  }
+  dft8<T>(v);
+  if constexpr (NS * 8 < R::N) {
+    load_tw<T, LG, NS * 8>(t, tw, j);
+    const int jm = j & (NS - 1), base = ((j - jm) << 3) + jm;
+    vec2<T>* b = xbuf<T, LG>(b0, b1, E);
+    xwait<T, LG>();
+    if (NS >= 8) {
+      vec2<T>* p = b + pad8(base);
+#pragma unroll
+      for (int q = 0; q < 8; q++) p[q * (NS + NS / 8)] = v[q];
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; q++) b[pad8(base + q * NS)] = v[q];
+    }
+    seq_sync<R::TPF>();
+    xread<T, LG>(v, b, j);
+    pass8<T, LG, NS * 8, E + 1>(v, t, b0, b1, j, tw);
+  }
+}
+
+// forward transform, its exchanges numbered from E
+template <class T, int LG, int E>
+__device__ __forceinline__ void fft_regs(vec2<T>* v, vec2<T>* b0, vec2<T>* b1, int j,
+                                         const vec2<T>* __restrict__ tw) {
+  typedef RegFft<LG> R;
+  typedef vec2<T> V;
+  V t[7];
+  if constexpr (R::R0 == 1) {
+    pass8<T, LG, 1, E>(v, t, b0, b1, j, tw);
+  } else {
+    load_tw<T, LG, R::R0>(t, tw, j);
+    V* b = xbuf<T, LG>(b0, b1, E);
+    xwait<T, LG>();
+    if constexpr (R::R0 == 2) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        V* p = b + pad8(2 * (j + q * R::TPF));
+        p[0] = v[q] + v[q + 4];
+        p[1] = v[q] - v[q + 4];
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        V* p = b + pad8(4 * (j + q * R::TPF));
+        const V s0 = v[q] + v[q + 4], s1 = v[q] - v[q + 4];
+        const V s2 = v[q + 2] + v[q + 6], s3 = vmi<T>(v[q + 2] - v[q + 6]);
+        p[0] = s0 + s2;
+        p[1] = s1 + s3;
+        p[2] = s0 - s2;
+        p[3] = s1 - s3;
+      }
+    }
+    seq_sync<R::TPF>();
+    xread<T, LG>(v, b, j);
+    pass8<T, LG, R::R0, E + 1>(v, t, b0, b1, j, tw);
   }
 }
 
@@ -187,21 +347,6 @@ __device__ __forceinline__ double bsum256(double v, double* sh) {
   }
   __syncthreads();
   return r;
-}
-
-// workgroup size of the FFT passes: 512 threads from 1024 points per
-// workgroup (a radix-4 pass has a butterfly for half of them), 1024 from
-// 4096 (FP64: from 2048), so that a CU holding one or two such workgroups
-// (their LDS) still has waves to switch between.  Measured: 256 threads at
-// 1024 points made the 1024^2 step 9% slower, 1024 threads at 2048 points
-// the 2048^2 FP32 step 9% slower; on the closed 1024^2 basin (2048-point
-// transforms) 1024 threads took the FP64 step from 0.680 to 0.636 ms and
-// the FP32 step from 0.425 to 0.449 ms, 256 threads made both slower.
-template <class T>
-static inline int fft_threads(int points) {
-  // (in place, FP64 4096: exactly one butterfly a thread, 1024)
-  if (sizeof(T) == 8 && points >= 2048) return 1024;
-  return points >= 4096 ? 1024 : (points >= 1024 ? 512 : 256);
 }
 
 // right-hand side of a refinement: (b - mb) - A x64 at padded index k
@@ -353,22 +498,15 @@ __device__ __forceinline__ double masked_res(const FftArgs& a, double g, const i
 // mean of b for the singular operator).  With x64 (or x32): the rows of
 // the residual (b - mb) - A x, mb = (sum of the nbp partials bpin) / (nx ny);
 // bpart, if given, still receives the sums of b.
-template <class T, class TB>
-__global__ __launch_bounds__(1024) void k_fft_rows_fwd(FftArgs a,
-                                                      const TB* __restrict__ b,
-                                                      int gmode,
-                                                      cplx<T>* __restrict__ S,
-                                                      const cplx<T>* __restrict__ tw,
-                                                      double* __restrict__ bpart,
-                                                      const double* __restrict__ x64,
-                                                      const double* __restrict__ bpin,
-                                                      int nbp,
-                                                      const float* __restrict__ x32,
-                                                      FftMask fm = FftMask(),
-                                                      const FftBatchPtrs* __restrict__ bt =
-                                                          nullptr) {
+template <class T, class TB, int LG>
+__global__ __launch_bounds__(LG ? 512 : 1024) void k_fft_rows_fwd(
+    FftArgs a, const TB* __restrict__ b, int gmode, cplx<T>* __restrict__ S,
+    const cplx<T>* __restrict__ tw, double* __restrict__ bpart,
+    const double* __restrict__ x64, const double* __restrict__ bpin, int nbp,
+    const float* __restrict__ x32, FftMask fm = FftMask(),
+    const FftBatchPtrs* __restrict__ bt = nullptr) {
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ double sh[256];
+  __shared__ double sh[16];
   if (bt) {  // a batch: this member's b, spectrum and masks
     b = reinterpret_cast<const TB*>(bt[blockIdx.y].b);
     S = reinterpret_cast<cplx<T>*>(bt[blockIdx.y].S);
@@ -378,7 +516,7 @@ __global__ __launch_bounds__(1024) void k_fft_rows_fwd(FftArgs a,
   cplx<T>* b0 = reinterpret_cast<cplx<T>*>(smem);
   cplx<T>* b1 = b0 + P * nx;
   cplx<T>* tl = b1 + P * nx;  // twiddles, staged in LDS
-  if (!a.ipx)
+  if (!LG)
     for (int w = threadIdx.x; w < nx; w += blockDim.x) tl[w] = tw[w];
   const int y0 = row_block(blockIdx.x, gridDim.x) * 2 * P;
   double mb = 0.0;
@@ -388,12 +526,41 @@ __global__ __launch_bounds__(1024) void k_fft_rows_fwd(FftArgs a,
     mb = bsum256(acc, sh) / ((double)a.onx * (double)a.ony);
   }
   double sum = 0.0;
-  if (a.ex | a.ey) {
-    // extension of a closed direction: the value (or residual) at each of
-    // the problem's points once, written to its doubled-grid point and,
-    // in a closed x, to the mirror point with the reflection's sign (0 on
-    // an odd extension's boundary lines).  Component h of the complex row
-    // pair holds row y0 + 2p + h.
+  // rows y0 + 2p, y0 + 2p + 1 of a periodic grid at column n
+  auto pair_at = [&](int p, int n, double& va, double& vb) {
+    const int64_t ka = (int64_t)(y0 + 2 * p + 3) * a.NXP + n + 3;
+    if (x32) {
+      const double ga = gval(b, ka, a.NXP, gmode), gb = gval(b, ka + a.NXP, a.NXP, gmode);
+      sum += ga + gb;
+      va = rval32(a, ga, x32, y0 + 2 * p, n, mb);
+      vb = rval32(a, gb, x32, y0 + 2 * p + 1, n, mb);
+    } else if (x64) {
+      va = rval(a, b, gmode, x64, ka, mb);
+      vb = rval(a, b, gmode, x64, ka + a.NXP, mb);
+    } else {
+      va = gval(b, ka, a.NXP, gmode);
+      vb = gval(b, ka + a.NXP, a.NXP, gmode);
+      if (fm.in) {
+        if (fm.xr) {
+          va = masked_res(a, va, fm.in, fm.xr, y0 + 2 * p + 3, n + 3);
+          vb = masked_res(a, vb, fm.in, fm.xr, y0 + 2 * p + 4, n + 3);
+        } else {
+          if (!fm.in[ka]) va = 0.0;
+          if (!fm.in[ka + a.NXP]) vb = 0.0;
+        }
+        reinterpret_cast<TB*>(fm.out)[ka] = TB(va);
+        reinterpret_cast<TB*>(fm.out)[ka + a.NXP] = TB(vb);
+      }
+      sum += va + vb;
+    }
+  };
+  // extension of a closed direction: the value (or residual) at each of
+  // the problem's points once, written to its doubled-grid point and,
+  // in a closed x, to the mirror point with the reflection's sign (0 on
+  // an odd extension's boundary lines).  Component h of the complex row
+  // pair holds row y0 + 2p + h.
+  const bool ext = a.ex | a.ey;
+  if (ext) {
     const int nh = a.ex ? a.onx : nx;
     const int lg2 = a.ex ? lg : lg + 1;  // 2 nh = 2^lg2
     T* bs = reinterpret_cast<T*>(b0);
@@ -429,71 +596,81 @@ __global__ __launch_bounds__(1024) void k_fft_rows_fwd(FftArgs a,
         bs[2 * (q + 2 * a.onx - 1 - n) + h] = T(v);
       }
     }
-  } else {
+  } else if (!LG) {
     for (int w = threadIdx.x; w < P * nx; w += blockDim.x) {
-      const int p = w >> lg, n = w & (nx - 1);
-      const int64_t ka = (int64_t)(y0 + 2 * p + 3) * a.NXP + n + 3;
       double va, vb;
-      if (x32) {
-        const double ga = gval(b, ka, a.NXP, gmode), gb = gval(b, ka + a.NXP, a.NXP, gmode);
-        sum += ga + gb;
-        va = rval32(a, ga, x32, y0 + 2 * p, n, mb);
-        vb = rval32(a, gb, x32, y0 + 2 * p + 1, n, mb);
-      } else if (x64) {
-        va = rval(a, b, gmode, x64, ka, mb);
-        vb = rval(a, b, gmode, x64, ka + a.NXP, mb);
-      } else {
-        va = gval(b, ka, a.NXP, gmode);
-        vb = gval(b, ka + a.NXP, a.NXP, gmode);
-        if (fm.in) {
-          if (fm.xr) {
-            va = masked_res(a, va, fm.in, fm.xr, y0 + 2 * p + 3, n + 3);
-            vb = masked_res(a, vb, fm.in, fm.xr, y0 + 2 * p + 4, n + 3);
-          } else {
-            if (!fm.in[ka]) va = 0.0;
-            if (!fm.in[ka + a.NXP]) vb = 0.0;
-          }
-          reinterpret_cast<TB*>(fm.out)[ka] = TB(va);
-          reinterpret_cast<TB*>(fm.out)[ka + a.NXP] = TB(vb);
-        }
-        sum += va + vb;
-      }
+      pair_at(w >> lg, w & (nx - 1), va, vb);
       b0[w] = mk<T>(T(va), T(vb));
     }
   }
-  if (bpart) {
-    sum = bsum256(sum, sh);
-    if (threadIdx.x == 0) bpart[blockIdx.x] = sum;
-  }
-  __syncthreads();
-  const cplx<T>* r = b0;
-  if (a.ipx)
-    fft_inplace<T>(b0, nx, tw);
-  else
-    r = fft_lds<T>(b0, b1, nx, lg, P, tl);
+  auto store_sum = [&]() {
+    if (bpart) {
+      sum = bsum256(sum, sh);
+      if (threadIdx.x == 0) bpart[blockIdx.x] = sum;
+    }
+  };
   // half spectra of the two rows: Xa = (C + D) / 2, Xb = -i (C - D) / 2 with
   // C = F(k), D = conj(F(nx - k))
-  const int n2 = a.nk * 2 * P;
-  const int lgP = __ffs(P) - 1;  // P is a power of two
-  for (int w = threadIdx.x; w < n2; w += blockDim.x) {
-    const int ab = w & 1, p = (w >> 1) & (P - 1), k = (w >> 1) >> lgP;
-    const cplx<T> C = r[p * nx + k];
-    const cplx<T> D0 = r[p * nx + ((nx - k) & (nx - 1))];
-    const cplx<T> D = mk<T>(D0.x, -D0.y);
-    cplx<T> X;
-    if (ab == 0) {
-      X = mk<T>(T(0.5) * (C.x + D.x), T(0.5) * (C.y + D.y));
+  // (closed y: the workgroups cover rows 0 .. ony-1; the column pass forms
+  // the reflected rows itself)
+  auto unpack = [&](int p, int k, T Cx, T Cy, T Dx, T Dy) {  // D0 = F(nx - k)
+    const int64_t at = (int64_t)k * a.ny + y0 + 2 * p;
+    const cplx<T> Xa = mk<T>(T(0.5) * (Cx + Dx), T(0.5) * (Cy - Dy));
+    const cplx<T> Xb = mk<T>(T(0.5) * (Cy + Dy), T(-0.5) * (Cx - Dx));
+    if (a.ex == 1) {  // odd x: the spectrum of an odd real row is imaginary
+      reinterpret_cast<T*>(S)[at] = Xa.y;
+      reinterpret_cast<T*>(S)[at + 1] = Xb.y;
     } else {
-      const cplx<T> u = csub<T>(C, D);
-      X = mk<T>(T(0.5) * u.y, T(-0.5) * u.x);
+      S[at] = Xa;
+      S[at + 1] = Xb;
     }
-    // (closed y: the workgroups cover rows 0 .. ony-1; the column pass
-    // forms the reflected rows itself)
-    const int64_t at = (int64_t)k * a.ny + y0 + 2 * p + ab;
-    if (a.ex == 1)  // odd x: the spectrum of an odd real row is imaginary
-      reinterpret_cast<T*>(S)[at] = X.y;
-    else
-      S[at] = X;
+  };
+  const int lgP = __ffs(P) - 1;  // P is a power of two
+  if constexpr (LG > 0) {
+    typedef RegFft<LG> R;
+    typedef vec2<T> V;
+    V* base = reinterpret_cast<V*>(smem);
+    const int seq = threadIdx.x / R::TPF, j = threadIdx.x & (R::TPF - 1);
+    V* x0 = base + seq * R::PN;
+    V* x1 = base + (P + seq) * R::PN;
+    const V* twv = reinterpret_cast<const V*>(tw);
+    V v[8];
+    constexpr int E = R::exchanges;
+    if (ext) {
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < 8; m++) v[m] = base[seq * R::N + j + m * R::TPF];
+      __syncthreads();  // (the staged rows lie unpadded over all regions)
+    } else {
+#pragma unroll
+      for (int m = 0; m < 8; m++) {
+        double va, vb;
+        pair_at(seq, j + m * R::TPF, va, vb);
+        v[m] = V{T(va), T(vb)};
+      }
+    }
+    store_sum();
+    fft_regs<T, LG, 0>(v, x0, x1, j, twv);
+    V* xo = xbuf<T, LG>(x0, x1, E);
+    xwait<T, LG>();
+    xwrite<T, LG>(v, xo, j);
+    __syncthreads();
+    V* xs = xbuf<T, LG>(base, base + P * R::PN, E);
+    for (int w = threadIdx.x; w < a.nk * P; w += blockDim.x) {
+      const int p = w & (P - 1), k = w >> lgP;
+      const V C = xs[p * R::PN + pad8(k)];
+      const V D = xs[p * R::PN + pad8((R::N - k) & (R::N - 1))];
+      unpack(p, k, C.x, C.y, D.x, D.y);
+    }
+  } else {
+    store_sum();
+    __syncthreads();
+    const cplx<T>* r = fft_lds<T>(b0, b1, nx, lg, P, tl);
+    for (int w = threadIdx.x; w < a.nk * P; w += blockDim.x) {
+      const int p = w & (P - 1), k = w >> lgP;
+      const cplx<T> C = r[p * nx + k], D = r[p * nx + ((nx - k) & (nx - 1))];
+      unpack(p, k, C.x, C.y, D.x, D.y);
+    }
   }
 }
 
@@ -507,18 +684,15 @@ __global__ __launch_bounds__(1024) void k_fft_rows_fwd(FftArgs a,
 // ky, so both stay spectra of real columns) the inverse of
 // F(s1) c1 + i F(s2) c2 = Z (c1 + c2) / 2 + Zc (c1 - c2) / 2 returns the two
 // solved columns as its real and imaginary parts.
-template <class T>
-__device__ void cols_real_pairs(const FftArgs& a, T* __restrict__ Sr,
-                                const cplx<T>* __restrict__ tw,
-                                const double* __restrict__ lamx,
-                                const double* __restrict__ lamy) {
+template <class T, int LG>
+__device__ __forceinline__ void cols_real_pairs(const FftArgs& a, T* __restrict__ Sr,
+                                                const cplx<T>* __restrict__ tw,
+                                                const double* __restrict__ lamx,
+                                                const double* __restrict__ lamy) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int ny = a.ny, lg = a.lgy, on = a.ony;
   const int u0 = blockIdx.x * a.Q;
   const int nq = min(a.Q, a.ncu - u0);
-  cplx<T>* b0 = reinterpret_cast<cplx<T>*>(smem);
-  cplx<T>* b1 = b0 + a.Q * ny;
-  cplx<T>* tl = b1 + a.Q * ny;
   // value of stored column k at doubled row y (closed y: reflected rows)
   auto sval = [&](int k, int y) -> T {
     const T* c = Sr + (int64_t)k * ny;
@@ -526,18 +700,9 @@ __device__ void cols_real_pairs(const FftArgs& a, T* __restrict__ Sr,
     if (a.ey == 1) return y > on ? -c[2 * on - y] : T(0);
     return c[2 * on - 1 - y];
   };
-  for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) {
-    const int q = w >> lg, y = w & (ny - 1);
-    const int k1 = 2 * (u0 + q), k2 = k1 + 1;
-    b0[w] = mk<T>(sval(k1, y), k2 < a.nk ? sval(k2, y) : T(0));
-  }
-  for (int w = threadIdx.x; w < ny; w += blockDim.x) tl[w] = tw[w];
-  __syncthreads();
-  cplx<T>* r = fft_lds<T>(b0, b1, ny, lg, nq, tl);
-  cplx<T>* o = r == b0 ? b1 : b0;
   const double inv = 1.0 / ((double)a.nx * (double)a.ny);
-  for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) {
-    const int q = w >> lg, ky = w & (ny - 1);
+  // the divided spectrum of unit u0 + q at ky, conjugated: inverse by forward
+  auto divided = [&](int q, int ky, T Zx, T Zy, T Mx, T My, T& zx, T& zy) {
     const int k1 = 2 * (u0 + q), k2 = k1 + 1;
     const double l1 = lamx[k1] + lamy[ky];
     const T c1 = l1 != 0.0 ? T(inv / l1) : T(0);
@@ -546,94 +711,185 @@ __device__ void cols_real_pairs(const FftArgs& a, T* __restrict__ Sr,
       const double l2 = lamx[k2] + lamy[ky];
       c2 = l2 != 0.0 ? T(inv / l2) : T(0);
     }
-    const cplx<T> Z = r[w], Zm = r[q * ny + ((ny - ky) & (ny - 1))];
+    if (LG > 0 && a.ey == 1) {
+      // odd columns: an imaginary odd spectrum each, column k2 in the real
+      // part of Z and column k1 in the imaginary one; their even parts are
+      // rounding (k_fft_cols)
+      zx = T(0.5) * (Zx - Mx) * c2;
+      zy = -(T(0.5) * (Zy - My) * c1);
+      return;
+    }
     const T hp = T(0.5) * (c1 + c2), hm = T(0.5) * (c1 - c2);
-    const T zx = Z.x * hp + Zm.x * hm, zy = Z.y * hp - Zm.y * hm;
-    o[w] = mk<T>(zx, -zy);  // conjugate: inverse by forward
-  }
-  __syncthreads();
-  const cplx<T>* z = fft_lds<T>(o, r, ny, lg, nq, tl);
+    zx = Zx * hp + Mx * hm;
+    zy = -(Zy * hp - My * hm);
+  };
   // (closed y: the row pass reads the problem's rows only)
-  for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) {
-    const int q = w >> lg, y = w & (ny - 1);
-    if (a.ey && y >= on) continue;
+  auto put = [&](int q, int y, T vx, T vy) {
+    if (a.ey && y >= on) return;
     const int k1 = 2 * (u0 + q), k2 = k1 + 1;
-    const cplx<T> v = z[w];
-    Sr[(int64_t)k1 * ny + y] = v.x;
-    if (k2 < a.nk) Sr[(int64_t)k2 * ny + y] = -v.y;
+    Sr[(int64_t)k1 * ny + y] = vx;
+    if (k2 < a.nk) Sr[(int64_t)k2 * ny + y] = -vy;
+  };
+  if constexpr (LG > 0) {
+    typedef RegFft<LG> R;
+    typedef vec2<T> V;
+    V* base = reinterpret_cast<V*>(smem);
+    const int seq = threadIdx.x / R::TPF, j = threadIdx.x & (R::TPF - 1);
+    V* x0 = base + seq * R::PN;
+    V* x1 = base + (a.Q + seq) * R::PN;
+    const V* twv = reinterpret_cast<const V*>(tw);
+    const bool live = seq < nq;
+    const int k1 = 2 * (u0 + seq), k2 = k1 + 1;
+    V v[8];
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      const int y = j + m * R::TPF;
+      v[m] = V{live ? sval(k1, y) : T(0), live && k2 < a.nk ? sval(k2, y) : T(0)};
+    }
+    constexpr int E = R::exchanges;
+    fft_regs<T, LG, 0>(v, x0, x1, j, twv);
+    V* xo = xbuf<T, LG>(x0, x1, E);
+    xwait<T, LG>();
+    xwrite<T, LG>(v, xo, j);
+    seq_sync<R::TPF>();
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      const int ky = j + m * R::TPF;
+      const V Zm = xo[pad8((R::N - ky) & (R::N - 1))];
+      T zx = T(0), zy = T(0);
+      if (live) divided(seq, ky, v[m].x, v[m].y, Zm.x, Zm.y, zx, zy);
+      v[m] = V{zx, zy};
+    }
+    fft_regs<T, LG, E + 1>(v, x0, x1, j, twv);
+    if (!live) return;
+#pragma unroll
+    for (int m = 0; m < 8; m++) put(seq, j + m * R::TPF, v[m].x, v[m].y);
+  } else {
+    cplx<T>* b0 = reinterpret_cast<cplx<T>*>(smem);
+    cplx<T>* b1 = b0 + a.Q * ny;
+    cplx<T>* tl = b1 + a.Q * ny;
+    for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) {
+      const int q = w >> lg, y = w & (ny - 1);
+      const int k1 = 2 * (u0 + q), k2 = k1 + 1;
+      b0[w] = mk<T>(sval(k1, y), k2 < a.nk ? sval(k2, y) : T(0));
+    }
+    for (int w = threadIdx.x; w < ny; w += blockDim.x) tl[w] = tw[w];
+    __syncthreads();
+    cplx<T>* r = fft_lds<T>(b0, b1, ny, lg, nq, tl);
+    cplx<T>* o = r == b0 ? b1 : b0;
+    for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) {
+      const int q = w >> lg, ky = w & (ny - 1);
+      const cplx<T> Z = r[w], Zm = r[q * ny + ((ny - ky) & (ny - 1))];
+      T zx, zy;
+      divided(q, ky, Z.x, Z.y, Zm.x, Zm.y, zx, zy);
+      o[w] = mk<T>(zx, zy);
+    }
+    __syncthreads();
+    const cplx<T>* z = fft_lds<T>(o, r, ny, lg, nq, tl);
+    for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) put(w >> lg, w & (ny - 1), z[w].x, z[w].y);
   }
 }
 
-template <class T>
-__global__ __launch_bounds__(1024) void k_fft_cols(FftArgs a,
-                                                  cplx<T>* __restrict__ S,
-                                                  const cplx<T>* __restrict__ tw,
-                                                  const double* __restrict__ lamx,
-                                                  const double* __restrict__ lamy,
-                                                  const FftBatchPtrs* __restrict__ bt =
-                                                      nullptr) {
+template <class T, int LG>
+__global__ __launch_bounds__(LG ? 512 : 1024) void k_fft_cols(
+    FftArgs a, cplx<T>* __restrict__ S, const cplx<T>* __restrict__ tw,
+    const double* __restrict__ lamx, const double* __restrict__ lamy,
+    const FftBatchPtrs* __restrict__ bt = nullptr) {
   extern __shared__ __align__(16) unsigned char smem[];
   if (bt) S = reinterpret_cast<cplx<T>*>(bt[blockIdx.y].S);
   if (a.ex == 1) {
-    cols_real_pairs<T>(a, reinterpret_cast<T*>(S), tw, lamx, lamy);
+    cols_real_pairs<T, LG>(a, reinterpret_cast<T*>(S), tw, lamx, lamy);
     return;
   }
-  const int ny = a.ny, lg = a.lgy;
+  const int ny = a.ny, lg = a.lgy, on = a.ony;
   const int k0 = blockIdx.x * a.Q;
   const int nq = min(a.Q, a.nk - k0);
-  cplx<T>* b0 = reinterpret_cast<cplx<T>*>(smem);
-  cplx<T>* b1 = b0 + a.Q * ny;
-  cplx<T>* tl = b1 + a.Q * ny;
   cplx<T>* col = S + (int64_t)k0 * ny;
-  if (a.ey) {
-    // closed y: rows 0 .. ony-1 are stored; row 2 ony - y is row y with the
-    // opposite sign and row ony a boundary line (odd), or row 2 ony - 1 - y
-    // is row y (even)
-    const int on = a.ony;
-    for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) {
-      const int q = w >> lg, y = w & (ny - 1);
-      cplx<T> v;
-      if (y < on) {
-        v = col[w];
-      } else if (a.ey == 1) {
-        const cplx<T> u = y > on ? col[q * ny + 2 * on - y] : mk<T>(T(0), T(0));
-        v = mk<T>(-u.x, -u.y);
-      } else {
-        v = col[q * ny + 2 * on - 1 - y];
-      }
-      b0[w] = v;
+  // entry y of column k0 + q.  Closed y: rows 0 .. ony-1 are stored; row
+  // 2 ony - y is row y with the opposite sign and row ony a boundary line
+  // (odd), or row 2 ony - 1 - y is row y (even)
+  auto cval = [&](int q, int y) -> cplx<T> {
+    const cplx<T>* c = col + q * ny;
+    if (!a.ey || y < on) return c[y];
+    if (a.ey == 1) {
+      const cplx<T> u = y > on ? c[2 * on - y] : mk<T>(T(0), T(0));
+      return mk<T>(-u.x, -u.y);
+    }
+    return c[2 * on - 1 - y];
+  };
+  const double inv = 1.0 / ((double)a.nx * (double)a.ny);
+  auto factor = [&](int q, int ky) -> T {
+    const double lam = lamx[k0 + q] + lamy[ky];
+    return lam != 0.0 ? T(inv / lam) : T(0);
+  };
+  if constexpr (LG > 0) {
+    typedef RegFft<LG> R;
+    typedef vec2<T> V;
+    V* base = reinterpret_cast<V*>(smem);
+    const int seq = threadIdx.x / R::TPF, j = threadIdx.x & (R::TPF - 1);
+    V* x0 = base + seq * R::PN;
+    V* x1 = base + (a.Q + seq) * R::PN;
+    const V* twv = reinterpret_cast<const V*>(tw);
+    const bool live = seq < nq;
+    V v[8];
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      const cplx<T> c = live ? cval(seq, j + m * R::TPF) : mk<T>(T(0), T(0));
+      v[m] = V{c.x, c.y};
+    }
+    constexpr int E = R::exchanges;
+    fft_regs<T, LG, 0>(v, x0, x1, j, twv);
+    // (without the next exchange, exchange E + 1 goes where E would)
+    constexpr bool swap = !R::template one<T>();
+    V *c0 = swap ? x1 : x0, *c1 = swap ? x0 : x1;
+    if (a.ey == 1) {
+      // the spectrum of an odd extension is odd: what rounding leaves of an
+      // even part would be amplified by 1/lambda and is no solution of the
+      // Dirichlet problem
+      V* xo = xbuf<T, LG>(x0, x1, E);
+      xwait<T, LG>();
+      xwrite<T, LG>(v, xo, j);
+      seq_sync<R::TPF>();
+#pragma unroll
+      for (int m = 0; m < 8; m++)
+        v[m] = T(0.5) * (v[m] - xo[pad8((R::N - (j + m * R::TPF)) & (R::N - 1))]);
+      c0 = x0;
+      c1 = x1;
+    }
+#pragma unroll
+    for (int m = 0; m < 8; m++) {  // conjugate: inverse by forward
+      const T f = live ? factor(seq, j + m * R::TPF) : T(0);
+      v[m] = V{v[m].x * f, -(v[m].y * f)};
+    }
+    fft_regs<T, LG, E + 1>(v, c0, c1, j, twv);
+    if (!live) return;
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      const int y = j + m * R::TPF;
+      if (a.ey && y >= on) continue;  // the row pass reads the problem's rows only
+      col[seq * ny + y] = mk<T>(v[m].x, -v[m].y);
     }
   } else {
-    for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) b0[w] = col[w];
-  }
-  if (!a.ipy)
+    cplx<T>* b0 = reinterpret_cast<cplx<T>*>(smem);
+    cplx<T>* b1 = b0 + a.Q * ny;
+    cplx<T>* tl = b1 + a.Q * ny;
+    for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) b0[w] = cval(w >> lg, w & (ny - 1));
     for (int w = threadIdx.x; w < ny; w += blockDim.x) tl[w] = tw[w];
-  __syncthreads();
-  cplx<T>* r = b0;
-  if (a.ipy)
-    fft_inplace<T>(b0, ny, tw);
-  else
-    r = fft_lds<T>(b0, b1, ny, lg, nq, tl);
-  cplx<T>* o = r == b0 ? b1 : b0;
-  const double inv = 1.0 / ((double)a.nx * (double)a.ny);
-  for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) {
-    const int q = w >> lg, ky = w & (ny - 1);
-    const double lam = lamx[k0 + q] + lamy[ky];
-    const T s = lam != 0.0 ? T(inv / lam) : T(0);
-    const cplx<T> v = r[w];
-    r[w] = mk<T>(v.x * s, -(v.y * s));  // conjugate: inverse by forward
-  }
-  __syncthreads();
-  const cplx<T>* z = r;
-  if (a.ipy)
-    fft_inplace<T>(r, ny, tw);
-  else
-    z = fft_lds<T>(r, o, ny, lg, nq, tl);
-  // (closed y: the row pass reads the problem's rows only)
-  for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) {
-    if (a.ey && (w & (ny - 1)) >= a.ony) continue;
-    const cplx<T> v = z[w];
-    col[w] = mk<T>(v.x, -v.y);
+    __syncthreads();
+    cplx<T>* r = fft_lds<T>(b0, b1, ny, lg, nq, tl);
+    cplx<T>* o = r == b0 ? b1 : b0;
+    for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) {
+      const T f = factor(w >> lg, w & (ny - 1));
+      const cplx<T> v = r[w];
+      r[w] = mk<T>(v.x * f, -(v.y * f));  // conjugate: inverse by forward
+    }
+    __syncthreads();
+    const cplx<T>* z = fft_lds<T>(r, o, ny, lg, nq, tl);
+    for (int w = threadIdx.x; w < nq * ny; w += blockDim.x) {
+      if (a.ey && (w & (ny - 1)) >= on) continue;
+      const cplx<T> v = z[w];
+      col[w] = mk<T>(v.x, -v.y);
+    }
   }
 }
 
@@ -655,18 +911,12 @@ __device__ __forceinline__ void put_images(TX* x, int y, int n, const FftArgs& a
 // x = (TX) x64; 3: x += result in FP64 (x = (TX)(x + result)), also into x64
 // when given (each interior point is read and written by one thread; the
 // halo images written are never read)
-template <class T, class TX, int MODE>
-__global__ __launch_bounds__(1024) void k_fft_rows_inv(FftArgs a,
-                                                      const cplx<T>* __restrict__ S,
-                                                      const cplx<T>* __restrict__ tw,
-                                                      TX* __restrict__ x,
-                                                      double* __restrict__ x64,
-                                                      const double* __restrict__ rs_src =
-                                                          nullptr,
-                                                      double* __restrict__ rs_dst = nullptr,
-                                                      FftMask fm = FftMask(),
-                                                      const FftBatchPtrs* __restrict__ bt =
-                                                          nullptr) {
+template <class T, class TX, int MODE, int LG>
+__global__ __launch_bounds__(LG ? 512 : 1024) void k_fft_rows_inv(
+    FftArgs a, const cplx<T>* __restrict__ S, const cplx<T>* __restrict__ tw,
+    TX* __restrict__ x, double* __restrict__ x64, const double* __restrict__ rs_src = nullptr,
+    double* __restrict__ rs_dst = nullptr, FftMask fm = FftMask(),
+    const FftBatchPtrs* __restrict__ bt = nullptr) {
   extern __shared__ __align__(16) unsigned char smem[];
   if (bt) {  // a batch: this member's spectrum, solution and mask
     S = reinterpret_cast<const cplx<T>*>(bt[blockIdx.y].S);
@@ -680,7 +930,7 @@ __global__ __launch_bounds__(1024) void k_fft_rows_inv(FftArgs a,
   cplx<T>* b0 = reinterpret_cast<cplx<T>*>(smem);
   cplx<T>* b1 = b0 + P * nx;
   cplx<T>* tl = b1 + P * nx;
-  if (!a.ipx)
+  if (!LG)
     for (int w = threadIdx.x; w < nx; w += blockDim.x) tl[w] = tw[w];
   const int y0 = row_block(blockIdx.x, gridDim.x) * 2 * P;
   // conj(C) with C(k) = Xa(k) + i Xb(k) and C(nx - k) = conj(Xa(k)) +
@@ -697,22 +947,21 @@ __global__ __launch_bounds__(1024) void k_fft_rows_inv(FftArgs a,
       Xa = S[at];
       Xb = S[at + 1];
     }
-    cplx<T>* c = b0 + p * nx;
-    c[k] = mk<T>(Xa.x - Xb.y, -(Xa.y + Xb.x));
-    if (k > 0 && k < h) c[nx - k] = mk<T>(Xa.x + Xb.y, -(Xb.x - Xa.y));
+    // The imaginary parts of a real row's modes 0 and nx/2 are 0, through the
+    // column pass too (the spectrum of a real column is symmetric): fft_lds
+    // keeps that to the last bit, the register transforms (fused products) do
+    // not, and what rounding leaves there, amplified by 1/lambda in the low
+    // column modes, would go to the paired row (an FP32 refinement at 1024^2
+    // then contracts by 1e-3 a pass, not 1e-6)
+    if (a.real0 && (k == 0 || k == h)) Xa.y = Xb.y = T(0);
+    cplx<T>* c = b0 + p * (LG ? nx + nx / 8 : nx);
+    c[LG ? pad8(k) : k] = mk<T>(Xa.x - Xb.y, -(Xa.y + Xb.x));
+    if (k > 0 && k < h)
+      c[LG ? pad8(nx - k) : nx - k] = mk<T>(Xa.x + Xb.y, -(Xb.x - Xa.y));
   }
   __syncthreads();
-  const cplx<T>* r = b0;
-  if (a.ipx)
-    fft_inplace<T>(b0, nx, tw);
-  else
-    r = fft_lds<T>(b0, b1, nx, lg, P, tl);
-  // conj of the result: row a = Re, row b = -Im of r
-  for (int w = threadIdx.x; w < P * nx; w += blockDim.x) {
-    const int p = w >> lg, n = w & (nx - 1);
-    const int ya = y0 + 2 * p;
-    const cplx<T> v = r[w];
-    const double va = (double)v.x, vb = -(double)v.y;
+  // rows ya, ya + 1 at column n (va, vb: conj of the result's parts)
+  auto store = [&](int ya, int n, double va, double vb) {
     if (a.ex | a.ey) {
       // closed direction: only the problem's unknowns are written
       for (int h = 0; h < 2; h++) {
@@ -737,7 +986,7 @@ __global__ __launch_bounds__(1024) void k_fft_rows_inv(FftArgs a,
           if (MODE == 1) put_ext<double>(x64, y, n, a, val);
         }
       }
-      continue;
+      return;
     }
     if (MODE == 3 && fm.res) {
       const int64_t ka = (int64_t)(ya + 3) * a.NXP + n + 3;
@@ -770,6 +1019,26 @@ __global__ __launch_bounds__(1024) void k_fft_rows_inv(FftArgs a,
         put_images<double>(x64, ya, n, a, va);
         put_images<double>(x64, ya + 1, n, a, vb);
       }
+    }
+  };
+  if constexpr (LG > 0) {
+    typedef RegFft<LG> R;
+    typedef vec2<T> V;
+    V* base = reinterpret_cast<V*>(smem);
+    const int seq = threadIdx.x / R::TPF, j = threadIdx.x & (R::TPF - 1);
+    V* x0 = base + seq * R::PN;
+    V* x1 = base + (P + seq) * R::PN;
+    V v[8];
+    xread<T, LG>(v, x0, j);
+    fft_regs<T, LG, 1>(v, x0, x1, j, reinterpret_cast<const V*>(tw));
+#pragma unroll
+    for (int m = 0; m < 8; m++)
+      store(y0 + 2 * seq, j + m * R::TPF, (double)v[m].x, -(double)v[m].y);
+  } else {
+    const cplx<T>* r = fft_lds<T>(b0, b1, nx, lg, P, tl);
+    for (int w = threadIdx.x; w < P * nx; w += blockDim.x) {
+      const cplx<T> v = r[w];
+      store(y0 + 2 * (w >> lg), w & (nx - 1), (double)v.x, -(double)v.y);
     }
   }
 }
@@ -893,10 +1162,16 @@ __global__ __launch_bounds__(256) void k_fft_stats(const double* __restrict__ pa
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
+struct FftPlan {
+  int P = 1, Q = 1;      // row pairs, columns (units) per workgroup
+  int lgr = 0, lgc = 0;  // register transforms of rows, columns (0: fft_lds)
+  int thr = 0, thc = 0;  // threads
+  size_t lr = 0, lc = 0; // LDS
+};
+
 struct FftSolver {
   FftArgs a{};
-  int P64 = 1, Q64 = 1, P32 = 1, Q32 = 1;
-  size_t lds_r64 = 0, lds_c64 = 0, lds_r32 = 0, lds_c32 = 0;
+  FftPlan p64, p32;
   double* lamx = nullptr;
   double* lamy = nullptr;
   double2* twx64 = nullptr;
@@ -926,19 +1201,22 @@ static int ilog2(int64_t v) {
 
 static bool pow2(int64_t v) { return v > 0 && (v & (v - 1)) == 0; }
 
-// a transform of n points in place: 4096 points of a workgroup of 1024
-// threads, where two buffers and the twiddles exceed the LDS
-static bool inplace(int64_t n, bool f64) { return f64 && n == 4096; }
+// log2 of the points of a register transform (RegFft), 0: fft_lds
+static int reg_lg(int64_t n, int64_t from) {
+  int l = 0;
+  while ((int64_t(1) << l) < n) l++;
+  return n >= from && l <= 12 ? l : 0;
+}
 
 bool fft_fits(int64_t ny, int64_t nx, int xper, int yper, bool f64, bool two_buffers) {
-  // one row (column) per workgroup: two FFT buffers and the twiddles in LDS
-  // (plan_blocks), or 4096 points of a periodic direction in place (closed
-  // directions: the column pass of an odd x reads a mirror entry)
+  // one row (column) per workgroup, two FFT buffers and the twiddles, in LDS;
+  // or FP64 4096 points of a periodic direction in one buffer (RegFft)
   const size_t c = f64 ? 16 : 8;
   const int64_t tx = xper ? nx : 2 * nx, ty = yper ? ny : 2 * ny;
   auto lds = [&](int64_t n) { return 3 * (size_t)n * c <= 160 * 1024; };
-  const bool okx = lds(tx) || (!two_buffers && inplace(tx, f64) && xper);
-  const bool oky = lds(ty) || (!two_buffers && inplace(ty, f64) && xper && yper);
+  auto one = [&](int64_t n) { return !two_buffers && f64 && n == 4096; };
+  const bool okx = lds(tx) || (one(tx) && xper);
+  const bool oky = lds(ty) || (one(ty) && xper && yper);
   return okx && oky;
 }
 
@@ -989,47 +1267,129 @@ static C* twiddles(FftSolver* f, int N) {
   return d;
 }
 
-static const size_t LDS_CAP = 64 * 1024;
-
-// one row pair (one spectral column) per workgroup, more for short rows
-// (columns) so that a workgroup holds at least 1024 points: many
-// workgroups keep all CUs busy
-template <class T>
-static void plan_blocks(const FftArgs& a, int& P, int& Q, size_t& lr, size_t& lc) {
-  const size_t c = sizeof(T) * 2;
-  P = a.nx >= 1024 ? 1 : 1024 / a.nx;
-  // (closed y: the row passes cover the first half of the doubled rows)
-  while (P > 1 && ((a.ny / 2) % P || (a.ey && (a.ny / 4) % P) ||
-                   (2 * P + 1) * a.nx * c > LDS_CAP))
-    P >>= 1;
-  Q = a.ny >= 1024 ? 1 : 1024 / a.ny;
-  // (odd x: a unit is a pair of columns; as many workgroups as unpaired)
-  if (a.ex == 1 && Q > 1) Q >>= 1;
-  while (Q > 1 && (2 * Q + 1) * a.ny * c > LDS_CAP) Q >>= 1;
-  lr = (a.ipx ? 1 : 2 * (size_t)P + 1) * a.nx * c;
-  lc = (a.ipy ? 1 : 2 * (size_t)Q + 1) * a.ny * c;
+// The same for the register transforms: the radix-8 pass of sub-length Ns
+// (from the first that has twiddles) reads seven runs of Ns entries, run q
+// holding exp(-2 pi i q jm / (8 Ns)).
+template <class C>
+static C* reg_twiddles(FftSolver* f, int N, int lg) {
+  std::vector<C> t;
+  t.reserve(N);
+  for (int Ns = lg % 3 ? 1 << (lg % 3) : 8; Ns < N; Ns *= 8)
+    for (int q = 1; q < 8; q++)
+      for (int jm = 0; jm < Ns; jm++) {
+        const long double ang = -2.0L * 3.14159265358979323846264338327950288L *
+                                (long double)(q * jm) / (long double)(8 * Ns);
+        C c;
+        c.x = (decltype(c.x))cosl(ang);
+        c.y = (decltype(c.y))sinl(ang);
+        t.push_back(c);
+      }
+  C* d = falloc<C>(f, sizeof(C) * t.size());
+  F2D_HIP(hipMemcpy(d, t.data(), sizeof(C) * t.size(), hipMemcpyHostToDevice));
+  return d;
 }
 
+static const size_t LDS_CAP = 64 * 1024;
+
+// sequences per workgroup of a register transform of 2^lg points: one wave
+// at least
+static int reg_seqs(int lg) { return lg >= 9 ? 1 : 2; }
+
+// Register transforms (RegFft) or passes through LDS (fft_lds).  Registers
+// (us a pass, fft_lds first): from 2048 points in every pass (FP64 2048^2
+// periodic: rows 30.5 -> 29.5, columns 44.5 -> 25.5, inverse rows 31.3 ->
+// 23.1; FP32 17.8 -> 14.4, 21.4 -> 15.9, 19.4 -> 16.6), and FP64 columns from
+// 256 points (256^2 6.4 -> 5.3, 1024^2 11.3 -> 8.5), from 1024 where y is
+// closed (512^2 closed 9.3 -> 8.4; 256^2 closed 6.9 -> 6.9).  Shorter rows
+// are bound by their strided stores and lose with 8 points a thread (1024^2
+// FP64 8.0 -> 9.6, closed 512^2 6.7 -> 8.3); shorter FP32 columns gain 1 us
+// alone and nothing in a step (1024^2: 49.3 us with either; two solves side
+// by side, 512^2: 1% slower).
+// One row pair (one spectral column) per workgroup, more for short rows
+// (columns): many workgroups keep all CUs busy.  Threads a workgroup (fft_lds:
+// 512 from 1024 points per workgroup, 256 below) and its LDS.
 template <class T>
-static void set_lds(size_t lr, size_t lc) {
-  // (the row passes hold 2 KB of static LDS besides)
-  if (lr > 62 * 1024) {
-    F2D_HIP(hipFuncSetAttribute((const void*)k_fft_rows_fwd<T, double>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr));
-    F2D_HIP(hipFuncSetAttribute((const void*)k_fft_rows_fwd<T, float>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr));
-    F2D_HIP(hipFuncSetAttribute((const void*)k_fft_rows_inv<T, T, 0>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr));
-    F2D_HIP(hipFuncSetAttribute((const void*)k_fft_rows_inv<T, T, 1>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr));
-    F2D_HIP(hipFuncSetAttribute((const void*)k_fft_rows_inv<T, T, 2>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr));
-    F2D_HIP(hipFuncSetAttribute((const void*)k_fft_rows_inv<T, T, 3>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr));
+static void plan_blocks(const FftArgs& a, FftPlan& p) {
+  const size_t c = sizeof(T) * 2;
+  p.lgr = reg_lg(a.nx, 2048);
+  p.lgc = reg_lg(a.ny, sizeof(T) == 4 ? 2048 : a.ey ? 1024 : 256);
+  auto reg = [&](int n, int lg, int k, int& th, size_t& lds) {
+    th = k * (n / 8);
+    const int bufs = sizeof(T) == 8 && lg == 12 ? 1 : 2;
+    lds = (size_t)bufs * k * (n + n / 8) * c;
+  };
+  p.P = p.lgr ? reg_seqs(p.lgr) : (a.nx >= 1024 ? 1 : 1024 / a.nx);
+  // (closed y: the row passes cover the first half of the doubled rows)
+  while (p.P > 1 && ((a.ny / 2) % p.P || (a.ey && (a.ny / 4) % p.P) ||
+                     (2 * p.P + 1) * a.nx * c > LDS_CAP))
+    p.P >>= 1;
+  p.Q = p.lgc ? reg_seqs(p.lgc) : (a.ny >= 1024 ? 1 : 1024 / a.ny);
+  // (odd x: a unit is a pair of columns; as many workgroups as unpaired)
+  if (!p.lgc && a.ex == 1 && p.Q > 1) p.Q >>= 1;
+  while (p.Q > 1 && !p.lgc && (2 * p.Q + 1) * a.ny * c > LDS_CAP) p.Q >>= 1;
+  if (p.lgr) {
+    reg(a.nx, p.lgr, p.P, p.thr, p.lr);
+  } else {
+    p.thr = p.P * a.nx >= 1024 ? 512 : 256;
+    p.lr = (2 * (size_t)p.P + 1) * a.nx * c;
   }
-  if (lc > 62 * 1024)
-    F2D_HIP(hipFuncSetAttribute((const void*)k_fft_cols<T>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lc));
+  if (p.lgc) {
+    reg(a.ny, p.lgc, p.Q, p.thc, p.lc);
+  } else {
+    p.thc = p.Q * a.ny >= 1024 ? 512 : 256;
+    p.lc = (2 * (size_t)p.Q + 1) * a.ny * c;
+  }
+}
+
+template <class K>
+static void lds_limit(K* kernel, size_t lds) {
+  // (the row passes hold some static LDS besides)
+  if (lds > 62 * 1024)
+    F2D_HIP(hipFuncSetAttribute((const void*)kernel,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+}
+
+// the three passes on a plan, each kernel's instantiation by its length
+template <class T, class TB, class... A>
+static void rows_fwd(const FftPlan& p, dim3 grid, hipStream_t s, A... args) {
+  auto go = [&](auto* k) {
+    lds_limit(k, p.lr);
+    k<<<grid, p.thr, p.lr, s>>>(args...);
+  };
+  switch (p.lgr) {
+    case 11: go(k_fft_rows_fwd<T, TB, 11>); break;
+    case 12: go(k_fft_rows_fwd<T, TB, 12>); break;
+    default: go(k_fft_rows_fwd<T, TB, 0>);
+  }
+}
+template <class T, class... A>
+static void cols(const FftPlan& p, dim3 grid, hipStream_t s, A... args) {
+  auto go = [&](auto* k) {
+    lds_limit(k, p.lc);
+    k<<<grid, p.thc, p.lc, s>>>(args...);
+  };
+  if constexpr (sizeof(T) == 8) {  // (plan_blocks)
+    if (p.lgc == 8) return go(k_fft_cols<T, 8>);
+    if (p.lgc == 9) return go(k_fft_cols<T, 9>);
+    if (p.lgc == 10) return go(k_fft_cols<T, 10>);
+  }
+  switch (p.lgc) {
+    case 11: go(k_fft_cols<T, 11>); break;
+    case 12: go(k_fft_cols<T, 12>); break;
+    default: go(k_fft_cols<T, 0>);
+  }
+}
+template <class T, class TX, int MODE, class... A>
+static void rows_inv(const FftPlan& p, dim3 grid, hipStream_t s, A... args) {
+  auto go = [&](auto* k) {
+    lds_limit(k, p.lr);
+    k<<<grid, p.thr, p.lr, s>>>(args...);
+  };
+  switch (p.lgr) {
+    case 11: go(k_fft_rows_inv<T, TX, MODE, 11>); break;
+    case 12: go(k_fft_rows_inv<T, TX, MODE, 12>); break;
+    default: go(k_fft_rows_inv<T, TX, MODE, 0>);
+  }
 }
 
 FftSolver* fft_create(int64_t ny, int64_t nx, double dx, double dy,
@@ -1077,26 +1437,24 @@ FftSolver* fft_create(int64_t ny, int64_t nx, double dx, double dy,
     f->mean_b = falloc<double>(f, sizeof(double));
     f->rowsum[0] = falloc<double>(f, sizeof(double) * (ny / 2 + 1));
     f->rowsum[1] = falloc<double>(f, sizeof(double) * (ny / 2 + 1));
+    auto table = [&](auto zero, int n, int lg) {
+      typedef decltype(zero) C;
+      return lg ? reg_twiddles<C>(f, n, lg) : twiddles<C>(f, n);
+    };
     if (f64) {
-      // (a plan of both precisions would share these: none is made)
-      a.ipx = inplace(nx, true) ? 1 : 0;
-      a.ipy = inplace(ny, true) ? 1 : 0;
-      F2D_REQUIRE(!(a.ipx || a.ipy) || !f32, "in-place plans are FP64 only");
-      f->twx64 = twiddles<double2>(f, (int)nx);
-      f->twy64 = twiddles<double2>(f, (int)ny);
-      f->S64 = falloc<double2>(f, sizeof(double2) * nspec);
-      plan_blocks<double>(a, f->P64, f->Q64, f->lds_r64, f->lds_c64);
-      F2D_REQUIRE(f->lds_r64 <= 160 * 1024 && f->lds_c64 <= 160 * 1024,
+      plan_blocks<double>(a, f->p64);
+      F2D_REQUIRE(f->p64.lr <= 160 * 1024 && f->p64.lc <= 160 * 1024,
                   "FFT rows do not fit in LDS");
-      set_lds<double>(f->lds_r64, f->lds_c64);
+      f->twx64 = table(double2{}, (int)nx, f->p64.lgr);
+      f->twy64 = table(double2{}, (int)ny, f->p64.lgc);
+      f->S64 = falloc<double2>(f, sizeof(double2) * nspec);
     }
     if (f32) {
-      f->twx32 = twiddles<float2>(f, (int)nx);
-      f->twy32 = twiddles<float2>(f, (int)ny);
+      plan_blocks<float>(a, f->p32);
+      f->twx32 = table(float2{}, (int)nx, f->p32.lgr);
+      f->twy32 = table(float2{}, (int)ny, f->p32.lgc);
       f->S32 = falloc<float2>(f, sizeof(float2) * nspec);
       f->x64 = falloc<double>(f, sizeof(double) * npad);
-      plan_blocks<float>(a, f->P32, f->Q32, f->lds_r32, f->lds_c32);
-      set_lds<float>(f->lds_r32, f->lds_c32);
     }
     F2D_HIP(hipDeviceSynchronize());
   } catch (...) {
@@ -1126,21 +1484,23 @@ static void spectral(FftSolver* f, const TB* b, int gmode, TX* x, double* x64,
                      const double* rs_in = nullptr, bool keep_sums = false) {
   FftArgs a = f->a;
   const bool d = sizeof(T) == 8;
-  a.P = d ? f->P64 : f->P32;
-  a.Q = d ? f->Q64 : f->Q32;
-  const size_t lr = d ? f->lds_r64 : f->lds_r32, lc = d ? f->lds_c64 : f->lds_c32;
+  const FftPlan& p = d ? f->p64 : f->p32;
+  a.P = p.P;
+  a.Q = p.Q;
+  a.real0 = p.lgc > 0;
   cplx<T>* S = d ? (cplx<T>*)f->S64 : (cplx<T>*)f->S32;
   const cplx<T>* twx = d ? (const cplx<T>*)f->twx64 : (const cplx<T>*)f->twx32;
   const cplx<T>* twy = d ? (const cplx<T>*)f->twy64 : (const cplx<T>*)f->twy32;
   // closed y: rows 0 .. ony-1 only (the rest mirror them, see k_fft_rows_fwd)
   const int gr = (a.ey ? a.ony : a.ny) / (2 * a.P), gc = (a.ncu + a.Q - 1) / a.Q;
   const double* bpin = ((xres || xres32) && a.singular) ? rs_in : nullptr;
-  k_fft_rows_fwd<T, TB><<<gr, fft_threads<T>(a.P * a.nx), lr, s>>>(a, b, gmode, S, twx, rs_out, xres, bpin, gr,
-                                            xres32);
-  k_fft_cols<T><<<gc, fft_threads<T>(a.Q * a.ny), lc, s>>>(a, S, twy, f->lamx, f->lamy);
-  k_fft_rows_inv<T, TX, MODE><<<gr, fft_threads<T>(a.P * a.nx), lr, s>>>(a, S, twx, x, x64,
-                                                  keep_sums ? f->rowsum[1] : nullptr,
-                                                  keep_sums ? f->rowsum[0] : nullptr);
+  const FftBatchPtrs* none = nullptr;
+  rows_fwd<T, TB>(p, dim3(gr), s, a, b, gmode, S, twx, rs_out, xres, bpin, gr, xres32,
+                  FftMask(), none);
+  cols<T>(p, dim3(gc), s, a, S, twy, (const double*)f->lamx, (const double*)f->lamy, none);
+  rows_inv<T, TX, MODE>(p, dim3(gr), s, a, (const cplx<T>*)S, twx, x, x64,
+                        (const double*)(keep_sums ? f->rowsum[1] : nullptr),
+                        keep_sums ? f->rowsum[0] : (double*)nullptr, FftMask(), none);
 }
 
 template <class TB>
@@ -1220,21 +1580,27 @@ void fft_solve_f32_batch(FftSolver* f, int nm, const FftBatchPtrs* table, hipStr
                          bool acc) {
   F2D_REQUIRE(f->S32, "FFT solver built without FP32 buffers");
   FftArgs a = f->a;
-  a.P = f->P32;
-  a.Q = f->Q32;
+  const FftPlan& p = f->p32;
+  a.P = p.P;
+  a.Q = p.Q;
+  a.real0 = p.lgc > 0;
   const int gr = (a.ey ? a.ony : a.ny) / (2 * a.P), gc = (a.ncu + a.Q - 1) / a.Q;
   const dim3 grr(gr, nm), grc(gc, nm);
-  k_fft_rows_fwd<float, float><<<grr, fft_threads<float>(a.P * a.nx), f->lds_r32, s>>>(
-      a, nullptr, 0, nullptr, f->twx32, nullptr, nullptr, nullptr, gr, nullptr, FftMask(),
-      table);
-  k_fft_cols<float><<<grc, fft_threads<float>(a.Q * a.ny), f->lds_c32, s>>>(a, nullptr, f->twy32,
-                                                                     f->lamx, f->lamy, table);
+  const float* nof = nullptr;
+  const double* nod = nullptr;
+  rows_fwd<float, float>(p, grr, s, a, nof, 0, (float2*)nullptr, (const float2*)f->twx32,
+                         (double*)nullptr, nod, nod, gr, nof, FftMask(), table);
+  cols<float>(p, grc, s, a, (float2*)nullptr, (const float2*)f->twy32, (const double*)f->lamx,
+              (const double*)f->lamy, table);
+  auto inv = [&](auto mode) {
+    rows_inv<float, float, decltype(mode)::value>(
+        p, grr, s, a, (const float2*)nullptr, (const float2*)f->twx32, (float*)nullptr,
+        (double*)nullptr, nod, (double*)nullptr, FftMask(), table);
+  };
   if (acc)
-    k_fft_rows_inv<float, float, 3><<<grr, fft_threads<float>(a.P * a.nx), f->lds_r32, s>>>(
-        a, nullptr, f->twx32, nullptr, nullptr, nullptr, nullptr, FftMask(), table);
+    inv(std::integral_constant<int, 3>());
   else
-    k_fft_rows_inv<float, float, 0><<<grr, fft_threads<float>(a.P * a.nx), f->lds_r32, s>>>(
-        a, nullptr, f->twx32, nullptr, nullptr, nullptr, nullptr, FftMask(), table);
+    inv(std::integral_constant<int, 0>());
 }
 
 void fft_solve_f32_masked(FftSolver* f, const float* b, int gmode, float* x, const FftMask& m,
@@ -1242,8 +1608,10 @@ void fft_solve_f32_masked(FftSolver* f, const float* b, int gmode, float* x, con
   F2D_REQUIRE(f->S32, "FFT solver built without FP32 buffers");
   F2D_REQUIRE(!m.in || m.out, "a masked right-hand side needs its output array");
   FftArgs a = f->a;
-  a.P = f->P32;
-  a.Q = f->Q32;
+  const FftPlan& p = f->p32;
+  a.P = p.P;
+  a.Q = p.Q;
+  a.real0 = p.lgc > 0;
   const int gr = (a.ey ? a.ony : a.ny) / (2 * a.P), gc = (a.ncu + a.Q - 1) / a.Q;
   FftMask mf = m, mi = m;
   mf.res = nullptr;
@@ -1251,17 +1619,21 @@ void fft_solve_f32_masked(FftSolver* f, const float* b, int gmode, float* x, con
   mi.out = nullptr;
   mi.xr = nullptr;
   F2D_REQUIRE(!acc || mi.res, "an accumulating masked solve needs its mask");
-  k_fft_rows_fwd<float, float><<<gr, fft_threads<float>(a.P * a.nx), f->lds_r32, s>>>(
-      a, b, gmode, (float2*)f->S32, (const float2*)f->twx32, nullptr, nullptr, nullptr, gr,
-      nullptr, mf);
-  k_fft_cols<float><<<gc, fft_threads<float>(a.Q * a.ny), f->lds_c32, s>>>(
-      a, (float2*)f->S32, (const float2*)f->twy32, f->lamx, f->lamy);
+  const FftBatchPtrs* none = nullptr;
+  const double* nod = nullptr;
+  rows_fwd<float, float>(p, dim3(gr), s, a, b, gmode, (float2*)f->S32, (const float2*)f->twx32,
+                         (double*)nullptr, nod, nod, gr, (const float*)nullptr, mf, none);
+  cols<float>(p, dim3(gc), s, a, (float2*)f->S32, (const float2*)f->twy32,
+              (const double*)f->lamx, (const double*)f->lamy, none);
+  auto inv = [&](auto mode) {
+    rows_inv<float, float, decltype(mode)::value>(
+        p, dim3(gr), s, a, (const float2*)f->S32, (const float2*)f->twx32, x, (double*)nullptr,
+        nod, (double*)nullptr, mi, none);
+  };
   if (acc)
-    k_fft_rows_inv<float, float, 3><<<gr, fft_threads<float>(a.P * a.nx), f->lds_r32, s>>>(
-        a, (const float2*)f->S32, (const float2*)f->twx32, x, nullptr, nullptr, nullptr, mi);
+    inv(std::integral_constant<int, 3>());
   else
-    k_fft_rows_inv<float, float, 0><<<gr, fft_threads<float>(a.P * a.nx), f->lds_r32, s>>>(
-        a, (const float2*)f->S32, (const float2*)f->twx32, x, nullptr, nullptr, nullptr, mi);
+    inv(std::integral_constant<int, 0>());
 }
 
 // whether two plans solve the same operator (same args and eigenvalues)
@@ -1269,7 +1641,7 @@ bool fft_same_plan(const FftSolver* f, const FftSolver* g) {
   const FftArgs &a = f->a, &b = g->a;
   return a.nx == b.nx && a.ny == b.ny && a.ex == b.ex && a.ey == b.ey && a.onx == b.onx &&
          a.ony == b.ony && a.cx == b.cx && a.cy == b.cy && a.d == b.d &&
-         a.singular == b.singular && f->P32 == g->P32 && f->Q32 == g->Q32 &&
+         a.singular == b.singular && f->p32.P == g->p32.P && f->p32.Q == g->p32.Q &&
          f->S32 != nullptr && g->S32 != nullptr;
 }
 
@@ -1294,9 +1666,10 @@ double fft_bench(FftSolver* f, bool f64, int kind, int reps, hipStream_t s,
   const size_t npad = (size_t)(f->a.ony + 6) * (f->a.onx + 6);
   if (!f->bench_buf) f->bench_buf = falloc<double>(f, sizeof(double) * npad);
   FftArgs a = f->a;
-  a.P = f64 ? f->P64 : f->P32;
-  a.Q = f64 ? f->Q64 : f->Q32;
-  const size_t lr = f64 ? f->lds_r64 : f->lds_r32, lc = f64 ? f->lds_c64 : f->lds_c32;
+  const FftPlan& p = f64 ? f->p64 : f->p32;
+  a.P = p.P;
+  a.Q = p.Q;
+  a.real0 = p.lgc > 0;
   // closed y: rows 0 .. ony-1 only (the rest mirror them, see k_fft_rows_fwd)
   const int gr = (a.ey ? a.ony : a.ny) / (2 * a.P), gc = (a.ncu + a.Q - 1) / a.Q;
   const double N = (double)a.nx * a.ny, NS = (double)a.nk * a.ny;
@@ -1304,39 +1677,44 @@ double fft_bench(FftSolver* f, bool f64, int kind, int reps, hipStream_t s,
   hipEvent_t e0, e1;
   F2D_HIP(hipEventCreate(&e0));
   F2D_HIP(hipEventCreate(&e1));
+  const FftBatchPtrs* none = nullptr;
+  const double* nod = nullptr;
+  const float* nof = nullptr;
+  double* out = nullptr;
+  const double *lx = f->lamx, *ly = f->lamy;
   auto launch = [&]() {
     if (f64) {
       double* buf = f->bench_buf;
+      const double2 *tx = f->twx64, *ty = f->twy64, *S = f->S64;
       if (kind == 0)
-        k_fft_rows_fwd<double, double><<<gr, fft_threads<double>(a.P * a.nx), lr, s>>>(a, buf, 0, f->S64, f->twx64,
-                                                           nullptr, nullptr, nullptr, gr,
-                                                           nullptr);
+        rows_fwd<double, double>(p, dim3(gr), s, a, (const double*)buf, 0, f->S64, tx, out, nod,
+                                 nod, gr, nof, FftMask(), none);
       else if (kind == 2)
-        k_fft_cols<double><<<gc, fft_threads<double>(a.Q * a.ny), lc, s>>>(a, f->S64, f->twy64, f->lamx, f->lamy);
+        cols<double>(p, dim3(gc), s, a, f->S64, ty, lx, ly, none);
       else
-        k_fft_rows_inv<double, double, 0><<<gr, fft_threads<double>(a.P * a.nx), lr, s>>>(a, f->S64, f->twx64, buf,
-                                                              nullptr);
+        rows_inv<double, double, 0>(p, dim3(gr), s, a, S, tx, buf, out, nod, out, FftMask(),
+                                    none);
     } else {
       float* buf = reinterpret_cast<float*>(f->bench_buf);
+      const float2 *tx = f->twx32, *ty = f->twy32, *S = f->S32;
+      const double* x64 = f->x64;
       if (kind == 0 || kind == 1)
-        k_fft_rows_fwd<float, float><<<gr, fft_threads<float>(a.P * a.nx), lr, s>>>(
-            a, buf, 0, f->S32, f->twx32, nullptr, kind == 1 ? f->x64 : nullptr,
-            nullptr, gr, nullptr);
+        rows_fwd<float, float>(p, dim3(gr), s, a, (const float*)buf, 0, f->S32, tx, out,
+                               kind == 1 ? x64 : nod, nod, gr, nof, FftMask(), none);
       else if (kind == 2)
-        k_fft_cols<float><<<gc, fft_threads<float>(a.Q * a.ny), lc, s>>>(a, f->S32, f->twy32, f->lamx, f->lamy);
+        cols<float>(p, dim3(gc), s, a, f->S32, ty, lx, ly, none);
       else if (kind == 3)
-        k_fft_rows_inv<float, float, 0><<<gr, fft_threads<float>(a.P * a.nx), lr, s>>>(a, f->S32, f->twx32, buf,
-                                                            nullptr);
+        rows_inv<float, float, 0>(p, dim3(gr), s, a, S, tx, buf, out, nod, out, FftMask(), none);
       else if (kind == 4)
-        k_fft_rows_inv<float, float, 2><<<gr, fft_threads<float>(a.P * a.nx), lr, s>>>(a, f->S32, f->twx32, buf,
-                                                            f->x64);
+        rows_inv<float, float, 2>(p, dim3(gr), s, a, S, tx, buf, f->x64, nod, out, FftMask(),
+                                  none);
       else if (kind == 5)
-        k_fft_rows_fwd<float, float><<<gr, fft_threads<float>(a.P * a.nx), lr, s>>>(
-            a, buf, 0, f->S32, f->twx32, f->rowsum[1], nullptr,
-            a.singular ? f->rowsum[0] : nullptr, gr, buf);
+        rows_fwd<float, float>(p, dim3(gr), s, a, (const float*)buf, 0, f->S32, tx,
+                               f->rowsum[1], nod,
+                               (const double*)(a.singular ? f->rowsum[0] : nullptr), gr,
+                               (const float*)buf, FftMask(), none);
       else
-        k_fft_rows_inv<float, float, 3><<<gr, fft_threads<float>(a.P * a.nx), lr, s>>>(a, f->S32, f->twx32, buf,
-                                                            nullptr);
+        rows_inv<float, float, 3>(p, dim3(gr), s, a, S, tx, buf, out, nod, out, FftMask(), none);
     }
   };
   launch();
