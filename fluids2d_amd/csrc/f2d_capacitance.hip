@@ -7,19 +7,17 @@
 // the masked operator of get_Laplacian_sparse (elliptic.py:114-195).
 //
 // Kernels of one FP64 solve:
-//   k_cap_rhs    b masked to the unknowns W (b_W), zero elsewhere
-//   (3 spectral passes)   y = A_R^-1 b_W
+//   (3 spectral passes)   y = A_R^-1 b_W; the first masks b to the unknowns W
 //   k_cap_symv   partial products of the symmetric M = (-C)^-1 with y_B,
 //                one 64 x 64 tile of its lower triangle per workgroup
 //   k_cap_symv_sum  s = M y_B from the partials, written into b_W at B
-//   (3 spectral passes)   y = A_R^-1 (b_W + P_B^T s)
-//   k_cap_out    x = y at the unknowns W
+//   (3 spectral passes)   y = A_R^-1 (b_W + P_B^T s), the last writes x at W
 // The FP32 mode wraps the same sequence, in FP32 with an FP32 M, into FP64
 // refinement (k_cap_res forms the FP64 residual, k_cap_acc accumulates).
 //
 // Rectangles whose sizes are not powers of two take the eigenvector solve
 // (f2d_modal) in place of the spectral passes, in FP64 for every precision of
-// b and x: no refinement to make, and its last pass writes x at W itself.
+// b and x: no refinement to make; k_cap_rhs masks b.
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>
 
@@ -202,34 +200,38 @@ __global__ __launch_bounds__(256) void k_cap_symv(const T* __restrict__ Mt, int 
 }
 
 // s_i = sum_{J <= I} part[(I, J)][0][r] + sum_{K > I} part[(K, I)][1][r],
-// i = 64 I + r, into rhs at the point B_i
+// i = 64 I + r, into rhs at the point B_i.  A workgroup takes one tile row I,
+// its wave p the partials p, p + 16, ...: bound by the latency of the loads
+// (a thread that sums all nt partials of a row serially, n / 256 workgroups:
+// 7.2 us on a 512^2 basin, this 3.6 us).
+constexpr int CSUM = 16;  // waves of the sum
 template <class T>
-__device__ __forceinline__ void cap_symv_sum_at(int n, int nt, const double* __restrict__ part,
-                                                const int* __restrict__ bidx,
-                                                T* __restrict__ rhs, int i) {
-  const int I = i / CT, r = i - I * CT;
+__device__ __forceinline__ void cap_symv_sum_tile(int n, int nt, const double* __restrict__ part,
+                                                  const int* __restrict__ bidx,
+                                                  T* __restrict__ rhs, int I) {
+  __shared__ double sh[CSUM][CT];
+  const int r = threadIdx.x & (CT - 1), p = threadIdx.x / CT;
   double acc = 0.0;
-  for (int J = 0; J <= I; J++) acc += part[((int64_t)I * (I + 1) / 2 + J) * 2 * CT + r];
-  for (int K = I + 1; K < nt; K++)
-    acc += part[((int64_t)K * (K + 1) / 2 + I) * 2 * CT + CT + r];
-  rhs[bidx[i]] = T(acc);
+  for (int J = p; J < nt; J += CSUM) {
+    const int64_t t = J <= I ? (int64_t)I * (I + 1) / 2 + J : (int64_t)J * (J + 1) / 2 + I;
+    acc += part[t * 2 * CT + (J <= I ? 0 : CT) + r];
+  }
+  sh[p][r] = acc;
+  __syncthreads();
+  const int i = I * CT + r;
+  if (p || i >= n) return;
+  double v = 0.0;
+#pragma unroll
+  for (int q = 0; q < CSUM; q++) v += sh[q][r];
+  rhs[bidx[i]] = T(v);
 }
 
 template <class T>
-__global__ __launch_bounds__(256) void k_cap_symv_sum(int n, int nt,
-                                                      const double* __restrict__ part,
-                                                      const int* __restrict__ bidx,
-                                                      T* __restrict__ rhs) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) cap_symv_sum_at<T>(n, nt, part, bidx, rhs, i);
-}
-
-// x = y at the unknowns
-template <class T>
-__global__ __launch_bounds__(256) void k_cap_out(int64_t n, const int8_t* __restrict__ mw,
-                                                 const T* __restrict__ y, T* __restrict__ x) {
-  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (k < n && mw[k]) x[k] = y[k];
+__global__ __launch_bounds__(CSUM* CT) void k_cap_symv_sum(int n, int nt,
+                                                          const double* __restrict__ part,
+                                                          const int* __restrict__ bidx,
+                                                          T* __restrict__ rhs) {
+  cap_symv_sum_tile<T>(n, nt, part, bidx, rhs, (int)blockIdx.x);
 }
 
 // x64 = x0 + e at the unknowns (x0 NULL: 0; x0 may be x64 itself)
@@ -346,10 +348,10 @@ __global__ __launch_bounds__(256) void k_cap_symv_b(const CapMember* __restrict_
   cap_symv_tile<float>(m.M, m.n, m.bidx, m.y, m.part, (int)blockIdx.x);
 }
 
-__global__ __launch_bounds__(256) void k_cap_symv_sum_b(const CapMember* __restrict__ t) {
+__global__ __launch_bounds__(CSUM* CT) void k_cap_symv_sum_b(const CapMember* __restrict__ t) {
   const CapMember& m = t[blockIdx.y];
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < m.n) cap_symv_sum_at<float>(m.n, m.nt, m.part, m.bidx, m.rhs, i);
+  if ((int)blockIdx.x >= m.nt) return;
+  cap_symv_sum_tile<float>(m.n, m.nt, m.part, m.bidx, m.rhs, (int)blockIdx.x);
 }
 
 // x64 = x0 + y at the unknowns (from as in k_cap_res_b)
@@ -657,8 +659,7 @@ template <class T>
 static void gemv(CapSolver* c, hipStream_t s) {
   k_cap_symv<T><<<c->ntl, 256, 0, s>>>((const T*)c->M, c->n, c->bidx, (const T*)c->y,
                                        c->tpart);
-  k_cap_symv_sum<T><<<blocks(c->n), 256, 0, s>>>(c->n, c->nt, c->tpart, c->bidx,
-                                                  (T*)c->rhs);
+  k_cap_symv_sum<T><<<c->nt, CSUM * CT, 0, s>>>(c->n, c->nt, c->tpart, c->bidx, (T*)c->rhs);
 }
 
 template <class TB, class TX>
@@ -695,14 +696,17 @@ template void cap_solve_modal(CapSolver*, const float*, int, float*, bool, doubl
 void cap_solve_f64(CapSolver* c, const double* b, int gmode, double* x, bool measure,
                    double* stats, hipStream_t s) {
   F2D_REQUIRE(c->f64 && !c->modal, "capacitance solver built for FP32");
-  const int64_t N = (int64_t)c->g.NYP * c->g.NXP;
   double* rhs = (double*)c->rhs;
   double* y = (double*)c->y;
-  k_cap_rhs<double, double><<<blocks(N), 256, 0, s>>>(c->g, b, gmode, c->mw, rhs);
-  fft_solve_f64(c->fft, rhs, 0, y, 0.0, false, nullptr, s);
+  // the first spectral solve reads b at W and leaves b_W in rhs, the second
+  // writes its result to x at W (no passes of their own, 4 us each at 512^2)
+  FftMask m1, m2;
+  m1.in = c->mw;
+  m1.out = rhs;
+  m2.res = c->mw;
+  fft_solve_f64_masked(c->fft, b, gmode, y, m1, s);
   gemv<double>(c, s);
-  fft_solve_f64(c->fft, rhs, 0, y, 0.0, false, nullptr, s);
-  k_cap_out<double><<<blocks(N), 256, 0, s>>>(N, c->mw, y, x);
+  fft_solve_f64_masked(c->fft, rhs, 0, x, m2, s);
   if (measure && stats) measure_res<double, double>(c, b, gmode, x, 1, stats, s);
   c->solved = true;
 }
@@ -782,7 +786,7 @@ struct CapBatch {
   FftBatchPtrs* fa = nullptr;  // plain solves: b (masked, kept in rhs) -> y
   FftBatchPtrs* fb = nullptr;  // plain solves: rhs -> x at the unknowns
   FftBatchPtrs* fr = nullptr;  // one warm refinement: residual of x (kept in rhs) -> y
-  int maxntl = 0, maxn = 0;
+  int maxntl = 0, maxnt = 0;
 };
 
 static bool same_geo(const CapGeo& a, const CapGeo& b) {
@@ -817,7 +821,7 @@ CapBatch* cap_batch_create(CapSolver* const* c, int nm, const float* const* b,
       fr[i] = fa[i];
       fr[i].m.xr = x[i];
       if (m->ntl > bt->maxntl) bt->maxntl = m->ntl;
-      if (m->n > bt->maxn) bt->maxn = m->n;
+      if (m->nt > bt->maxnt) bt->maxnt = m->nt;
     }
     F2D_HIP(hipMalloc(&bt->t, sizeof(CapMember) * nm));
     F2D_HIP(hipMalloc(&bt->ft, sizeof(FftBatchPtrs) * nm));
@@ -860,7 +864,7 @@ void cap_batch_solve(CapBatch* bt, int nref, bool warm, hipStream_t s) {
   if (nref == 0) {  // plain FP32 solves (cap_solve_f32 with nref 0)
     fft_solve_f32_batch(bt->c[0]->fft, nm, bt->fa, s);
     k_cap_symv_b<<<dim3((unsigned)bt->maxntl, (unsigned)nm), 256, 0, s>>>(bt->t);
-    k_cap_symv_sum_b<<<dim3(blocks(bt->maxn), (unsigned)nm), 256, 0, s>>>(bt->t);
+    k_cap_symv_sum_b<<<dim3((unsigned)bt->maxnt, (unsigned)nm), CSUM * CT, 0, s>>>(bt->t);
     fft_solve_f32_batch(bt->c[0]->fft, nm, bt->fb, s);
     for (CapSolver* m : bt->c) m->solved = true;
     return;
@@ -877,7 +881,7 @@ void cap_batch_solve(CapBatch* bt, int nref, bool warm, hipStream_t s) {
   if (from_x && nref == 1) {  // cap_solve_f32's fused warm refinement
     fft_solve_f32_batch(bt->c[0]->fft, nm, bt->fr, s);
     k_cap_symv_b<<<dim3((unsigned)bt->maxntl, (unsigned)nm), 256, 0, s>>>(bt->t);
-    k_cap_symv_sum_b<<<dim3(blocks(bt->maxn), (unsigned)nm), 256, 0, s>>>(bt->t);
+    k_cap_symv_sum_b<<<dim3((unsigned)bt->maxnt, (unsigned)nm), CSUM * CT, 0, s>>>(bt->t);
     fft_solve_f32_batch(bt->c[0]->fft, nm, bt->fb, s, true);
     for (CapSolver* m : bt->c) m->solved = true;
     return;
@@ -889,7 +893,7 @@ void cap_batch_solve(CapBatch* bt, int nref, bool warm, hipStream_t s) {
     k_cap_res_b<<<gp, 256, 0, s>>>(g, bt->t, from);
     fft_solve_f32_batch(bt->c[0]->fft, nm, bt->ft, s);
     k_cap_symv_b<<<dim3((unsigned)bt->maxntl, (unsigned)nm), 256, 0, s>>>(bt->t);
-    k_cap_symv_sum_b<<<dim3(blocks(bt->maxn), (unsigned)nm), 256, 0, s>>>(bt->t);
+    k_cap_symv_sum_b<<<dim3((unsigned)bt->maxnt, (unsigned)nm), CSUM * CT, 0, s>>>(bt->t);
     fft_solve_f32_batch(bt->c[0]->fft, nm, bt->ft, s);
     k_cap_acc_b<<<gp, 256, 0, s>>>(N, bt->t, from);
   }

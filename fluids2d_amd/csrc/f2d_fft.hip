@@ -1603,37 +1603,53 @@ void fft_solve_f32_batch(FftSolver* f, int nm, const FftBatchPtrs* table, hipStr
     inv(std::integral_constant<int, 0>());
 }
 
-void fft_solve_f32_masked(FftSolver* f, const float* b, int gmode, float* x, const FftMask& m,
-                          hipStream_t s, bool acc) {
-  F2D_REQUIRE(f->S32, "FFT solver built without FP32 buffers");
+// (acc: FP32 only)
+template <class T>
+static void solve_masked(FftSolver* f, const T* b, int gmode, T* x, const FftMask& m,
+                         hipStream_t s, bool acc) {
   F2D_REQUIRE(!m.in || m.out, "a masked right-hand side needs its output array");
   FftArgs a = f->a;
-  const FftPlan& p = f->p32;
+  constexpr bool d = sizeof(T) == 8;
+  const FftPlan& p = d ? f->p64 : f->p32;
   a.P = p.P;
   a.Q = p.Q;
   a.real0 = p.lgc > 0;
+  cplx<T>* S = d ? (cplx<T>*)f->S64 : (cplx<T>*)f->S32;
+  const cplx<T>* twx = d ? (const cplx<T>*)f->twx64 : (const cplx<T>*)f->twx32;
+  const cplx<T>* twy = d ? (const cplx<T>*)f->twy64 : (const cplx<T>*)f->twy32;
   const int gr = (a.ey ? a.ony : a.ny) / (2 * a.P), gc = (a.ncu + a.Q - 1) / a.Q;
   FftMask mf = m, mi = m;
   mf.res = nullptr;
   mi.in = nullptr;
   mi.out = nullptr;
   mi.xr = nullptr;
-  F2D_REQUIRE(!acc || mi.res, "an accumulating masked solve needs its mask");
+  F2D_REQUIRE(!acc || (mi.res && !d), "an accumulating masked solve: FP32, with its mask");
   const FftBatchPtrs* none = nullptr;
   const double* nod = nullptr;
-  rows_fwd<float, float>(p, dim3(gr), s, a, b, gmode, (float2*)f->S32, (const float2*)f->twx32,
-                         (double*)nullptr, nod, nod, gr, (const float*)nullptr, mf, none);
-  cols<float>(p, dim3(gc), s, a, (float2*)f->S32, (const float2*)f->twy32,
-              (const double*)f->lamx, (const double*)f->lamy, none);
-  auto inv = [&](auto mode) {
-    rows_inv<float, float, decltype(mode)::value>(
-        p, dim3(gr), s, a, (const float2*)f->S32, (const float2*)f->twx32, x, (double*)nullptr,
-        nod, (double*)nullptr, mi, none);
-  };
-  if (acc)
-    inv(std::integral_constant<int, 3>());
-  else
-    inv(std::integral_constant<int, 0>());
+  rows_fwd<T, T>(p, dim3(gr), s, a, b, gmode, S, twx, (double*)nullptr, nod, nod, gr,
+                 (const float*)nullptr, mf, none);
+  cols<T>(p, dim3(gc), s, a, S, twy, (const double*)f->lamx, (const double*)f->lamy, none);
+  if constexpr (!d) {
+    if (acc) {
+      rows_inv<T, T, 3>(p, dim3(gr), s, a, (const cplx<T>*)S, twx, x, (double*)nullptr, nod,
+                        (double*)nullptr, mi, none);
+      return;
+    }
+  }
+  rows_inv<T, T, 0>(p, dim3(gr), s, a, (const cplx<T>*)S, twx, x, (double*)nullptr, nod,
+                    (double*)nullptr, mi, none);
+}
+
+void fft_solve_f32_masked(FftSolver* f, const float* b, int gmode, float* x, const FftMask& m,
+                          hipStream_t s, bool acc) {
+  F2D_REQUIRE(f->S32, "FFT solver built without FP32 buffers");
+  solve_masked<float>(f, b, gmode, x, m, s, acc);
+}
+
+void fft_solve_f64_masked(FftSolver* f, const double* b, int gmode, double* x, const FftMask& m,
+                          hipStream_t s) {
+  F2D_REQUIRE(f->S64, "FFT solver built without FP64 buffers");
+  solve_masked<double>(f, b, gmode, x, m, s, false);
 }
 
 // whether two plans solve the same operator (same args and eigenvalues)

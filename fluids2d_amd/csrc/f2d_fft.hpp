@@ -81,9 +81,12 @@ struct FftBatchPtrs {
 // acc: the inverse row pass adds its result to x in FP64 (x = (float)(x + e))
 void fft_solve_f32_batch(FftSolver* f, int nm, const FftBatchPtrs* table, hipStream_t s,
                          bool acc = false);
-// one plain FP32 spectral solve with masks (x = the result, gmode as b's)
+// one plain spectral solve with masks (x = the result, gmode as b's; m.xr:
+// FP32 solves)
 void fft_solve_f32_masked(FftSolver* f, const float* b, int gmode, float* x, const FftMask& m,
                           hipStream_t s, bool acc = false);
+void fft_solve_f64_masked(FftSolver* f, const double* b, int gmode, double* x, const FftMask& m,
+                          hipStream_t s);
 bool fft_same_plan(const FftSolver* f, const FftSolver* g);
 float2* fft_spectrum32(FftSolver* f);
 
