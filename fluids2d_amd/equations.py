@@ -169,10 +169,10 @@ class QG(_Base):
         """work = centerstovertices(pv - hb*qgcoef) - f (operators.py:186-190;
         hb = 0 on the device, so pv - 0 is pv bit for bit)."""
         m = self.mesh
-        op.centerstovertices(m, s.pv, s.work)
         if self.param.beta != 0:
-            # work + (-1 * f) is work - f exactly
-            op.addto_terms(s.work, [self._planetary(s.work)], [-1.0])
+            op.centerstovertices_minus(m, s.pv, self._planetary(s.work), s.work)
+        else:
+            op.centerstovertices(m, s.pv, s.work)
 
     def rhs(self, s, ds):
         m, p = self.mesh, self.param

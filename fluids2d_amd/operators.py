@@ -102,6 +102,14 @@ def centerstovertices(mesh, omega, vomega, addto=False):
          ptr(mesh.d_mskv), int(addto), stream_ptr())
 
 
+def centerstovertices_minus(mesh, omega, f, vomega):
+    """centerstovertices less the vertex field f (operators.py:186-190)"""
+    if f.numel() < vomega.numel():
+        raise ValueError("f must cover the padded grid")
+    call("f2d_c2v_minus", _dt(omega), mesh.grid_ref(), ptr(omega), ptr(f), ptr(vomega),
+         ptr(mesh.d_mskv), stream_ptr())
+
+
 def perpgrad(mesh, psi, U, contravariant=False, fill=False, dt_dev=None, cfl=0.0,
              dtmax=0.0, cfl_part=None):
     """operators.py:144-149 (+ fill, + the CFL step of model.py:84-87 into

@@ -188,6 +188,10 @@ int f2d_addto(int dtype, void* y, const void* x0, const void* x1, const void* x2
 /* centerstovertices, operators.py:126-133 (addto=0/1) */
 int f2d_c2v(int dtype, const f2d_grid* g, const void* c, void* v,
             const int8_t* mskv, int addto, void* stream);
+/* centerstovertices less a vertex field, operators.py:186-190 (the inversion's
+ * right-hand side): v = centerstovertices(c) * mskv - f over the padded array */
+int f2d_c2v_minus(int dtype, const f2d_grid* g, const void* c, const void* f, void* v,
+                  const int8_t* mskv, void* stream);
 /* perpgrad (+ fill), operators.py:144-149, equations.py:79-84.
  * If maxabs (device float64[2]) is not NULL it receives
  * (max|Ux|, max|Uy|) over the padded arrays. */
