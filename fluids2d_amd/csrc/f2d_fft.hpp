@@ -31,7 +31,7 @@ bool fft_applicable_cells(int64_t ny, int64_t nx, int xper, int yper, int64_t nw
 
 // the transforms of a row and of a column fit in a workgroup's LDS
 // (FP64: transformed sizes up to 2048, and 4096 in periodic directions;
-// FP32: up to 4096).  two_buffers: without the in-place 4096
+// FP32: up to 4096).  two_buffers: without the one-buffer 4096
 bool fft_fits(int64_t ny, int64_t nx, int xper, int yper, bool f64, bool two_buffers = false);
 
 // cells: the Neumann cell operator (even extensions), else the vertex
