@@ -484,8 +484,10 @@ __global__ __launch_bounds__(256) void k_transport(TransportArgs<T> a,
 // and per cell the arithmetic is that of k_transport.
 // Against bounds-tested tiles (k_transport, kept for interiors smaller than a
 // tile): 16 steps of rsw FP64 on 501 x 333 1416 -> 1347 us, 8 of eulerpsi FP64
-// on an 800 x 304 channel 1319 -> 1261 us.
-template <class T, int M, int TY, int TX, bool B = false>
+// on an 800 x 304 channel 1319 -> 1261 us.  (MOVED: an instantiation of its
+// own; with the move tested in the kernel for tiles that divide, four FP64
+// steps on 4096 x 4096 took 7.32 ms, not 6.95.)
+template <class T, int M, int TY, int TX, bool B, bool MOVED>
 __global__ __launch_bounds__(256) void k_transport_full(TransportArgs<T> a,
                                                         const TransportArgs<T>* tab) {
   if (B) a = tab[blockIdx.y];
@@ -508,7 +510,8 @@ __global__ __launch_bounds__(256) void k_transport_full(TransportArgs<T> a,
   const uint32_t P = (uint32_t)a.P;
   const int tile = tile_of((int)blockIdx.x - a.nhb, a.ntiles);
   const int by = tile / a.tiles_x, bx = tile - by * a.tiles_x;
-  const int j0 = 3 + min(by * TY, a.ny - TY), i0 = 3 + min(bx * TX, a.nx - TX);
+  const int j0 = 3 + (MOVED ? min(by * TY, a.ny - TY) : by * TY);
+  const int i0 = 3 + (MOVED ? min(bx * TX, a.nx - TX) : bx * TX);
   const int c = t & (TX - 1), r0 = t / TX;
   const uint32_t oc = (uint32_t)(j0 + r0) * P + (uint32_t)(i0 + c);  // cell (r0, c)
   constexpr uint32_t one = 1;
@@ -668,9 +671,12 @@ void launch_transport_tile(const TransportArgs<T>& a0, hipStream_t s) {
   auto shared = [&](const T* o) { return o && (o == a.ds0 || o == a.ds1 || o == a.q); };
   const bool whole = a.ny >= TY && a.nx >= TX && (exact || (!shared(a.dso) && !shared(a.qo))) &&
                      (int64_t)(a.ny + 6) * (int64_t)a.P < ((int64_t)1 << 31);
-  if (whole)
-    launch_rec(k_transport_full<T, M, TY, TX, false>, k_transport_full<T, M, TY, TX, true>,
-               dim3(nb), dim3(256), 0, s, a);
+  if (whole && exact)
+    launch_rec(k_transport_full<T, M, TY, TX, false, false>,
+               k_transport_full<T, M, TY, TX, true, false>, dim3(nb), dim3(256), 0, s, a);
+  else if (whole)
+    launch_rec(k_transport_full<T, M, TY, TX, false, true>,
+               k_transport_full<T, M, TY, TX, true, true>, dim3(nb), dim3(256), 0, s, a);
   else
     launch_rec(k_transport<T, M, TY, TX, false>, k_transport<T, M, TY, TX, true>, dim3(nb),
                dim3(256), 0, s, a);
