@@ -27,10 +27,9 @@
 #include <vector>
 
 #include "f2d_modal.hpp"
+#include "f2d_modal_plan.hpp"
 
 namespace f2d {
-
-enum { BC_RING = 0, BC_WALL = 1, BC_EVEN = 2 };
 
 typedef double d2 __attribute__((ext_vector_type(2)));
 typedef double d4 __attribute__((ext_vector_type(4)));
@@ -42,7 +41,7 @@ struct ModalPass {
   void* out;
   int64_t ldi, ldo;
   int M;               // rows of the input
-  int K, LJ;           // padded contraction length (multiple of 32), pitch of mat
+  int K, LJ;           // padded contraction length, pitch of mat (ModalSizes)
   int nk;              // contraction pairs (forward: mirror pairs; back: modes)
   int npts, refl;      // forward: points of the direction, mirror of p is refl - p
   int ne, no;          // even and odd modes
@@ -432,14 +431,9 @@ __global__ __launch_bounds__(256) void k_modal_stats(const double* __restrict__ 
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-struct ModalDir {  // one direction
-  int bc = 0, n = 0;           // kind, cells
-  int pts = 0, refl = 0, nh = 0;  // unknowns, mirror constant, mirror pairs
-  int ne = 0, no = 0;
-  int cpts = 0, crefl = 0, cnh = 0;  // the same for a cell field
-  int KF = 0, LF = 0, KB = 0, LB = 0, KC = 0;
+struct ModalDir : ModalSizes {  // one direction
   d2 *fwd = nullptr, *back = nullptr, *cell = nullptr;
-  double* lam = nullptr;       // even modes, then odd modes
+  double* lam = nullptr;  // even modes, then odd modes
 };
 
 struct ModalSolver {
@@ -466,24 +460,8 @@ static P* malloc_dev(ModalSolver* m, size_t bytes) {
   return reinterpret_cast<P*>(p);
 }
 
-static int up32(int v) { return (v + 31) / 32 * 32; }
-
 static void dir_create(ModalSolver* m, ModalDir& d, int bc, int n, double c, double md) {
-  d.bc = bc;
-  d.n = n;
-  d.pts = bc == BC_WALL ? n - 1 : n;
-  d.refl = bc == BC_WALL ? n - 2 : (bc == BC_EVEN ? n - 1 : n);
-  d.nh = bc == BC_RING ? n / 2 + 1 : (d.pts + 1) / 2;
-  d.ne = bc == BC_WALL ? n / 2 : (bc == BC_RING ? n / 2 + 1 : (n + 1) / 2);
-  d.no = d.pts - d.ne;
-  d.cpts = n;
-  d.crefl = n - 1;
-  d.cnh = (n + 1) / 2;
-  d.KF = up32(d.nh);
-  d.LF = up32(d.ne);
-  d.KB = up32(d.ne);
-  d.LB = up32(d.nh);
-  d.KC = up32(d.cnh);
+  static_cast<ModalSizes&>(d) = modal_sizes(bc, n);
   const long double pi = 3.14159265358979323846264338327950288L;
   std::vector<double> t(4 * (size_t)n), lam(d.pts);
   for (int j = 0; j < 4 * n; j++) t[j] = (double)cosl(pi * j / (2.0L * n));
@@ -551,31 +529,22 @@ void modal_destroy(ModalSolver* m) {
   delete m;
 }
 
-static int64_t tiles(const ModalPass& a, int bm, int bn) {
-  return (int64_t)((a.M + bm - 1) / bm) * ((a.nj + bn - 1) / bn);
-}
-
-template <int BM, int BN, int MT, int NT, int WK, int KC, int D, bool FOLD, int EPI, class TI,
-          class TO>
+template <int T, int MT, int NT, int WK, bool FOLD, int EPI, class TI, class TO>
 static void launch_tile(const ModalPass& a, hipStream_t s) {
-  const int64_t t = (tiles(a, BM, BN) + 7) / 8 * 8;
-  k_modal<BM, BN, MT, NT, WK, KC, D, FOLD, EPI, TI, TO><<<(unsigned)t, 256, 0, s>>>(a);
+  constexpr int B = MODAL_TILES[T].b, KC = MODAL_TILES[T].kc;
+  // the loads of whole tiles and chunks stay inside the matrix
+  F2D_REQUIRE(modal_up(a.nj, B) <= a.LJ && a.K % KC == 0, "tile does not fit the matrix");
+  const int64_t t = (modal_tiles(a.M, a.nj, B) + 7) / 8 * 8;
+  k_modal<B, B, MT, NT, WK, KC, 2, FOLD, EPI, TI, TO><<<(unsigned)t, 256, 0, s>>>(a);
 }
 
 template <bool FOLD, int EPI, class TI, class TO>
 static void launch_pass(const ModalPass& a, hipStream_t s) {
-  // Measured on closed n x n grids (us a solve): 64 x 64 tiles fill the chip
-  // from about 640 of them (3000 x 2000: 1129 against 1306 with 32 x 32;
-  // 1600^2, 325 tiles: 505 against 380), 32 x 32 from about 400 (1000^2, 512
-  // tiles: 119 against 150 with 16 x 16; 1000 x 600, 304 tiles: 97 against
-  // 87), below them 16 x 16 tiles whose four waves split the contraction
-  // (256^2: 19 against 29; 40^2: 13.5 against 15.2).
-  if (tiles(a, 64, 64) >= 640)
-    launch_tile<64, 64, 2, 2, 1, 8, 2, FOLD, EPI, TI, TO>(a, s);
-  else if (tiles(a, 32, 32) >= 400)
-    launch_tile<32, 32, 1, 1, 1, 16, 2, FOLD, EPI, TI, TO>(a, s);
-  else
-    launch_tile<16, 16, 1, 1, 4, 32, 2, FOLD, EPI, TI, TO>(a, s);
+  switch (modal_tile(a.M, a.nj)) {
+    case 0: launch_tile<0, 2, 2, 1, FOLD, EPI, TI, TO>(a, s); break;
+    case 1: launch_tile<1, 1, 1, 1, FOLD, EPI, TI, TO>(a, s); break;
+    default: launch_tile<2, 1, 1, 4, FOLD, EPI, TI, TO>(a, s);
+  }
 }
 
 template <class TB, class TX>
