@@ -125,6 +125,7 @@ class Poisson2D:
         # learned from the solves checked on the host, plus a margin
         self.est = None
         self.margin = 2
+        self.refine = -1  # set_refine's choice (-1: the handle's option)
         # solve calls made from the host (``calls``) and solves replayed by
         # captured HIP graphs that the library's own counter does not see
         # (direct solves enqueued without statistics count on the host)
@@ -266,9 +267,9 @@ class Poisson2D:
         host state only, so a captured graph keeps the choice each of its
         solves was made with."""
         v = -1 if nref is None else int(nref)
-        if getattr(self, "_refine", -1) != v:
+        if self.refine != v:
             _lib.call("f2d_poisson_set_refine", self._h, v)
-            self._refine = v
+            self.refine = v
 
     def _stats_host(self):
         buf = (ctypes.c_double * 8)()

@@ -365,23 +365,30 @@ class RKIntegrator:
         for k, e in enumerate(sols):
             e.check_worst(float(self._h_run[1 + k]))
 
+    # the parameters that a stage reads as it is launched, part of a captured
+    # step's key (with the sign of ``dt``, the value of a fixed one is on the
+    # device)
+    BAKED = ("model", "precision", "integrator", "cfl", "dtmax", "compflux", "vortexforce",
+             "innerproduct", "f0", "g", "H", "beta", "xperiodic", "yperiodic",
+             "poisson_refine")
+
     def _checked_step(self):
         """The captured host-checked step of the current buffers and
         parameters: (graph, state and alternate state after it, solvers).
         The next step's dt and the solvers' worst residuals go to pinned host
         memory by kernels of the graph."""
-        p, m = self.param, self.mesh
-        key = self._graph_key() + self.model.graph_operands(self.dstate) + (
-            p.cfl, p.dtmax, p.dt > 0, p.compflux, p.vortexforce, p.innerproduct, p.f0, p.g, p.H,
-            p.beta, getattr(p, "poisson_refine", "every"), m.grid.tile,
-            getattr(self.model, "fused", True), tuple(id(e) for e in self._solvers()))
+        m = self.mesh
+        sols = self._solvers()
+        key = self._graph_key() + self.model.graph_operands(self.dstate) + tuple(
+            getattr(self.param, n, None) for n in self.BAKED) + (
+            self._wants_dtn(), m.dx, m.dy, m.area, m.grid.tile,
+            getattr(self.model, "fused", True), tuple((id(e), e.refine) for e in sols))
         got = self._checked.get(key)
         if got is not None:
             return got
         if len(self._checked) >= 16:  # parameters that change as the run goes
             self._checked.clear()
         keep = (self.dstate, self.dalt, self._dtn_valid, self._dtn_part, self._dt_part)
-        sols = self._solvers()
         graph = torch.cuda.CUDAGraph()
         side = torch.cuda.Stream(m.device)
         side.wait_stream(torch.cuda.current_stream())

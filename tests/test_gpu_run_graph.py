@@ -112,3 +112,58 @@ def test_planetary_vorticity_rebound_between_steps(dev):
         m.run()
         out.append(m.state.pv.copy())
     assert np.array_equal(*out)
+
+
+@pytest.mark.parametrize("precision,change", [
+    ("fp64", lambda m: setattr(m.param, "integrator", "enrk3")),
+    ("fp64", lambda m: setattr(m.param, "compflux", "centered")),
+    ("fp32", lambda m: m.mesh.poisson_vertices.set_refine(0))])
+def test_changes_between_runs_reach_replayed_steps(dev, precision, change):
+    """What an eager stage reads at every call -- the integrator's
+    coefficients, the flux method, the refinements of a solve -- is not kept
+    from an earlier run's graph."""
+    out = []
+    for g in (True, False):
+        m = _start("eulerpsi", 64, 64, 0, precision, g, poisson_refine="every")
+        m.run()
+        before = m.state.omega.copy()
+        change(m)
+        m.time.ite0 = m.time.ite
+        m.run()
+        out.append(m.state.omega.copy())
+    assert np.array_equal(*out) and not np.array_equal(out[0], before)
+
+
+class _Reads:
+    """A Param that notes the names read from it."""
+
+    def __init__(self, param, names):
+        self.__dict__.update(_param=param, _names=names)
+
+    def __getattr__(self, name):
+        self._names.add(name)
+        return getattr(self._param, name)
+
+    def __setattr__(self, name, value):
+        setattr(self._param, name, value)
+
+
+@pytest.mark.parametrize("model,precision,kw", [
+    ("euler", "fp64", {}), ("eulerpsi", "fp64", {}), ("eulerpsi", "fp32", {}),
+    ("qg", "fp64", dict(beta=1.0)), ("qgrsw", "fp32", dict(dtmax=0.02)), ("rsw", "fp64", {}),
+    ("advection", "fp64", {})])
+def test_captured_steps_read_keyed_parameters_only(dev, model, precision, kw):
+    """Every parameter read while a step is captured is part of its key."""
+    m = _start(model, 64, 64, 0, precision, True, **kw)
+    m.run()
+    integ, names = m.integrator, set()
+    integ._checked.clear()
+    integ.begin(m.state)
+    integ.set_dt(m.time)
+    for o in (integ, integ.model, m.mesh):
+        o.param = _Reads(o.param, names)
+    if integ._wants_dtn():
+        integ._dtn_valid = True
+    names.clear()
+    assert integ._checked_step() is not None
+    assert "integrator" in names and names <= set(integ.BAKED) | {"dt"}, names
