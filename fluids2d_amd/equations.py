@@ -8,6 +8,8 @@ Each model class offers
     diagnostic fields (Poisson solve with the right-hand side formed inside
     the solver, perp-gradient + fill + next CFL step in one kernel).
 """
+import torch
+
 from . import _lib
 from . import operators as op
 from .elliptic import PoissonNotConverged  # noqa: F401  (re-export)
@@ -20,6 +22,17 @@ class _Base:
     def __init__(self, param, mesh):
         self.param = param
         self.mesh = mesh
+        # block maxima of the CFL step: the model's own, as captured steps
+        # hold the address (the library's scratch belongs to a stream, and
+        # other models share it)
+        self._npart = op.cfl_partials(mesh)  # perpgrad's
+        self._cfl_part = torch.empty(max(op.CFL_PARTS, self._npart), dtype=torch.float64,
+                                     device=mesh.device)
+
+    def _cfl_dt(self, U, dt_next):
+        """The CFL step of velocities U into dt_next (model.py:84-87)."""
+        p = self.param
+        op.cfl_dt(U, p.cfl, p.dtmax, dt_next, part=self._cfl_part)
 
     def materialize(self, s, names=None):
         """Fill the diagnostic fields the fused path does not store, before a
@@ -126,7 +139,7 @@ class Advection(_Base):
                            p.integrator, k, dt, dt_log if k == 0 else None)
         s, alt = s._replace(q=alt.q), alt._replace(q=s.q)
         if dt_next is not None:
-            op.cfl_dt(s.U, p.cfl, p.dtmax, dt_next)
+            self._cfl_dt(s.U, dt_next)
         return s, alt
 
 
@@ -153,7 +166,6 @@ class QG(_Base):
                                  "vorticity at the vertices, times the cell area)")
         if f is not self._f_src or self._f_dev is None or self._f_dev.dtype != like.dtype:
             import numpy as np
-            import torch
             if isinstance(f, torch.Tensor):
                 d = f.to(device=like.device, dtype=like.dtype)
             else:
@@ -205,8 +217,10 @@ class QG(_Base):
         else:
             m.qg_helmholtz.solve_c2v(s.pv, s.psi, stats=stats)
         if k == _lib.NSTAGES[p.integrator] - 1:
-            op.perpgrad(m, s.psi, s.U, contravariant=True, fill=False, dt_dev=dt_next,
-                        cfl=p.cfl, dtmax=p.dtmax)
+            part = None if dt_next is None else self._cfl_part[:self._npart]
+            op.perpgrad(m, s.psi, s.U, contravariant=True, fill=False, cfl_part=part)
+            if part is not None:
+                op.cfl_finish(part, dt_next, p.cfl, p.dtmax)
         return s, alt
 
     def materialize(self, s, names=None):

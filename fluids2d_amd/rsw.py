@@ -46,7 +46,6 @@ class _SW(_Base):
         super().__init__(param, mesh)
         self._ds_last = None
         self._pre = None
-        self._cflpart = None  # block maxima of stage_split's CFL step
         self._stats = True  # host-checked solves unless a stage says otherwise
 
     def _grid(self):
@@ -122,7 +121,7 @@ class _SW(_Base):
         if self.fused:
             s, alt = self._stage_fused(s, alt, ds_prev, ds_out, k, dt, stats, dt_log)
             if dt_next is not None:
-                op.cfl_dt(self.cfl_velocity(s), self.param.cfl, self.param.dtmax, dt_next)
+                self._cfl_dt(self.cfl_velocity(s), dt_next)
             return s, alt
         p = self.param
         if ds_out is None:
@@ -146,7 +145,7 @@ class _SW(_Base):
             op.rk_addto(y, [pv[n] for pv in prev] + [dsl[n]], p.integrator, k, dt)
         self.diag(s)
         if dt_next is not None:
-            op.cfl_dt(s.U, p.cfl, p.dtmax, dt_next)
+            self._cfl_dt(s.U, dt_next)
         return s, alt
 
 
@@ -276,17 +275,10 @@ class QGRSW(_SW):
         f2d_record_begin can record."""
         cfl = None
         if dt_next is not None:
-            if self._cflpart is None:
-                if _lib.capturing():
-                    raise RuntimeError("stage_split: CFL array not allocated before a capture")
-                self._cflpart = torch.zeros(op.CFL_PARTS, dtype=torch.float64,
-                                            device=s.h.device)
-            part = self._cflpart
-
             def cfl():
-                # its own block-maxima array: recordable into a member batch
-                op.cfl_dt(self.cfl_velocity(s), self.param.cfl, self.param.dtmax, dt_next,
-                          part=part)
+                # the model's own block-maxima array: recordable into a
+                # member batch
+                self._cfl_dt(self.cfl_velocity(s), dt_next)
         return ((lambda: self._stage_pre(s, k, dt, dt_log)),
                 (lambda: self._stage_post(s, ds_prev, ds_out, k, dt)), cfl)
 
@@ -421,7 +413,7 @@ class Euler(_SW):
         finally:
             self._stats = True
         if dt_next is not None:
-            op.cfl_dt(s.U, p.cfl, p.dtmax, dt_next)
+            self._cfl_dt(s.U, dt_next)
         return s, alt
 
 

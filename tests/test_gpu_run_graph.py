@@ -167,3 +167,58 @@ def test_captured_steps_read_keyed_parameters_only(dev, model, precision, kw):
     names.clear()
     assert integ._checked_step() is not None
     assert "integrator" in names and names <= set(integ.BAKED) | {"dt"}, names
+
+
+@pytest.mark.parametrize("model,kw", [("qg", dict(beta=1.0)), ("euler", {}), ("advection", {}),
+                                      ("qgrsw", dict(dtmax=0.02)), ("eulerpsi", {})])
+def test_captured_steps_own_their_reductions(dev, monkeypatch, model, kw):
+    """A captured step (of a run, or of device_steps) forms the CFL step in
+    arrays of its model, not in the library's scratch of the stream it was
+    captured on: that is another stream's, or another model's to grow."""
+    from fluids2d_amd import _lib, operators
+    made = []
+    plain = _lib.call
+
+    def call(name, *args):
+        if torch.cuda.is_current_stream_capturing():
+            made.append((name, args))
+        return plain(name, *args)
+    monkeypatch.setattr(_lib, "call", call)
+    monkeypatch.setattr(operators, "call", call)
+    m = _start(model, 64, 64, 0, "fp64", True, **kw)
+    m.run()
+    m.integrator.begin(m.state)
+    m.integrator.device_steps(12)
+    assert m.integrator._checked and m.integrator.graph_count()
+    assert any(n.startswith(("f2d_cfl", "f2d_perpgrad_part")) for n, _ in made)
+    for name, args in made:
+        assert name != "f2d_cfl_dt"
+        assert name != "f2d_perpgrad_ex" or args[10:12] == (None, None)
+
+
+def test_captured_step_outlives_larger_reductions(dev):
+    """The library's reduction scratch grows (its old allocation freed) for a
+    grid of more blocks than the smallest allocation holds, between two runs
+    of a captured model."""
+    from fluids2d_amd import _lib
+    n = 2920  # 4 points a thread of 256: 8360 blocks, 8192 is the smallest
+    out = []
+    for g in (True, False):
+        m = _start("qg", 64, 64, 0, "fp64", g, beta=1.0)
+        m.run()
+        if g:
+            assert m.integrator._checked
+            param = type(m.param)()
+            param.nx = param.ny = n
+            grid = _lib.make_grid(param)
+            a = [torch.zeros(n + 6, n + 6, dtype=torch.float32, device=dev) for _ in range(3)]
+            msk = torch.ones(n + 6, n + 6, dtype=torch.int8, device=dev)
+            dt = torch.zeros(1, dtype=torch.float64, device=dev)
+            _lib.call("f2d_perpgrad_ex", _lib.F32, grid, *map(_lib.ptr, a), _lib.ptr(msk),
+                      _lib.ptr(msk), 1.0, 1.0, 0, None, _lib.ptr(dt), 0.5, 2.0,
+                      _lib.stream_ptr())
+            assert float(dt) == 2.0
+        m.time.ite0 = m.time.ite
+        m.run()
+        out.append(m.state.pv.copy())
+    assert np.array_equal(*out)
