@@ -67,11 +67,10 @@ class RKIntegrator:
         self._h_dt = torch.zeros(1, dtype=torch.float64).pin_memory()
         # run loop (device_step): captured host-checked steps, the pinned
         # array they leave the next dt [0] and the solvers' worst residuals
-        # in, the solvers of the step whose residuals are to be checked
+        # in, whether that dt is still the next step's
         self._checked = {}
         self._h_run = torch.zeros(4, dtype=torch.float64).pin_memory()
         self._dt_on_host = False
-        self._unchecked = ()
         self._run_steps, self._run_mesh = 0, None
         self._no_replay = False
         self._dtn_valid = False
@@ -137,7 +136,6 @@ class RKIntegrator:
         return [a for n in self.specs.prognostic for a in leaves(getattr(s, n))]
 
     def _host_rhs(self, s, ds):
-        self._check_step()
         upload(s, self.dstate)
         dds = self.dscratch[0]
         self.model.rhs(self.dstate, dds)
@@ -146,12 +144,11 @@ class RKIntegrator:
             download(self.dstate, s, names=["flx"])
 
     def _host_diag(self, s):
-        self._check_step()
         upload(s, self.dstate)
         self.model.diag(self.dstate)
         self.model.materialize(self.dstate)
         download(self.dstate, s)
-        self._dtn_valid = self._dtn_part = self._dt_part = False
+        self._dtn_valid = self._dtn_part = self._dt_part = self._dt_on_host = False
 
     def step(self, state, time):
         """RKIntegrator.step (integrators.py:76-79): one step of time.dt on
@@ -165,13 +162,11 @@ class RKIntegrator:
     # -- device path --------------------------------------------------------------
     def begin(self, state):
         """Host state -> device twin."""
-        self._check_step()
         upload(state, self.dstate)
-        self._dtn_valid = self._dtn_part = self._dt_part = False
+        self._dtn_valid = self._dtn_part = self._dt_part = self._dt_on_host = False
 
     def end(self, state, names=None):
         """Device twin -> host state."""
-        self._check_step()
         self.model.materialize(self.dstate, names)
         download(self.dstate, state, names)
 
@@ -179,7 +174,6 @@ class RKIntegrator:
         """Model.set_dt (model.py:71-87): dt on the device and on the host."""
         p = self.param
         if p.dt > 0:
-            self._check_step()
             time.dt = p.dt
             self._write_dt(p.dt)
             return
@@ -198,7 +192,7 @@ class RKIntegrator:
         self._dtn_part = self._dt_part = False
         self.d_dt, self.d_dtn = self.d_dtn, self.d_dt
         if self._dt_on_host:  # left there by the step's graph
-            self._check_step()
+            self._dt_on_host = False
             time.dt = float(self._h_run[0])
             return
         self._h_dt.copy_(self.d_dt, non_blocking=True)
@@ -238,7 +232,6 @@ class RKIntegrator:
         """Names of the prognostic fields of the device state with a
         non-finite value on a wet cell (one flag per field, read on the host:
         a synchronisation point)."""
-        self._check_step()
         names = [n for n in self.specs.prognostic]
         flags = torch.zeros(len(names), dtype=torch.int32, device=self.d_dt.device)
         m = self.mesh
@@ -256,7 +249,7 @@ class RKIntegrator:
     def advance(self, stats=True, dt_log=None):
         """One RK step on the device with the dt already in d_dt; dt_log (a
         one-element float64 device tensor) receives that dt."""
-        self._check_step()
+        self._dt_on_host = False
         s, alt = self.dstate, self.dalt
         dtn = self.d_dtn if self._wants_dtn() else None
         if self.forcings:
@@ -305,7 +298,7 @@ class RKIntegrator:
         stage).  Running pre, the solve, post, cfl for k = 0, 1, ... is the
         step.  The dt is the one in d_dt now (call after _select_dt)."""
         assert not self.forcings and hasattr(self.model, "stage_split")
-        self._check_step()
+        self._dt_on_host = False
         self._dt_ready()
         if dt_log is not None and not getattr(self.model, "logs_dt", False):
             self._log_dt(dt_log)
@@ -327,23 +320,26 @@ class RKIntegrator:
     def device_step(self, time):
         """One host-checked step (Model.run's): with direct solvers and
         ``param.hipgraph``, after two eager steps, the replay of a captured
-        step whose solves leave their measured residuals on the device.
-        They are checked -- the same test, the same exception -- where the
-        loop next waits for the device: at set_dt or end."""
-        self._check_step()
+        step whose solves leave their measured residuals on the device and
+        then in pinned memory, with the next dt.  They are waited for here:
+        a replayed step's solves are checked as an eager step's are, before
+        the time goes forward."""
         g = self._checked_step() if self._can_replay() else None
         if g is None:
             self.advance()
             self._run_steps += 1
         else:
-            graph, (self.dstate, self.dalt), sols = g[:3]
+            graph, after, sols = g[:3]
+            dtn = self._wants_dtn()
             graph.replay()
-            self._dtn_valid = self._wants_dtn()
-            self._dt_part = self._dtn_part = False
-            self._dt_on_host = self._dtn_valid
-            self._unchecked = sols
-            for e in sols:
+            if sols or dtn:
+                torch.cuda.current_stream().synchronize()
+            for k, e in enumerate(sols):
                 e.calls += self.nstages
+                e.check_worst(float(self._h_run[1 + k]))
+            self.dstate, self.dalt = after
+            self._dtn_valid = self._dt_on_host = dtn
+            self._dt_part = self._dtn_part = False
         time.pushforward()
 
     def _can_replay(self):
@@ -355,15 +351,6 @@ class RKIntegrator:
                 and getattr(self.model, "capturable", True)
                 and getattr(self.model, "events", None) is None
                 and all(e.method in DIRECT for e in self._solvers()))
-
-    def _check_step(self):
-        """Wait for the last replayed step and check its solves."""
-        if not (self._dt_on_host or self._unchecked):
-            return
-        torch.cuda.current_stream().synchronize()
-        sols, self._unchecked, self._dt_on_host = self._unchecked, (), False
-        for k, e in enumerate(sols):
-            e.check_worst(float(self._h_run[1 + k]))
 
     # the parameters that a stage reads as it is launched, part of a captured
     # step's key (with the sign of ``dt``, the value of a fixed one is on the
@@ -433,8 +420,7 @@ class RKIntegrator:
         pending as block maxima stays so, and the step's first stage forms
         it."""
         p = self.param
-        self._check_step()
-        self._dt_part = False
+        self._dt_part = self._dt_on_host = False
         if p.dt > 0:
             self._write_dt(p.dt)
         elif p.model == "rsw":
@@ -459,6 +445,7 @@ class RKIntegrator:
         ``graph_steps`` steps are captured once into a HIP graph and
         replayed; the launches are the eager ones, so results are
         identical."""
+        self._dt_on_host = False
         dts = torch.zeros(nsteps, dtype=torch.float64, device=self.d_dt.device)
         use = getattr(self.param, "hipgraph", True) if graph is None else graph
         use = use and not stats and getattr(self.model, "capturable", True) \

@@ -222,3 +222,45 @@ def test_captured_step_outlives_larger_reductions(dev):
         m.run()
         out.append(m.state.pv.copy())
     assert np.array_equal(*out)
+
+
+@pytest.mark.parametrize("graph", [True, False])
+def test_rejected_step_is_not_pushed_forward(dev, monkeypatch, graph):
+    """The exception of a solve that is not accepted comes from its own step:
+    the time stays where it was and no diagnostic sees the step."""
+    from fluids2d_amd.elliptic import PoissonNotConverged
+    m = _start("eulerpsi", 64, 64, 0, "fp64", graph)
+    m.run()
+    seen = []
+    diag = lambda: seen.append(m.time.ite)  # noqa: E731
+    diag.device, diag.finalize = True, lambda: None
+    m.diags.append(diag)
+    monkeypatch.setattr(type(m.mesh.poisson_vertices), "_accepted", lambda self, r: r <= 1e-30)
+    m.time.ite0 = ite = m.time.ite
+    t = m.time.t
+    with pytest.raises(PoissonNotConverged):
+        m.run()
+    assert m.time.ite == ite and m.time.t == t and not seen
+
+
+def test_resident_steps_after_replayed_ones(dev):
+    """device_steps may capture its own graph right after a replayed
+    device_step."""
+    out = []
+    for g in (True, False):
+        m = _start("eulerpsi", 64, 64, 0, "fp64", g)
+        integ = m.integrator
+        integ.begin(m.state)
+        dts = []
+        for n in (16, 3, 8, 1, 8):
+            if n % 8:
+                for _ in range(n):
+                    integ.set_dt(m.time)
+                    integ.device_step(m.time)
+                    dts.append(m.time.dt)
+            else:
+                dts += integ.device_steps(n).cpu().tolist()
+        integ.end(m.state)
+        out.append((m.state.omega.copy(), dts))
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
+
