@@ -289,10 +289,8 @@ __global__ __launch_bounds__(256) void k_cap_norms(CapGeo g, const TB* __restric
 // one block: relative residual into the solve statistics
 // [iterations, relres, converged, refinements | failed, max, solves]
 // (a direct solve is accepted unless its residual is above 1e-6 or not finite)
-// nan_fails: a norm that is not a number is reported (as multigrid does)
 __global__ __launch_bounds__(256) void k_cap_stats(const double* __restrict__ part, int nb,
-                                                   int passes, int nan_fails,
-                                                   double* __restrict__ st) {
+                                                   int passes, double* __restrict__ st) {
   __shared__ double sh[4];
   double a = 0.0, c = 0.0;
   for (int i = threadIdx.x; i < nb; i += 256) {
@@ -303,7 +301,7 @@ __global__ __launch_bounds__(256) void k_cap_stats(const double* __restrict__ pa
   c = bsum(c, sh);
   if (threadIdx.x != 0) return;
   double rel = c > 0.0 ? sqrt(a / c) : 0.0;
-  if (nan_fails && !(a - a == 0.0 && c - c == 0.0)) rel = NAN;
+  if (!(a - a == 0.0 && c - c == 0.0)) rel = NAN;
   const double conv = (rel <= 1e-6) ? 1.0 : 0.0;
   st[0] = (double)passes;
   st[1] = rel;
@@ -666,7 +664,7 @@ template <class TB, class TX>
 static void measure_res(CapSolver* c, const TB* b, int gmode, const TX* x, int passes,
                         double* stats, hipStream_t s) {
   k_cap_norms<TB, TX><<<c->nbres, 256, 0, s>>>(c->g, b, gmode, c->mw, x, c->part);
-  k_cap_stats<<<1, 256, 0, s>>>(c->part, c->nbres, passes, c->modal != nullptr, stats);
+  k_cap_stats<<<1, 256, 0, s>>>(c->part, c->nbres, passes, stats);
 }
 
 template <class T>

@@ -1140,8 +1140,11 @@ __global__ __launch_bounds__(256) void k_fft_stats(const double* __restrict__ pa
       rr -= v[1] * v[1] / n;
       bb -= v[3] * v[3] / n;
     }
-    rr = rr > 0.0 ? rr : 0.0;
-    rel = bb > 0.0 ? sqrt(rr / bb) : 0.0;
+    // (a norm that is not finite is reported as NaN)
+    if (!(rr - rr == 0.0 && bb - bb == 0.0))
+      rel = NAN;
+    else
+      rel = bb > 0.0 && rr > 0.0 ? sqrt(rr / bb) : 0.0;
     // a direct solve is exact up to rounding: its true residual sits at
     // eps times the condition number (about 1e-11 at 1024^2 in FP64), so
     // rtol is not its acceptance test; it is accepted unless the residual

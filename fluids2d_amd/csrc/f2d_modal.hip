@@ -416,8 +416,8 @@ __global__ __launch_bounds__(256) void k_modal_stats(const double* __restrict__ 
   if (threadIdx.x != 0) return;
   double rr = v[0];
   if (singular) rr -= v[1] * v[1] / n;
-  rr = rr > 0.0 ? rr : (rr == rr ? 0.0 : rr);
-  const double rel = v[2] > 0.0 ? sqrt(rr / v[2]) : (rr == rr && v[2] == v[2] ? 0.0 : NAN);
+  const bool finite = rr - rr == 0.0 && v[2] - v[2] == 0.0;
+  const double rel = !finite ? NAN : (v[2] > 0.0 && rr > 0.0 ? sqrt(rr / v[2]) : 0.0);
   const double conv = rel <= 1e-6 ? 1.0 : 0.0;
   st[0] = 1.0;
   st[1] = rel;

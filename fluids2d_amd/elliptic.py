@@ -192,6 +192,10 @@ class Poisson2D:
         return None
 
     def _accepted(self, relres):
+        if relres != relres and self.method in ("fft", "capacitance"):
+            # the state is not finite: a run goes on to its own check for
+            # that, which stops it cleanly (Model._check_finite)
+            return True
         if self.method in DIRECT:
             # direct: exact up to rounding.  FP32 transforms refined once from
             # the previous solution: the FP64 residual of FP32 rounding at

@@ -537,7 +537,8 @@ int f2d_poisson_solve_c2v(f2d_poisson* h, const void* omega, void* x,
  * [4] number of solves that did not converge, [5] maximum iterations
  * (F32_REFINE: refinements), [6] number of solves,
  * [7] the largest relative residual a direct solve measured (NaN once one
- * was NaN).  Without iters/relres a
+ * was NaN).  A direct solve whose norms are not finite (NaN or infinity in b)
+ * reports NaN and counts as not converged.  Without iters/relres a
  * solve enqueues exactly `maxit` iterations (refinements), those after
  * convergence returning at once, and never synchronises: these counters are
  * how a caller checks such solves afterwards. */
