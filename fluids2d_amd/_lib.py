@@ -26,7 +26,7 @@ EXPORTS = [
     "f2d_poisson_create", "f2d_poisson_destroy", "f2d_poisson_solve",
     "f2d_poisson_solve_c2v", "f2d_poisson_stats", "f2d_poisson_reset_stats",
     "f2d_poisson_bench_kernel", "f2d_perpgrad_ex", "f2d_poisson_read_stats",
-    "f2d_poisson_method", "f2d_poisson_measure", "f2d_coriolis", "f2d_addgrad", "f2d_sharp", "f2d_vorticity",
+    "f2d_poisson_method", "f2d_poisson_accept", "f2d_poisson_measure", "f2d_coriolis", "f2d_addgrad", "f2d_sharp", "f2d_vorticity",
     "f2d_ke_finish", "f2d_pressure", "f2d_div", "f2d_c2v_scaled", "f2d_v2c_scaled",
     "f2d_adj_stage", "f2d_adj_combine", "f2d_bulk_diagnostics",
     "f2d_perpgrad_cfl_noalloc", "f2d_sw_momentum", "f2d_sw_momentum_u", "f2d_sw_diag",
@@ -161,6 +161,7 @@ def lib():
                                      ctypes.POINTER(vp)]),
         "f2d_poisson_destroy": (i32, [vp]),
         "f2d_poisson_method": (i32, [vp]),
+        "f2d_poisson_accept": (d, [vp, d]),
         "f2d_poisson_measure": (i32, [vp, i32]),
         "f2d_coriolis": (i32, [i32, gp, vp, vp, vp, vp, d, vp]),
         "f2d_addgrad": (i32, [i32, gp, vp, vp, vp, vp, vp, vp]),

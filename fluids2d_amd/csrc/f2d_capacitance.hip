@@ -288,9 +288,10 @@ __global__ __launch_bounds__(256) void k_cap_norms(CapGeo g, const TB* __restric
 
 // one block: relative residual into the solve statistics
 // [iterations, relres, converged, refinements | failed, max, solves]
-// (a direct solve is accepted unless its residual is above 1e-6 or not finite)
+// (accept: f2d_poisson_accept's)
 __global__ __launch_bounds__(256) void k_cap_stats(const double* __restrict__ part, int nb,
-                                                   int passes, double* __restrict__ st) {
+                                                   int passes, double accept,
+                                                   double* __restrict__ st) {
   __shared__ double sh[4];
   double a = 0.0, c = 0.0;
   for (int i = threadIdx.x; i < nb; i += 256) {
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(256) void k_cap_stats(const double* __restrict__ pa
   if (threadIdx.x != 0) return;
   double rel = c > 0.0 ? sqrt(a / c) : 0.0;
   if (!(a - a == 0.0 && c - c == 0.0)) rel = NAN;
-  const double conv = (rel <= 1e-6) ? 1.0 : 0.0;
+  const double conv = (rel <= accept) ? 1.0 : 0.0;
   st[0] = (double)passes;
   st[1] = rel;
   st[2] = conv;
@@ -567,7 +568,7 @@ CapSolver* cap_create(const int8_t* unk, int64_t ny, int64_t nx, double dx, doub
     const double one = 1.0;
     F2D_HIP(hipMemcpy(src + 3 * (nx2 + 6) + 3, &one, sizeof(double), hipMemcpyHostToDevice));
     if (modal)
-      modal_solve(gms, src, 0, G, false, nullptr, 0);
+      modal_solve(gms, src, 0, G, false, 0.0, nullptr, 0);
     else
       fft_solve_f64(gfs, src, 0, G, 0.0, false, nullptr, 0);
     double* A = nullptr;
@@ -662,33 +663,34 @@ static void gemv(CapSolver* c, hipStream_t s) {
 
 template <class TB, class TX>
 static void measure_res(CapSolver* c, const TB* b, int gmode, const TX* x, int passes,
-                        double* stats, hipStream_t s) {
+                        double accept, double* stats, hipStream_t s) {
   k_cap_norms<TB, TX><<<c->nbres, 256, 0, s>>>(c->g, b, gmode, c->mw, x, c->part);
-  k_cap_stats<<<1, 256, 0, s>>>(c->part, c->nbres, passes, stats);
+  k_cap_stats<<<1, 256, 0, s>>>(c->part, c->nbres, passes, accept, stats);
 }
 
 template <class T>
-void cap_solve_modal(CapSolver* c, const T* b, int gmode, T* x, bool measure, double* stats,
-                     hipStream_t s) {
+void cap_solve_modal(CapSolver* c, const T* b, int gmode, T* x, bool measure, double accept,
+                     double* stats, hipStream_t s) {
   F2D_REQUIRE(c->modal, "capacitance solver built on the spectral solve");
   const int64_t N = (int64_t)c->g.NYP * c->g.NXP;
   double* rhs = (double*)c->rhs;
   double* y = (double*)c->y;
   k_cap_rhs<T, double><<<blocks(N), 256, 0, s>>>(c->g, b, gmode, c->mw, rhs);
-  modal_solve(c->modal, rhs, 0, y, false, nullptr, s);
+  modal_solve(c->modal, rhs, 0, y, false, 0.0, nullptr, s);
   gemv<double>(c, s);
-  modal_solve(c->modal, rhs, 0, x, false, nullptr, s, nullptr, c->mw);
+  modal_solve(c->modal, rhs, 0, x, false, 0.0, nullptr, s, nullptr, c->mw);
   if (measure && stats) {
     // (FP32 x: the residual of the FP64 result, as modal_solve measures it)
-    if (sizeof(T) == 4) modal_solve(c->modal, rhs, 0, y, false, nullptr, s, nullptr, c->mw);
-    measure_res<T, double>(c, b, gmode, sizeof(T) == 4 ? y : (double*)x, 1, stats, s);
+    if (sizeof(T) == 4)
+      modal_solve(c->modal, rhs, 0, y, false, 0.0, nullptr, s, nullptr, c->mw);
+    measure_res<T, double>(c, b, gmode, sizeof(T) == 4 ? y : (double*)x, 1, accept, stats, s);
   }
   c->solved = true;
 }
 
-template void cap_solve_modal(CapSolver*, const double*, int, double*, bool, double*,
+template void cap_solve_modal(CapSolver*, const double*, int, double*, bool, double, double*,
                               hipStream_t);
-template void cap_solve_modal(CapSolver*, const float*, int, float*, bool, double*,
+template void cap_solve_modal(CapSolver*, const float*, int, float*, bool, double, double*,
                               hipStream_t);
 
 void cap_solve_f64(CapSolver* c, const double* b, int gmode, double* x, bool measure,
@@ -705,7 +707,7 @@ void cap_solve_f64(CapSolver* c, const double* b, int gmode, double* x, bool mea
   fft_solve_f64_masked(c->fft, b, gmode, y, m1, s);
   gemv<double>(c, s);
   fft_solve_f64_masked(c->fft, rhs, 0, x, m2, s);
-  if (measure && stats) measure_res<double, double>(c, b, gmode, x, 1, stats, s);
+  if (measure && stats) measure_res<double, double>(c, b, gmode, x, 1, DIRECT_ACCEPT, stats, s);
   c->solved = true;
 }
 
@@ -725,7 +727,7 @@ void cap_solve_f32(CapSolver* c, const float* b, int gmode, float* x, int nref, 
     fft_solve_f32_masked(c->fft, b, gmode, y, m1, s);
     gemv<float>(c, s);
     fft_solve_f32_masked(c->fft, rhs, 0, x, m2, s);
-    if (measure && stats) measure_res<float, float>(c, b, gmode, x, 1, stats, s);
+    if (measure && stats) measure_res<float, float>(c, b, gmode, x, 1, DIRECT_ACCEPT, stats, s);
     c->solved = true;
     return;
   }
@@ -768,7 +770,8 @@ void cap_solve_f32(CapSolver* c, const float* b, int gmode, float* x, int nref, 
       k_cap_acc<double><<<blocks(N), 256, 0, s>>>(N, c->mw, c->x64, y, c->x64);
   }
   k_cap_round<<<blocks(N), 256, 0, s>>>(N, c->mw, c->x64, x);
-  if (measure && stats) measure_res<float, double>(c, b, gmode, c->x64, passes, stats, s);
+  if (measure && stats)
+    measure_res<float, double>(c, b, gmode, c->x64, passes, DIRECT_ACCEPT, stats, s);
   c->solved = true;
 }
 

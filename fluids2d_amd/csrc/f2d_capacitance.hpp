@@ -43,10 +43,10 @@ int64_t cap_size(const CapSolver* c);
 bool cap_modal(const CapSolver* c);
 
 // x = A^-1 b of a modal solver, arguments as cap_solve_f64 (T: b's and x's
-// type, double or float)
+// type, double or float; accept: a measured residual up to it converged)
 template <class T>
-void cap_solve_modal(CapSolver* c, const T* b, int gmode, T* x, bool measure, double* stats,
-                     hipStream_t s);
+void cap_solve_modal(CapSolver* c, const T* b, int gmode, T* x, bool measure, double accept,
+                     double* stats, hipStream_t s);
 
 // x = A^-1 b at the unknowns (other entries untouched, halo not filled).
 // gmode 0: b at the vertices; 1: b = centerstovertices of the cell field.

@@ -16,6 +16,10 @@
 
 namespace f2d {
 
+// relative residual up to which a direct elliptic solve counts as converged
+// where it has no bound of its own (f2d_poisson_accept)
+constexpr double DIRECT_ACCEPT = 1e-6;
+
 // ---------------------------------------------------------------------------
 // errors
 // ---------------------------------------------------------------------------

@@ -1121,7 +1121,7 @@ __global__ __launch_bounds__(256) void k_fft_res(FftArgs a, const TB* __restrict
 // statistics [iterations, relres, converged, refinements | failed, max, solves]
 __global__ __launch_bounds__(256) void k_fft_stats(const double* __restrict__ part,
                                                    int nb, double n, int singular,
-                                                   double rtol, int nref,
+                                                   double accept, int nref,
                                                    int measured,
                                                    double* __restrict__ st) {
   __shared__ double sh[256];
@@ -1146,11 +1146,9 @@ __global__ __launch_bounds__(256) void k_fft_stats(const double* __restrict__ pa
     else
       rel = bb > 0.0 && rr > 0.0 ? sqrt(rr / bb) : 0.0;
     // a direct solve is exact up to rounding: its true residual sits at
-    // eps times the condition number (about 1e-11 at 1024^2 in FP64), so
-    // rtol is not its acceptance test; it is accepted unless the residual
-    // is not finite or above 1e-6 (a broken solve)
-    (void)rtol;
-    conv = (rel <= 1e-6) ? 1.0 : 0.0;
+    // eps times the condition number (about 1e-11 at 1024^2 in FP64); accept
+    // is f2d_poisson_accept's
+    conv = (rel <= accept) ? 1.0 : 0.0;
   }
   st[0] = (double)(nref + 1);
   st[1] = rel;
@@ -1523,17 +1521,17 @@ static const double* mean_of(FftSolver* f, const TB* b, int gmode, hipStream_t s
 }
 
 void fft_solve_f64(FftSolver* f, const double* b, int gmode, double* x,
-                   double rtol, bool measure, double* stats, hipStream_t s) {
+                   double accept, bool measure, double* stats, hipStream_t s) {
   F2D_REQUIRE(f->S64, "FFT solver built without FP64 buffers");
   spectral<double, double, double, 0>(f, b, gmode, x, nullptr, s);
   if (measure) residual<double>(f, b, gmode, x, nullptr, s, mean_of(f, b, gmode, s));
   if (stats && measure)
     k_fft_stats<<<1, 256, 0, s>>>(f->part, f->nbres, (double)f->a.onx * f->a.ony,
-                                  f->a.singular, rtol, 0, measure ? 1 : 0, stats);
+                                  f->a.singular, accept, 0, measure ? 1 : 0, stats);
 }
 
 void fft_solve_f32_refine(FftSolver* f, const float* b, int gmode, float* x,
-                          int nref, bool warm, double rtol, bool measure,
+                          int nref, bool warm, double accept, bool measure,
                           double* stats, hipStream_t s) {
   F2D_REQUIRE(f->S32, "FFT solver built without FP32 buffers");
   if (nref <= 0) {
@@ -1573,7 +1571,7 @@ void fft_solve_f32_refine(FftSolver* f, const float* b, int gmode, float* x,
   f->solved = true;
   if (stats && measure)
     k_fft_stats<<<1, 256, 0, s>>>(f->part, f->nbres, (double)f->a.onx * f->a.ony,
-                                  f->a.singular, rtol, nref, measure ? 1 : 0, stats);
+                                  f->a.singular, accept, nref, measure ? 1 : 0, stats);
 }
 
 // One FP32 spectral solve (rows forward, columns, rows inverse; x = the

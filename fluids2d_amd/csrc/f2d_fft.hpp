@@ -44,9 +44,10 @@ void fft_destroy(FftSolver* f);
 // x = A^-1 b on the padded (ny+6) x (nx+6) layout, halo filled.  gmode 0:
 // b given at the vertices; 1: b = centerstovertices(omega) of the cell
 // field passed as `b`.  FP64 throughout.  With `stats` (8 doubles, device)
-// the relative residual of the result is measured and recorded.
+// the relative residual of the result is measured and recorded, converged
+// up to accept.
 void fft_solve_f64(FftSolver* f, const double* b, int gmode, double* x,
-                   double rtol, bool measure, double* stats, hipStream_t s);
+                   double accept, bool measure, double* stats, hipStream_t s);
 
 // FP32 transforms with FP64 iterative refinement: x64 = S32(b), then
 // `nref` times r = b - A x64 (FP64), x64 += S32(r); x = (float) x64.
@@ -54,7 +55,7 @@ void fft_solve_f64(FftSolver* f, const double* b, int gmode, double* x,
 // starts from the caller's x (its interior; the halo is not read):
 // x64 = x + S32(b - A x), then nref - 1 further refinements.
 void fft_solve_f32_refine(FftSolver* f, const float* b, int gmode, float* x,
-                          int nref, bool warm, double rtol, bool measure,
+                          int nref, bool warm, double accept, bool measure,
                           double* stats, hipStream_t s);
 
 // Batched FP32 spectral solves of same-size members (blockIdx.y = member):

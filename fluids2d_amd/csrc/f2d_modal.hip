@@ -405,7 +405,8 @@ __global__ __launch_bounds__(256) void k_modal_norms(ModalRes g, const TB* __res
 // relative residual of the (projected) system into the solve statistics
 // [iterations, relres, converged, refinements | failed, max, solves]
 __global__ __launch_bounds__(256) void k_modal_stats(const double* __restrict__ part, double n,
-                                                     int singular, double* __restrict__ st) {
+                                                     int singular, double accept,
+                                                     double* __restrict__ st) {
   __shared__ double sh[4];
   double v[3];
   for (int c = 0; c < 3; c++) {
@@ -418,7 +419,7 @@ __global__ __launch_bounds__(256) void k_modal_stats(const double* __restrict__ 
   if (singular) rr -= v[1] * v[1] / n;
   const bool finite = rr - rr == 0.0 && v[2] - v[2] == 0.0;
   const double rel = !finite ? NAN : (v[2] > 0.0 && rr > 0.0 ? sqrt(rr / v[2]) : 0.0);
-  const double conv = rel <= 1e-6 ? 1.0 : 0.0;
+  const double conv = rel <= accept ? 1.0 : 0.0;
   st[0] = 1.0;
   st[1] = rel;
   st[2] = conv;
@@ -548,8 +549,8 @@ static void launch_pass(const ModalPass& a, hipStream_t s) {
 }
 
 template <class TB, class TX>
-void modal_solve(ModalSolver* m, const TB* b, int gmode, TX* x, bool measure, double* stats,
-                 hipStream_t s, const double* skip, const int8_t* only) {
+void modal_solve(ModalSolver* m, const TB* b, int gmode, TX* x, bool measure, double accept,
+                 double* stats, hipStream_t s, const double* skip, const int8_t* only) {
   const ModalDir &dx = m->x, &dy = m->y;
   F2D_REQUIRE(!gmode || (dx.cell && dy.cell), "the cell operator takes b on the cells");
   // 1: rows of b -> modes of x (t1: one row per mode)
@@ -650,15 +651,16 @@ void modal_solve(ModalSolver* m, const TB* b, int gmode, TX* x, bool measure, do
     } else {
       k_modal_norms<TB, double><<<MODAL_NB, 256, 0, s>>>(g, b, x, m->singular, sum, m->part);
     }
-    k_modal_stats<<<1, 256, 0, s>>>(m->part, (double)g.ny * g.nx, m->singular, stats);
+    k_modal_stats<<<1, 256, 0, s>>>(m->part, (double)g.ny * g.nx, m->singular, accept,
+                                   stats);
   }
 }
 
-template void modal_solve(ModalSolver*, const double*, int, double*, bool, double*,
+template void modal_solve(ModalSolver*, const double*, int, double*, bool, double, double*,
                           hipStream_t, const double*, const int8_t*);
-template void modal_solve(ModalSolver*, const float*, int, float*, bool, double*, hipStream_t,
-                          const double*, const int8_t*);
-template void modal_solve(ModalSolver*, const double*, int, float*, bool, double*, hipStream_t,
-                          const double*, const int8_t*);
+template void modal_solve(ModalSolver*, const float*, int, float*, bool, double, double*,
+                          hipStream_t, const double*, const int8_t*);
+template void modal_solve(ModalSolver*, const double*, int, float*, bool, double, double*,
+                          hipStream_t, const double*, const int8_t*);
 
 }  // namespace f2d

@@ -32,12 +32,13 @@ void modal_destroy(ModalSolver* m);
 // given at the unknowns; 1 (vertices): b = centerstovertices of the cell
 // field (operators.py:126-133, formed inside the first transform: the
 // averaged eigenvectors).  measure: the relative residual goes to `stats` (8
-// doubles, device), as the other direct solves record it.  skip: a device
+// doubles, device), as the other direct solves record it, converged up to
+// accept.  skip: a device
 // flag; the passes of a solve enqueued behind a nonzero one do nothing.
 // only: a mask on the padded layout; x is written where it is set, without
 // halo images.
 template <class TB, class TX>
-void modal_solve(ModalSolver* m, const TB* b, int gmode, TX* x, bool measure, double* stats,
-                 hipStream_t s, const double* skip = nullptr, const int8_t* only = nullptr);
+void modal_solve(ModalSolver* m, const TB* b, int gmode, TX* x, bool measure, double accept,
+                 double* stats, hipStream_t s, const double* skip = nullptr, const int8_t* only = nullptr);
 
 }  // namespace f2d

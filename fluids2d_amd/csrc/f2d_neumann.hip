@@ -660,7 +660,7 @@ static void rcg(NeumannSolver* s, double rtol, int maxit, bool sync, hipStream_t
     if (s->fft)
       fft_solve_f64(s->fft, s->r, 0, s->z, 0.0, false, nullptr, st);
     else
-      modal_solve(s->modal, s->r, 0, s->z, false, nullptr, st, s->sc + 2);
+      modal_solve(s->modal, s->r, 0, s->z, false, 0.0, nullptr, st, s->sc + 2);
     k_rcg_rz<<<nb, NEU_BS, 0, st>>>(n, s->m, s->r, s->z, s->part, s->sc);
   };
   k_rcg_start<<<nb, NEU_BS, 0, st>>>(s->a, n, s->m, s->dg, s->g, s->x, s->r, e, s->part);

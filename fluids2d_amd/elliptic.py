@@ -19,7 +19,7 @@ DEFAULT_RTOL = {"fp64": 1e-13, "fp32": 1e-9}
 DEFAULT_MAXIT = {"fp64": 100, "fp32": 8}
 
 
-# methods that solve directly: no iteration count to learn, no rtol test
+# methods that solve directly: no iteration count to learn
 DIRECT = ("fft", "capacitance", "modal", "modal_capacitance")
 
 
@@ -112,7 +112,7 @@ class Poisson2D:
         _lib.call("f2d_poisson_create", unk.ctypes.data_as(ctypes.c_void_p), mesh.grid_ref(),
                   self.maindiag, ctypes.byref(opts), ctypes.byref(h))
         self._h = h
-        # "fft": direct spectral solve (exact to rounding, no rtol test);
+        # "fft": direct spectral solve (exact to rounding);
         # "modal": direct eigenvector solve; "capacitance",
         # "modal_capacitance": direct masked solves around them; "mg":
         # multigrid-preconditioned CG to rtol
@@ -182,7 +182,7 @@ class Poisson2D:
         self.last_iters, self.last_relres = it.value, rr.value
         if check and not self._accepted(rr.value):
             raise PoissonNotConverged(
-                f"Poisson solve reached relres {rr.value:.3e} > {self.rtol:.1e} "
+                f"Poisson solve reached relres {rr.value:.3e} > {self.accept():.1e} "
                 f"after {it.value} iterations")
         if not host:
             ref = int(self._stats_host()[3]) if self.precision != "fp64" else None
@@ -191,17 +191,23 @@ class Poisson2D:
             x[...] = dx.double().cpu().numpy()
         return None
 
+    def accept(self):
+        """The largest relative residual of an accepted solve: rtol, for the
+        direct solves that took the place of an iteration to rtol no less
+        than the bound of their rounding (f2d_poisson_accept), else 1e-6.
+        FP32 transforms refined once from the previous solution: 1e-4, the
+        FP64 residual of FP32 rounding at the high wavenumbers (the operator
+        amplifies them by k^2)."""
+        if self.precision != "fp64" and self.method in ("fft", "capacitance"):
+            return 1e-4
+        return _lib.lib().f2d_poisson_accept(self._h, self.rtol)
+
     def _accepted(self, relres):
         if relres != relres and self.method in ("fft", "capacitance"):
             # the state is not finite: a run goes on to its own check for
             # that, which stops it cleanly (Model._check_finite)
             return True
-        if self.method in DIRECT:
-            # direct: exact up to rounding.  FP32 transforms refined once from
-            # the previous solution: the FP64 residual of FP32 rounding at
-            # the high wavenumbers (the operator amplifies them by k^2)
-            return relres <= (1e-6 if self.precision == "fp64" else 1e-4)
-        return relres <= self.rtol
+        return relres <= self.accept()
 
     def _learn(self, it, refinements=None):
         n = refinements if self.precision != "fp64" else it
@@ -228,7 +234,7 @@ class Poisson2D:
             self.last_iters, self.last_relres = it.value, rr.value
             if not self._accepted(rr.value):
                 raise PoissonNotConverged(
-                    f"Poisson solve reached relres {rr.value:.3e} > {self.rtol:.1e} "
+                    f"Poisson solve reached relres {rr.value:.3e} > {self.accept():.1e} "
                     f"after {it.value} iterations")
             ref = None
             if self.precision != "fp64":
@@ -262,7 +268,7 @@ class Poisson2D:
         self.last_relres = relres
         if not self._accepted(relres):
             raise PoissonNotConverged(
-                f"Poisson solve reached relres {relres:.3e} > {self.rtol:.1e} "
+                f"Poisson solve reached relres {relres:.3e} > {self.accept():.1e} "
                 f"after 1 iterations")
 
     def set_refine(self, nref):

@@ -369,7 +369,7 @@ class RKIntegrator:
         key = self._graph_key() + self.model.graph_operands(self.dstate) + tuple(
             getattr(self.param, n, None) for n in self.BAKED) + (
             self._wants_dtn(), m.dx, m.dy, m.area, m.grid.tile,
-            getattr(self.model, "fused", True), tuple((id(e), e.refine) for e in sols))
+            getattr(self.model, "fused", True), tuple((id(e), e.refine, e.rtol) for e in sols))
         got = self._checked.get(key)
         if got is not None:
             return got

@@ -516,10 +516,17 @@ int f2d_poisson_solve(f2d_poisson* h, const void* b, void* x, double rtol,
  * SuperLU factor is its only method (elliptic.py:78).  With all but MG and
  * NEUMANN_CG the solve is direct: `maxit` is unused, *iters receives
  * 1 + the FP64 refinements, *relres the measured true relative residual,
- * and the solve counts as converged when that residual is below 1e-6
- * (`rtol` is not its acceptance test: a direct FP64 solve reaches eps times
- * the condition number, about 1e-11 at 1024^2). */
+ * and the solve counts as converged up to f2d_poisson_accept. */
 int f2d_poisson_method(f2d_poisson* h);
+/* The relative residual up to which a solve with `rtol` counts as converged
+ * (-1 for NULL; no counterpart in the reference, whose SuperLU tests
+ * nothing).  MG and NEUMANN_CG: rtol.  A direct solve reaches eps times the
+ * condition number, about 1e-11 at 1024^2, whatever rtol is: FFT and CAP
+ * count up to 1e-6; MODAL, MODAL_CAP and the FP64 FFT of 4096 points a
+ * direction up to rtol or, if that is larger, the bound of their rounding
+ * (64 times 2^-53, MODAL_CAP 512 times, the condition number of the
+ * rectangle's operator; at most 1e-6). */
+double f2d_poisson_accept(const f2d_poisson* h, double rtol);
 /* FP64 refinement passes of the handle's following direct (FFT or
  * capacitance) solves in the FP32 modes: 0 makes them plain FP32 solves, -1
  * returns to f2d_poisson_opts.fft_refine (no counterpart in the reference,

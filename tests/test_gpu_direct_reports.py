@@ -105,3 +105,60 @@ def test_spoilt_run_stops_cleanly(dev, nx, ny, nisl):
         m.diags.append(spoil)
         m.run()
         assert m.nonfinite == ["omega"] and m.time.ite == 24
+
+
+def _condition(nx, ny, xper=False, yper=False, lx=1.0, ly=1.0, maindiag=0.0, cells=False):
+    """Condition number of the rectangle's operator from its eigenvalues, on
+    the zero-mean functions where it is singular."""
+    def lam(n, per, c):
+        k = np.arange(n) if per or cells else np.arange(1, n)
+        return 4 * c * np.sin((np.pi if per else np.pi / 2) * k / n) ** 2
+    dx, dy = lx / nx, ly / ny
+    v = (lam(nx, xper, dy / dx)[:, None] + lam(ny, yper, dx / dy) + maindiag).ravel()
+    return v.max() / v[v > 1e-13 * v.max()].min()
+
+
+@pytest.mark.parametrize("method,kw,factor", [
+    ("modal", dict(nx=40, ny=48), 64), ("modal", dict(nx=9, ny=8, precision="fp32"), 64),
+    ("modal", dict(nx=300, ny=65, xperiodic=True), 64),
+    ("modal", dict(nx=61, ny=30, yperiodic=True, location="c"), 64),
+    ("modal", dict(nx=40, ny=41, xperiodic=True, yperiodic=True), 64),
+    ("modal_capacitance", dict(nx=40, ny=48, nisl=3), 512),
+    ("fft", dict(nx=4096, ny=64, xperiodic=True, yperiodic=True), 64),
+    ("fft", dict(nx=64, ny=64), None), ("fft", dict(nx=64, ny=64, precision="fp32"), None),
+    ("capacitance", dict(nx=64, ny=64, nisl=3), None), ("mg", dict(nx=40, ny=48), 0)])
+def test_acceptance(dev, method, kw, factor):
+    """A direct solve that takes the place of an iteration to rtol is accepted
+    at rtol or at the bound of its rounding; a smooth right-hand side, whose
+    solution is the largest, stays inside; the other routes' tests stay."""
+    kw = dict(kw)
+    if method == "mg":
+        kw["poisson_solver"] = "mg"
+    ps = _solver(**kw)
+    assert ps.method == method
+    single = kw.get("precision") == "fp32"
+    if factor is None:
+        assert ps.accept() == (1e-4 if single else 1e-6)
+        ps.rtol = 1e-2
+        assert ps.accept() == (1e-4 if single else 1e-6)
+        return
+    geo = {k: v for k, v in kw.items() if k in ("nx", "ny")}
+    cond = _condition(**geo, xper=kw.get("xperiodic", False), yper=kw.get("yperiodic", False),
+                      lx=kw["nx"] / 64.0, ly=kw["ny"] / 64.0, cells=kw.get("location") == "c")
+    bound = factor * 2.0 ** -53 * (cond + 100)
+    assert ps.accept() == pytest.approx(max(ps.rtol, bound), rel=1e-6)
+    if method != "mg":
+        assert bound < 5e-8  # not the 1e-6 of the other routes
+    wet = ps.msk != 0
+    j, i = np.mgrid[0:wet.shape[0], 0:wet.shape[1]]
+    b = np.cos(2 * np.pi * (i - 3) / kw["nx"]) * np.cos(np.pi * (j - 3) / kw["ny"]) * wet
+    if kw.get("location") == "c" or kw.get("yperiodic"):
+        b[wet] -= b[wet].mean()
+    x = torch.zeros(b.shape, dtype=ps.dtype, device=dev)
+    ps.reset_stats()
+    ps.solve(torch.from_numpy(b).to(dev, ps.dtype), x)
+    st = ps.read_stats()
+    assert st["failed"] == 0 and ps.last_relres <= ps.accept()
+    assert not ps._accepted(1e-7)
+    ps.rtol = 1e-3  # a looser one is the caller's to choose
+    assert ps._accepted(9e-4) and not ps._accepted(2e-3)
