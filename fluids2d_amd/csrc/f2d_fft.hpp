@@ -45,9 +45,11 @@ void fft_destroy(FftSolver* f);
 // b given at the vertices; 1: b = centerstovertices(omega) of the cell
 // field passed as `b`.  FP64 throughout.  With `stats` (8 doubles, device)
 // the relative residual of the result is measured and recorded, converged
-// up to accept.
+// up to accept.  skip: a device flag; the passes of a solve enqueued behind a
+// nonzero one do nothing.
 void fft_solve_f64(FftSolver* f, const double* b, int gmode, double* x,
-                   double accept, bool measure, double* stats, hipStream_t s);
+                   double accept, bool measure, double* stats, hipStream_t s,
+                   const double* skip = nullptr);
 
 // FP32 transforms with FP64 iterative refinement: x64 = S32(b), then
 // `nref` times r = b - A x64 (FP64), x64 += S32(r); x = (float) x64.

@@ -658,7 +658,7 @@ static void rcg(NeumannSolver* s, double rtol, int maxit, bool sync, hipStream_t
   auto precondition = [&](int it) {
     k_rcg_check<<<1, NEU_BS, 0, st>>>(s->part, nb, rtol, maxit, it, s->sc);
     if (s->fft)
-      fft_solve_f64(s->fft, s->r, 0, s->z, 0.0, false, nullptr, st);
+      fft_solve_f64(s->fft, s->r, 0, s->z, 0.0, false, nullptr, st, s->sc + 2);
     else
       modal_solve(s->modal, s->r, 0, s->z, false, 0.0, nullptr, st, s->sc + 2);
     k_rcg_rz<<<nb, NEU_BS, 0, st>>>(n, s->m, s->r, s->z, s->part, s->sc);
