@@ -4,7 +4,9 @@ The library is the only compute path of the package: if it is missing or the
 device is unavailable every entry point raises, there is no CPU fallback.
 """
 import ctypes
+import gc
 import os
+import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIBPATH = os.path.join(_HERE, "libfluids2d_amd.so")
@@ -244,43 +246,50 @@ def stream_ptr(stream=None):
     return ctypes.c_void_p(s.cuda_stream)
 
 
+class no_gc:
+    """Python's cyclic garbage collector held off: a collection during a graph
+    capture could run a finaliser that frees device memory (a solver handle),
+    which a capture does not allow.  The collector is the process's: it stays
+    off until the last of the threads inside has left, and comes back on only
+    if it was on when the first came."""
+    _lock = threading.Lock()
+    _inside, _was = 0, False
+
+    def __enter__(self):
+        with no_gc._lock:
+            if no_gc._inside == 0:
+                no_gc._was = gc.isenabled()
+                gc.disable()
+            no_gc._inside += 1
+
+    def __exit__(self, *exc):
+        with no_gc._lock:
+            no_gc._inside -= 1
+            if no_gc._inside == 0 and no_gc._was:
+                gc.enable()
+
+
 class capture:
-    """``with capture(graph):`` -- torch.cuda.graph with Python's cyclic
-    garbage collector held off: a collection during the capture could run a
-    finaliser that frees device memory (a solver handle), which a capture in
-    global mode does not allow."""
+    """``with capture(graph):`` -- torch.cuda.graph inside no_gc."""
 
     def __init__(self, graph, **kw):
         import torch
         self._ctx = torch.cuda.graph(graph, **kw)
+        self._off = no_gc()
 
     def __enter__(self):
-        import gc
-        self._gc = gc.isenabled()
-        gc.disable()
-        return self._ctx.__enter__()
+        self._off.__enter__()
+        try:
+            return self._ctx.__enter__()
+        except BaseException:
+            self._off.__exit__()
+            raise
 
     def __exit__(self, *exc):
-        import gc
         try:
             return self._ctx.__exit__(*exc)
         finally:
-            if self._gc:
-                gc.enable()
-
-
-class no_gc:
-    """Python's cyclic garbage collector held off (see ``capture``)."""
-
-    def __enter__(self):
-        import gc
-        self._gc = gc.isenabled()
-        gc.disable()
-
-    def __exit__(self, *exc):
-        import gc
-        if self._gc:
-            gc.enable()
+            self._off.__exit__()
 
 
 def capturing():
