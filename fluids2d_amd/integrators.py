@@ -71,7 +71,7 @@ class RKIntegrator:
         self._checked = {}
         self._h_run = torch.zeros(4, dtype=torch.float64).pin_memory()
         self._dt_on_host = False
-        self._run_steps, self._run_mesh = 0, None
+        self._run_steps, self._run_total, self._run_mesh = 0, 0, None
         self._no_replay = False
         self._dtn_valid = False
         # Models with ``defers_cfl``: the last stage leaves the next step's
@@ -319,12 +319,13 @@ class RKIntegrator:
 
     def device_step(self, time):
         """One host-checked step (Model.run's): with direct solvers and
-        ``param.hipgraph``, after two eager steps, the replay of a captured
-        step whose solves leave their measured residuals on the device and
+        ``param.hipgraph``, after two eager steps and where captures pay
+        (_pays), the replay of a captured step whose solves leave their measured residuals on the device and
         then in pinned memory, with the next dt.  They are waited for here:
         a replayed step's solves are checked as an eager step's are, before
         the time goes forward."""
-        g = self._checked_step() if self._can_replay() else None
+        g = self._checked_step(time) if self._can_replay(time) else None
+        self._run_total += 1
         if g is None:
             self.advance()
             self._run_steps += 1
@@ -342,7 +343,7 @@ class RKIntegrator:
             self._dt_part = self._dtn_part = False
         time.pushforward()
 
-    def _can_replay(self):
+    def _can_replay(self, time):
         if self._run_mesh != self.mesh.version:
             # a re-finalised mesh builds its solvers in the next eager steps
             self._run_mesh, self._run_steps = self.mesh.version, 0
@@ -350,7 +351,26 @@ class RKIntegrator:
                 and self._run_steps >= 2 and not self._dt_part and not self._no_replay
                 and getattr(self.model, "capturable", True)
                 and getattr(self.model, "events", None) is None
-                and all(e.method in DIRECT for e in self._solvers()))
+                and all(e.method in DIRECT for e in self._solvers())
+                and (self._checked or self._pays(time)))
+
+    # Steps from which a run's captures pay, without and with elliptic solves.
+    # A fresh model captures twice (the buffers alternate), 0.4 to 1 ms in all;
+    # a replayed step saves 0 (advection) to 40 us (rsw), with solves and their
+    # host checks 70 to 480.  Runs of a fresh model, captured / eager: eulerpsi 64^2 1.68 at 4
+    # steps, 1.22 at 8, 0.93 at 12; 512^2 1.15, 1.05, 0.99; euler 40^2 1.17,
+    # 0.76, 0.62; rsw 100^2 1.34 at 4, 1.04 at 12, 0.89 at 24; advection 256^2
+    # 1.50 at 4, 1.20 at 24, 1.02 at 40.
+    REPLAY_FROM = (36, 11)
+
+    def _pays(self, time):
+        """Whether the steps taken so far and those to come in this run (by
+        ``maxite``, and by ``tend`` at the present dt) are enough to capture."""
+        p = self.param
+        left = p.maxite - (time.ite - time.ite0)
+        if time.dt > 0:
+            left = min(left, (time.t0 + p.tend - time.t) / time.dt)
+        return self._run_total + left >= self.REPLAY_FROM[bool(self._solvers())]
 
     # the parameters that a stage reads as it is launched, part of a captured
     # step's key (with the sign of ``dt``, the value of a fixed one is on the
@@ -359,9 +379,10 @@ class RKIntegrator:
              "innerproduct", "f0", "g", "H", "beta", "xperiodic", "yperiodic",
              "poisson_refine")
 
-    def _checked_step(self):
+    def _checked_step(self, time):
         """The captured host-checked step of the current buffers and
-        parameters: (graph, state and alternate state after it, solvers).
+        parameters: (graph, state and alternate state after it, solvers), None
+        where there is none and a capture would not pay.
         The next step's dt and the solvers' worst residuals go to pinned host
         memory by kernels of the graph."""
         m = self.mesh
@@ -371,7 +392,7 @@ class RKIntegrator:
             self._wants_dtn(), m.dx, m.dy, m.area, m.grid.tile,
             getattr(self.model, "fused", True), tuple((id(e), e.refine, e.rtol) for e in sols))
         got = self._checked.get(key)
-        if got is not None:
+        if got is not None or not self._pays(time):
             return got
         if len(self._checked) >= 16:  # parameters that change as the run goes
             self._checked.clear()

@@ -164,8 +164,9 @@ def test_captured_steps_read_keyed_parameters_only(dev, model, precision, kw):
         o.param = _Reads(o.param, names)
     if integ._wants_dtn():
         integ._dtn_valid = True
+    integ._pays = lambda time: True  # (reads the run's length)
     names.clear()
-    assert integ._checked_step() is not None
+    assert integ._checked_step(m.time) is not None
     assert "integrator" in names and names <= set(integ.BAKED) | {"dt"}, names
 
 
@@ -186,6 +187,7 @@ def test_captured_steps_own_their_reductions(dev, monkeypatch, model, kw):
     monkeypatch.setattr(_lib, "call", call)
     monkeypatch.setattr(operators, "call", call)
     m = _start(model, 64, 64, 0, "fp64", True, **kw)
+    m.param.maxite = 40
     m.run()
     m.integrator.begin(m.state)
     m.integrator.device_steps(12)
@@ -264,3 +266,26 @@ def test_resident_steps_after_replayed_ones(dev):
         out.append((m.state.omega.copy(), dts))
     assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
 
+
+
+@pytest.mark.parametrize("model,kw,short,long", [
+    ("eulerpsi", {}, dict(maxite=8), dict(maxite=30)),
+    ("eulerpsi", dict(dt=0.01), dict(tend=0.05), dict(tend=0.4)),
+    ("rsw", {}, dict(maxite=24), dict(maxite=60))])
+def test_short_runs_capture_nothing(dev, model, kw, short, long):
+    """A capture costs what some ten replayed steps save: a run with fewer
+    steps to come, by maxite or by tend, stays eager, its first and (while all
+    its runs together are short) its later ones."""
+    m = _start(model, 64, 64, 0, "fp64", True, **kw)
+    m.param.maxite = 10 ** 6
+    for k, v in short.items():
+        setattr(m.param, k, v)
+    m.run()
+    integ = m.integrator
+    assert m.time.ite > 3 and not integ._checked
+    n = m.time.ite
+    for k, v in long.items():
+        setattr(m.param, k, v)
+    m.time.ite0, m.time.t0 = m.time.ite, m.time.t
+    m.run()
+    assert m.time.ite > n and integ._checked
