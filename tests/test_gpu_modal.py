@@ -1,9 +1,10 @@
 """The eigenvector solve of fully wet rectangles whose sizes are not powers
 of two (csrc/f2d_modal.hip) against SuperLU (the oracle's Poisson2D): every
-combination of closed and periodic directions at the edges of its tiles (16
-and 32 output pairs, chunks of 16 and 32 contraction pairs), odd and even
-point counts, with and without mass term, vertex and cell operators, the
-fused centerstovertices right-hand side, FP64 and FP32 storage."""
+combination of closed and periodic directions at the edges of its 16 x 16
+tiles and chunks of 32 contraction pairs (test_gpu_modal_tiles.py has the
+larger tiles), odd and even point counts, with and without mass term, vertex
+and cell operators, the fused centerstovertices right-hand side, FP64 and FP32
+storage."""
 import ctypes
 
 import numpy as np
@@ -16,8 +17,8 @@ from test_gpu_kernels import L, N, T, _poisson_case  # noqa: F401  (L: a fixture
 
 pytestmark = pytest.mark.gpu
 
-# tile edges: pairs of 32 / 33 / 64 / 65 points a side, the smallest sizes,
-# more output tiles than one per CU (800 x 304, 1000 x 600), odd sizes
+# tile and chunk edges: pairs of 32 / 33 / 64 / 65 points a side, the smallest
+# sizes, more output tiles than one per CU (800 x 304, 1000 x 600), odd sizes
 SIZES = [(8, 9), (11, 10), (33, 32), (65, 63), (40, 40), (130, 66), (61, 200)]
 
 
