@@ -2263,7 +2263,7 @@ int f2d_poisson_bench_kernel(f2d_poisson* h, int kind, int reps, double* us,
       *us = fft_bench(h->fft, h->opts.mode == F2D_POISSON_F64, kind - 3, reps, s, bytes);
       return;
     }
-    F2D_REQUIRE(!h->fft || h->p64.L > 0 || h->p32.L > 0, "no multigrid hierarchy");
+    F2D_REQUIRE(h->p64.L > 0 || h->p32.L > 0, "no multigrid hierarchy");
     if (h->opts.mode == F2D_POISSON_F64)
       *us = bench_kernel<double>(h, h->p64, kind, reps, s, bytes);
     else
@@ -2365,7 +2365,18 @@ int f2d_poisson_create(const int8_t* unknowns_host, const f2d_grid* g,
     h->scal = (double*)dalloc(h, sizeof(double) * 8);
     h->outer = (Ctl*)dalloc(h, sizeof(Ctl));
     h->bench_ctl = (Ctl*)dalloc(h, sizeof(Ctl));
-    if (h->opts.mode == F2D_POISSON_F64) {
+    // no multigrid solves a Neumann operator: the direct solves that took the
+    // place of the Jacobi-PCG need the control block alone (the hierarchy of
+    // a long, thin rectangle ends on a level that is refused)
+    const bool no_pcg =
+        h->opts.neumann &&
+        (modal_ok || !fft_fits(h->ny, h->nx, h->xper, h->yper,
+                               h->opts.mode == F2D_POISSON_F64, true));
+    if (no_pcg) {
+      Ctl* c = (Ctl*)dalloc(h, sizeof(Ctl));
+      F2D_HIP(hipMemset(c, 0, sizeof(Ctl)));
+      (h->opts.mode == F2D_POISSON_F64 ? h->p64.ctl : h->p32.ctl) = c;
+    } else if (h->opts.mode == F2D_POISSON_F64) {
       build_pcg<double>(h, h->p64);
       if (h->p64.Lt < h->p64.L) set_tail_attr<double>(h->p64.tail_lds);
     } else {
