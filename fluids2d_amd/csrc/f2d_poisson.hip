@@ -1565,11 +1565,9 @@ static double rect_condition(int64_t ny, int64_t nx, double dx, double dy, doubl
 // condition number is accepted: the rounding of x's transforms through the
 // operator.  Measured, in units of 2^-53 times the condition number, over
 // sizes 8 to 4096, cells of 1:1 and 7:1, smooth, noisy and point right-hand
-// sides: up to 13; around a capacitance solve (factor 8 here) up to 34, on
-// cells of 7:1 with scattered dry points.
-static double rounding_bound(double condition, bool capacitance) {
-  const double b = (capacitance ? 512.0 : 64.0) * 0x1p-53 * (condition + 100.0);
-  return std::min(b, DIRECT_ACCEPT);
+// sides: up to 13 (a capacitance solve is refined to 64 at most).
+static double rounding_bound(double condition) {
+  return std::min(64.0 * 0x1p-53 * (condition + 100.0), DIRECT_ACCEPT);
 }
 
 // relative residual at which a solve with this rtol counts as converged
@@ -2447,10 +2445,8 @@ int f2d_poisson_create(const int8_t* unknowns_host, const f2d_grid* g,
     if (h->modal || (h->cap && cap_modal(h->cap)) ||
         (h->fft && h->opts.mode == F2D_POISSON_F64 &&
          !fft_fits(h->ny, h->nx, h->xper, h->yper, true, true)))
-      h->accept = rounding_bound(
-          rect_condition(h->ny, h->nx, g->dx, g->dy, maindiag, h->xper, h->yper,
-                         h->opts.neumann != 0),
-          h->cap != nullptr);
+      h->accept = rounding_bound(rect_condition(h->ny, h->nx, g->dx, g->dy, maindiag, h->xper,
+                                                h->yper, h->opts.neumann != 0));
     F2D_HIP(hipDeviceSynchronize());
     *out = h;
   });

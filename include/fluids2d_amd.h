@@ -483,7 +483,8 @@ typedef struct f2d_poisson_opts {
  * eigenvector solve, which AUTO takes for a masked vertex operator inside a
  * rectangle of sizes that are not both powers of two (at most 4096, 2048 in
  * a closed direction; a closed direction or maindiag > 0; at most 8192
- * boundary points).  FP64 in every mode; not taken into batches. */
+ * boundary points).  FP64 in every mode, refined in FP64 where the mask needs
+ * it (found at creation); not taken into batches. */
 #define F2D_SOLVER_MODAL_CAP 6
 /* The masked vertex operator of a mask inside a rectangle the FFT solve
  * handles (power-of-two sizes, a closed direction or maindiag > 0): the
@@ -524,8 +525,8 @@ int f2d_poisson_method(f2d_poisson* h);
  * condition number, about 1e-11 at 1024^2, whatever rtol is: FFT and CAP
  * count up to 1e-6; MODAL, MODAL_CAP and the FP64 FFT of 4096 points a
  * direction up to rtol or, if that is larger, the bound of their rounding
- * (64 times 2^-53, MODAL_CAP 512 times, the condition number of the
- * rectangle's operator; at most 1e-6). */
+ * (64 times 2^-53 times the condition number of the rectangle's operator; at
+ * most 1e-6). */
 double f2d_poisson_accept(const f2d_poisson* h, double rtol);
 /* FP64 refinement passes of the handle's following direct (FFT or
  * capacitance) solves in the FP32 modes: 0 makes them plain FP32 solves, -1

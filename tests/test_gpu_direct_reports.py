@@ -123,7 +123,7 @@ def _condition(nx, ny, xper=False, yper=False, lx=1.0, ly=1.0, maindiag=0.0, cel
     ("modal", dict(nx=300, ny=65, xperiodic=True), 64),
     ("modal", dict(nx=61, ny=30, yperiodic=True, location="c"), 64),
     ("modal", dict(nx=40, ny=41, xperiodic=True, yperiodic=True), 64),
-    ("modal_capacitance", dict(nx=40, ny=48, nisl=3), 512),
+    ("modal_capacitance", dict(nx=40, ny=48, nisl=3), 64),
     ("fft", dict(nx=4096, ny=64, xperiodic=True, yperiodic=True), 64),
     ("fft", dict(nx=64, ny=64), None), ("fft", dict(nx=64, ny=64, precision="fp32"), None),
     ("capacitance", dict(nx=64, ny=64, nisl=3), None), ("mg", dict(nx=40, ny=48), 0)])
