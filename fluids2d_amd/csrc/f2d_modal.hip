@@ -444,7 +444,7 @@ struct ModalSolver {
   int singular = 0;
   double *t1 = nullptr, *t2 = nullptr;
   double* part = nullptr;
-  double* x64 = nullptr;  // FP64 result of a measured FP32 solve (on first use)
+  double* x64 = nullptr;  // FP64 result of a measured FP32 solve
   std::vector<void*> allocs;
 };
 
@@ -498,7 +498,7 @@ static void dir_create(ModalSolver* m, ModalDir& d, int bc, int n, double c, dou
 }
 
 ModalSolver* modal_create(int64_t ny, int64_t nx, double dx, double dy, double maindiag,
-                          int xper, int yper, bool cells) {
+                          int xper, int yper, bool cells, bool single) {
   ModalSolver* m = new ModalSolver();
   try {
     const int closed = cells ? BC_EVEN : BC_WALL;
@@ -515,6 +515,7 @@ ModalSolver* modal_create(int64_t ny, int64_t nx, double dx, double dy, double m
     m->t1 = malloc_dev<double>(m, sizeof(double) * n);
     m->t2 = malloc_dev<double>(m, sizeof(double) * n);
     m->part = malloc_dev<double>(m, sizeof(double) * 4 * MODAL_NB);
+    if (single) m->x64 = malloc_dev<double>(m, sizeof(double) * (size_t)(nx + 6) * (ny + 6));
     F2D_HIP(hipDeviceSynchronize());
   } catch (...) {
     modal_destroy(m);
@@ -639,10 +640,7 @@ void modal_solve(ModalSolver* m, const TB* b, int gmode, TX* x, bool measure, do
     if constexpr (sizeof(TX) == 4) {
       // the residual of x rounded to FP32 (1e-3 at 1024^2, the operator
       // amplifies the rounding) says nothing: that of the FP64 result
-      if (!m->x64) {
-        const size_t n = (size_t)m->NXP * (m->y.n + 6);
-        m->x64 = malloc_dev<double>(m, sizeof(double) * n);
-      }
+      F2D_REQUIRE(m->x64, "eigenvector solver built without its FP64 result");
       r.out = m->x64;
       r.only = nullptr;
       launch_pass<false, EPI_PADDED, double, double>(r, s);

@@ -23,8 +23,9 @@ struct ModalSolver;
 // and the sizes lie in [8, 4096] (a halo point is the image of one unknown)
 bool modal_applicable(int64_t ny, int64_t nx, int xper, int yper, int64_t nwet, bool cells);
 
+// single: FP32 solves are to be measured (modal_solve), from FP64 results
 ModalSolver* modal_create(int64_t ny, int64_t nx, double dx, double dy, double maindiag,
-                          int xper, int yper, bool cells);
+                          int xper, int yper, bool cells, bool single = false);
 void modal_destroy(ModalSolver* m);
 
 // x = A^-1 b at the unknowns and their periodic halo images, on the padded

@@ -2409,7 +2409,7 @@ int f2d_poisson_create(const int8_t* unknowns_host, const f2d_grid* g,
     // limit excludes keep multigrid.)
     if (!h->fft && modal_ok)
       h->modal = modal_create(h->ny, h->nx, g->dx, g->dy, maindiag, h->xper, h->yper,
-                              h->opts.neumann != 0);
+                              h->opts.neumann != 0, h->opts.mode != F2D_POISSON_F64);
     // a masked vertex operator inside a rectangle the spectral solve
     // handles: the direct capacitance solve (auto: with a boundary of at
     // most CAP_AUTO_MAX points, and multigrid if its set-up fails)

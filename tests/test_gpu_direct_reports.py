@@ -162,3 +162,33 @@ def test_acceptance(dev, method, kw, factor):
     assert not ps._accepted(1e-7)
     ps.rtol = 1e-3  # a looser one is the caller's to choose
     assert ps._accepted(9e-4) and not ps._accepted(2e-3)
+
+
+@pytest.mark.parametrize("method,kw", [r for r in ROUTES if "location" not in r[1]])
+def test_measured_solves_capture(dev, method, kw):
+    """A measured solve allocates nothing: the first of a handle may be
+    captured, and each replay measures what it solved."""
+    from fluids2d_amd import _lib
+    ps = _solver(**kw)
+    assert ps.method == method
+    wet = ps.msk != 0
+    rng = np.random.default_rng(4)
+    b, x = (torch.zeros(wet.shape, dtype=ps.dtype, device=dev) for _ in range(2))
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with _lib.capture(g):
+        x.zero_()
+        ps.solve(b, x, stats="device")
+    for _ in range(3):
+        w = rng.standard_normal(wet.shape) * wet
+        w[wet] -= w[wet].mean()
+        b.copy_(torch.from_numpy(w))
+        ps.reset_stats()
+        g.replay()
+        got = x.clone()
+        st = ps._stats_host()
+        assert st[6] == 1 and 0.0 < st[1] == st[7] <= ps.accept()
+        want = torch.zeros_like(x)
+        ps.solve(b, want)
+        err = (got - want).double().norm() / want.double().norm()
+        assert err <= (1e-5 if ps.dtype == torch.float32 else 1e-12)
