@@ -35,7 +35,8 @@ int64_t cap_boundary(const int8_t* unk, int64_t ny, int64_t nx, int xper, int yp
 
 // f64_mode: FP64 solves (M in FP64); otherwise FP32 spectral solves and an
 // FP32 M inside FP64 refinement.  modal: FP64 solves by eigenvectors whatever
-// the precision of b and x.  Synchronises the device.
+// the precision of b and x, with the FP64 refinements that this set-up finds
+// the mask to need (an Error where three do not do).  Synchronises the device.
 CapSolver* cap_create(const int8_t* unk, int64_t ny, int64_t nx, double dx, double dy,
                       double maindiag, int xper, int yper, bool f64_mode, bool modal = false);
 void cap_destroy(CapSolver* c);

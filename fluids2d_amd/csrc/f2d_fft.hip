@@ -10,8 +10,10 @@
 //   rows:    the two half spectra of a row pair repacked into one complex
 //            row, inverse FFT, real/imaginary parts stored as the two rows
 //            together with their periodic halo images
-// The FFTs are mixed radix-4/2 Stockham passes (self-sorting, ping-pong
-// between two LDS buffers) with twiddles from a table in pass order;
+// Lengths up to 1024 run as mixed radix-4/2 Stockham passes through LDS
+// (fft_lds: self-sorting, ping-pong between two buffers); 2048 and 4096, and
+// FP64 columns from 256 (plan_blocks), as radix-8 passes in registers with LDS
+// exchanges between them (RegFft).  Twiddles come from tables in pass order;
 // inverse transforms conjugate on the way in and out.
 #include <cmath>
 #include <type_traits>

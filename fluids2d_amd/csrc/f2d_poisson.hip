@@ -1517,7 +1517,7 @@ struct f2d_poisson {
                                    // levels, single-workgroup tail
   double inner_rtol = 1e-4;
   f2d::FftSolver* fft = nullptr;  // direct spectral solve, when it applies
-  f2d::NeumannSolver* neu = nullptr;  // Neumann (cell) operator: Jacobi-PCG
+  f2d::NeumannSolver* neu = nullptr;  // Neumann (cell) operator: preconditioned CG
   f2d::CapSolver* cap = nullptr;  // masked operator: spectral + capacitance
   f2d::ModalSolver* modal = nullptr;  // fully wet rectangles of other sizes
   int64_t fft_unmeasured = 0;     // FFT solves made without statistics
@@ -2252,7 +2252,7 @@ int f2d_poisson_bench_kernel(f2d_poisson* h, int kind, int reps, double* us,
                              double* bytes, void* stream) {
   return guarded([&] {
     F2D_REQUIRE(h && us && bytes, "NULL argument");
-    F2D_REQUIRE(!h->neu, "no kernel timing on a Neumann (Jacobi-PCG) handle");
+    F2D_REQUIRE(!h->neu, "no kernel timing on a Neumann (CG) handle");
     F2D_REQUIRE(kind >= 0 && kind <= 9, "kind must be in 0 .. 9");
     F2D_REQUIRE(reps > 0, "reps must be > 0");
     hipStream_t s = S(stream);
@@ -2319,7 +2319,7 @@ int f2d_poisson_create(const int8_t* unknowns_host, const f2d_grid* g,
       }
     h->nwet = (double)nwet;
     // the Neumann cell operator: the direct solve when every cell is wet
-    // (closed directions as even extensions), Jacobi-PCG otherwise
+    // (closed directions as even extensions, or eigenvectors), CG otherwise
     // (an explicit request keeps to the two-buffer transforms)
     const bool fits = fft_fits(h->ny, h->nx, h->xper, h->yper,
                                h->opts.mode == F2D_POISSON_F64,
@@ -2405,8 +2405,10 @@ int f2d_poisson_create(const int8_t* unknowns_host, const f2d_grid* g,
     // took 2.17 ms a solve on an 800 x 304 channel (0.1 ms a whole stage
     // now), Jacobi-PCG 4.4 ms on the 40^2 cell operator, and multigrid does
     // not converge where halving leaves a coarsest level of many points
-    // (300^2, 500^2, 1000^2).  (Grids of two powers of two that the FFT's LDS
-    // limit excludes keep multigrid.)
+    // (300^2, 500^2, 1000^2).  Grids of two powers of two that the FFT's LDS
+    // limit excludes, closed directions of 2048 in FP64, keep multigrid; that
+    // line is not drawn by speed (closed 2048^2: 4160 us a solve from 0;
+    // closed 2050^2 by eigenvectors 970 us).
     if (!h->fft && modal_ok)
       h->modal = modal_create(h->ny, h->nx, g->dx, g->dy, maindiag, h->xper, h->yper,
                               h->opts.neumann != 0, h->opts.mode != F2D_POISSON_F64);

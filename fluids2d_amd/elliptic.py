@@ -1,12 +1,14 @@
 """Poisson2D: masked Poisson/Helmholtz solve on the vertex grid
-(elliptic.py:71-203), by the library's multigrid-preconditioned CG, or by its
-direct FFT solve when the operator is fully wet and doubly periodic.
+(elliptic.py:71-203) by one of the library's methods: direct solves of a
+rectangle (FFT, eigenvectors) and of a mask inside one (capacitance matrix),
+or multigrid-preconditioned CG; the Neumann cell operator of a mask by CG
+preconditioned with the rectangle's direct solve.
 
 The reference factorises the masked 5-point operator with SuperLU once per
 ``mesh.finalize()`` and solves with it at every stage.  Here the operator is
-matrix-free; ``create`` builds the multigrid hierarchy from the mask (and the
-spectral tables when they apply) and every iterative solve is warm-started
-from the previous solution held in ``x``.
+matrix-free; ``create`` picks the method from the mask and sets it up, and
+every iterative solve is warm-started from the previous solution held in
+``x``.
 """
 import ctypes
 
@@ -85,7 +87,7 @@ class Poisson2D:
         # x (the state's streamfunction) instead of a cold FP32 solve
         opts.fft_warm = int(bool(getattr(p, "poisson_warm", True)))
         # "c": the Neumann cell operator (elliptic.py:186-190): the direct
-        # solve when every cell is wet, else Jacobi-PCG in FP64.  Its
+        # solve when every cell is wet, else preconditioned CG in FP64.  Its
         # right-hand side (the divergence a stage's update left) is not
         # close to the previous stage's: cold FP32 solves, refined once
         opts.neumann = int(location == "c")
@@ -115,7 +117,7 @@ class Poisson2D:
         # "fft": direct spectral solve (exact to rounding);
         # "modal": direct eigenvector solve; "capacitance",
         # "modal_capacitance": direct masked solves around them; "mg":
-        # multigrid-preconditioned CG to rtol
+        # multigrid-preconditioned CG to rtol; "neumann": CG to rtol
         self.method = {2: "fft", 3: "neumann", 4: "capacitance", 5: "modal",
                        6: "modal_capacitance"}.get(
             _lib.lib().f2d_poisson_method(h), "mg")

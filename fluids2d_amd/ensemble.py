@@ -13,9 +13,10 @@ graph is replayed: one launch advances the whole ensemble by G steps with
 no host work in between.
 
 Results do not depend on S, on the packing or on the graph: each member's
-kernels and their order are those of its own ``device_steps``.  Reductions
-of the CFL step use per-stream scratch (``f2d_reserve_stream_scratch``),
-so concurrent members share no buffer.
+kernels and their order are those of its own ``device_steps``.  The CFL
+step's reductions use the member's own arrays, its first one (before any
+step) scratch of the stream (``f2d_reserve_stream_scratch``), so concurrent
+members share no buffer.
 
 Member batching (``batch=True``, the default): members whose stages pause
 at a Helmholtz solve of the capacitance method in FP32 (qgrsw) are grouped

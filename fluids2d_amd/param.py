@@ -21,9 +21,9 @@ Fields of the MI355X path (after the reference's in the table):
 * ``poisson_maxit``  iteration cap of the Poisson solves (None: 100 in FP64,
                      8 refinements in FP32)
 * ``poisson_nu``     red-black Gauss-Seidel sweeps before/after each level
-* ``poisson_solver`` "auto" (direct FFT solve of a fully wet rectangle, direct
-                     capacitance solve of a mask inside one, multigrid CG
-                     otherwise), "mg", "fft" or "cap"
+* ``poisson_solver`` "auto" (direct FFT or eigenvector solve of a fully wet
+                     rectangle, direct capacitance solve of a mask inside
+                     one, multigrid CG otherwise), "mg", "fft" or "cap"
 * ``poisson_warm``   FP32 direct solves refine from the solution held in x
                      (the previous stage's streamfunction)
 * ``poisson_refine`` "last" (FP32): only the last RK stage's direct solve of

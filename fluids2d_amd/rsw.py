@@ -347,8 +347,8 @@ class Euler(_SW):
     kinetic-energy gradient, then the pressure projection
     (operators.py:114-119) with the Neumann cell Poisson solve.  With a
     direct solve (all-wet domains) stages may skip the
-    host check and steps are graph-captured; the Jacobi-PCG solve always
-    checks convergence on the host, so its steps are not."""
+    host check and steps are graph-captured; the CG solve of a masked domain
+    always checks convergence on the host, so its steps are not."""
     prognostic = ("u",)
     logs_dt = False
 

@@ -455,9 +455,11 @@ typedef struct f2d_poisson_opts {
                             solve (even extensions about closed walls; zero
                             mean when singular) unless solver is MG; every
                             cell wet, other sizes and solver AUTO: the
-                            eigenvector solve; else
-                            Jacobi-preconditioned CG in FP64 (x keeps the
-                            constant of its initial guess)                 */
+                            eigenvector solve; else CG in FP64 (x keeps the
+                            constant of its initial guess), preconditioned
+                            by the rectangle's direct solve, or by the
+                            diagonal (Jacobi) where none takes the sizes and
+                            for solver MG                                  */
 } f2d_poisson_opts;
 
 /* Solver selection.  AUTO takes the direct spectral (FFT) solve when every
