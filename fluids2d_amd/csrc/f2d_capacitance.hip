@@ -246,6 +246,16 @@ __global__ __launch_bounds__(256) void k_cap_acc(int64_t n, const int8_t* __rest
   if (k < n && mw[k]) x64[k] = (x0 ? (double)x0[k] : 0.0) + (double)e[k];
 }
 
+// b = 1 at the unknowns, x = 0
+__global__ __launch_bounds__(256) void k_cap_ones(int64_t n, const int8_t* __restrict__ mw,
+                                                  double* __restrict__ b,
+                                                  double* __restrict__ x) {
+  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (k >= n) return;
+  b[k] = mw[k] ? 1.0 : 0.0;
+  x[k] = 0.0;
+}
+
 // x64 += e at the unknowns, rounded to x
 template <class T>
 __global__ __launch_bounds__(256) void k_cap_add(int64_t n, const int8_t* __restrict__ mw,
@@ -732,28 +742,25 @@ void cap_solve_modal(CapSolver* c, const T* b, int gmode, T* x, bool measure, do
 // multigrid.
 static void set_refinements(CapSolver* c) {
   const size_t N = (size_t)c->g.NYP * c->g.NXP;
-  std::vector<int8_t> mw(N);
-  F2D_HIP(hipMemcpy(mw.data(), c->mw, N, hipMemcpyDeviceToHost));
-  std::vector<double> h(N);
-  for (size_t k = 0; k < N; k++) h[k] = mw[k] ? 1.0 : 0.0;
+  const int8_t* mw = c->mw;
   struct Buf {
     double* p = nullptr;
     explicit Buf(size_t n) { F2D_HIP(hipMalloc(&p, sizeof(double) * n)); }
     ~Buf() { (void)hipFree(p); }
   } b(N), x(N);
-  F2D_HIP(hipMemcpy(b.p, h.data(), sizeof(double) * N, hipMemcpyHostToDevice));
-  F2D_HIP(hipMemset(x.p, 0, sizeof(double) * N));
+  k_cap_ones<<<c->nbres, 256>>>((int64_t)N, mw, b.p, x.p);
   std::vector<double> part(2 * (size_t)c->nbres);
+  const size_t bytes = sizeof(double) * part.size();
   const double anorm = fabs(c->g.d) + 2.0 * (c->g.cx + c->g.cy);
   for (;; c->refine++) {
     cap_solve_modal<double>(c, b.p, 0, x.p, false, 0.0, nullptr, 0);
-    k_cap_norms<double, double><<<c->nbres, 256>>>(c->g, b.p, 0, c->mw, x.p, c->part);
-    F2D_HIP(hipMemcpy(part.data(), c->part, sizeof(double) * part.size(),
-                      hipMemcpyDeviceToHost));
-    F2D_HIP(hipMemcpy(h.data(), x.p, sizeof(double) * N, hipMemcpyDeviceToHost));
     double rr = 0.0, xx = 0.0;
+    k_cap_norms<double, double><<<c->nbres, 256>>>(c->g, b.p, 0, mw, x.p, c->part);
+    F2D_HIP(hipMemcpy(part.data(), c->part, bytes, hipMemcpyDeviceToHost));
     for (int i = 0; i < c->nbres; i++) rr += part[i];
-    for (size_t k = 0; k < N; k++) xx += mw[k] ? h[k] * h[k] : 0.0;
+    k_cap_norms<double, double><<<c->nbres, 256>>>(c->g, x.p, 0, mw, x.p, c->part);
+    F2D_HIP(hipMemcpy(part.data(), c->part, bytes, hipMemcpyDeviceToHost));
+    for (int i = 0; i < c->nbres; i++) xx += part[c->nbres + i];  // |b|^2, b = x
     if (sqrt(rr) <= 64.0 * 0x1p-53 * anorm * sqrt(xx)) break;
     F2D_REQUIRE(c->refine < 3, "capacitance solve of this mask is not accurate enough");
     if (!c->x64) c->x64 = (double*)calloc_dev(c, sizeof(double) * N);
