@@ -70,6 +70,7 @@ class RKIntegrator:
         # in, whether that dt is still the next step's
         self._checked = {}
         self._h_run = torch.zeros(4, dtype=torch.float64).pin_memory()
+        self._n_run = self._h_run.numpy()  # (read without a tensor of its own)
         self._dt_on_host = False
         self._run_steps, self._run_total, self._run_mesh = 0, 0, None
         self._no_replay = False
@@ -193,7 +194,7 @@ class RKIntegrator:
         self.d_dt, self.d_dtn = self.d_dtn, self.d_dt
         if self._dt_on_host:  # left there by the step's graph
             self._dt_on_host = False
-            time.dt = float(self._h_run[0])
+            time.dt = float(self._n_run[0])
             return
         self._h_dt.copy_(self.d_dt, non_blocking=True)
         torch.cuda.current_stream().synchronize()
@@ -337,7 +338,7 @@ class RKIntegrator:
                 torch.cuda.current_stream().synchronize()
             for k, e in enumerate(sols):
                 e.calls += self.nstages
-                e.check_worst(float(self._h_run[1 + k]))
+                e.check_worst(float(self._n_run[1 + k]))
             self.dstate, self.dalt = after
             self._dtn_valid = self._dt_on_host = dtn
             self._dt_part = self._dtn_part = False
